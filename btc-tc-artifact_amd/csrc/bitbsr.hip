@@ -12,15 +12,13 @@
 // counting pass sizes the row blocks, a scan gives indptr, a fill pass
 // writes indices, row_indices and tiles.
 //
-// Count: one wave64 per mask tile S = (I, J_L), as one warp per tile in
-// tc_16x128_mma_v5.h:9-211 / tc_16x32_mma_v6.h:9-238: popcount(S) > tau
-// picks the dense path (wave-uniform two-pointer merge of the tile columns of
-// row blocks I and J_out, every matched pair contributing a full 16 x 16 block
-// of AND+popcount dot products, masked by S afterwards) or the sparse path
-// (per-lane merge, only the set mask bits of the lane are evaluated).  Lane
-// (r, q) = (lane / 4, lane % 4) owns row r of the tile and the 4 columns
-// 4q..4q+3 of each 16-column J_out slab, so every lane's partial sum belongs
-// to a single vertex 16I + r.
+// Count: popcount(S) > tau routes a mask tile S = (I, J_L) to the dense path
+// (matched tile pairs of row blocks I and J_out as 16 x 16 blocks of AND +
+// popcount or i8 MFMA, masked by S: dense_unit_kernel, shared with the
+// engine) or the sparse path (only the set mask bits are evaluated), as in
+// tc_16x128_mma_v5.h:9-211 / tc_16x32_mma_v6.h:9-238.  The reference walks
+// tile columns in both; here the sparse mask bits go row by row over the CSR
+// that the handle keeps (rowcount.hip).
 #include <type_traits>
 
 #include "device_util.h"
@@ -226,7 +224,9 @@ struct RowBits<128> {
 };
 
 // FILL = false: counts[I] = number of tiles of row block I.
-// FILL = true: writes tile I's indices / row_indices / bits at offs[I].
+// FILL = true: writes tile I's indices / row_indices / bits at offs[I] and,
+// with pop, every tile's set bits (pop) and, beside each entry of L, those
+// of its tile (epop); *max_pop becomes the largest of them.
 template <int K, bool FILL>
 __global__ __launch_bounds__(256) void build_kernel(int n, int n_rb, const uint32_t* __restrict__ rowptr,
                                                      const int32_t* __restrict__ col,
@@ -234,7 +234,8 @@ __global__ __launch_bounds__(256) void build_kernel(int n, int n_rb, const uint3
                                                      const uint64_t* __restrict__ offs,
                                                      uint32_t* __restrict__ indices,
                                                      uint32_t* __restrict__ row_indices,
-                                                     uint64_t* __restrict__ tiles) {
+                                                     uint64_t* __restrict__ tiles, uint32_t* __restrict__ pop,
+                                                     uint16_t* __restrict__ epop, uint32_t* __restrict__ max_pop) {
     const int lane = threadIdx.x & 63;
     const int r = lane & 15;
     const int64_t I = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * 4 + (lane >> 4);
@@ -246,7 +247,7 @@ __global__ __launch_bounds__(256) void build_kernel(int n, int n_rb, const uint3
         e = rowptr[row + 1];
     }
     uint64_t t = (FILL && valid) ? offs[I] : 0;
-    uint32_t cnt = 0;
+    uint32_t cnt = 0, most = 0;
     // the row's next four ids (kNoId past its end), refilled one load
     // ahead per consumed id so a run of ids in one tile waits on memory
     // once every four ids instead of once per id
@@ -259,6 +260,7 @@ __global__ __launch_bounds__(256) void build_kernel(int n, int n_rb, const uint3
         if (__all(cur == kNoTile)) break;
         if (cur != kNoTile) {
             RowBits<K> bits;
+            const uint32_t p0 = p;
             while (b0 != kNoId && b0 / K == cur) {
                 bits.set((int)(b0 % K));
                 ++p;
@@ -281,12 +283,25 @@ __global__ __launch_bounds__(256) void build_kernel(int n, int n_rb, const uint3
                     tiles[t * 32 + 2 * r] = bits.w0;
                     tiles[t * 32 + 2 * r + 1] = bits.w1;
                 }
+                if (pop) {
+                    uint32_t c = p - p0;
+#pragma unroll
+                    for (int o = 8; o > 0; o >>= 1) c += (uint32_t)__shfl_xor((int)c, o, 16);
+                    if (r == 0) pop[t] = c;
+                    for (uint32_t q = p0; q < p; ++q) epop[q] = (uint16_t)c;
+                    most = max(most, c);
+                }
                 ++t;
             }
             ++cnt;
         }
     }
     if (!FILL && valid && r == 0) counts[I] = cnt;
+    if (FILL && pop) {
+#pragma unroll
+        for (int o = 32; o >= 16; o >>= 1) most = max(most, (uint32_t)__shfl_xor((int)most, o));
+        if (lane == 0 && most > *max_pop) atomicMax(max_pop, most);  // most waves find it raised already
+    }
 }
 
 __global__ void narrow_u64_to_u32(const uint64_t* __restrict__ in, uint32_t* __restrict__ out, size_t n) {
@@ -295,7 +310,7 @@ __global__ void narrow_u64_to_u32(const uint64_t* __restrict__ in, uint32_t* __r
 }
 
 template <int K>
-void build_impl(btc_graph_s* g, hipStream_t s, btc_bitbsr_s* b) {
+void build_impl(btc_graph_s* g, hipStream_t s, btc_bitbsr_s* b, bool counted) {
     const int n = g->n;
     const int n_rb = (n + 15) / 16;
     b->n = n;
@@ -310,7 +325,7 @@ void build_impl(btc_graph_s* g, hipStream_t s, btc_bitbsr_s* b) {
     offs.alloc((size_t)n_rb + 1, s);
     if (grid) {
         hipLaunchKernelGGL((build_kernel<K, false>), dim3(grid), dim3(256), 0, s, n, n_rb, g->d_rowptr.p,
-                           g->d_col.p, counts.p, nullptr, nullptr, nullptr, nullptr);
+                           g->d_col.p, counts.p, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
         BTC_CHECK_LAUNCH("build_kernel<count>");
     }
     scan_u32_to_u64(counts.p, offs.p, (size_t)n_rb, s);
@@ -324,14 +339,23 @@ void build_impl(btc_graph_s* g, hipStream_t s, btc_bitbsr_s* b) {
     b->indices.alloc(nblk);
     b->row_indices.alloc(nblk);
     b->tiles.alloc(nblk * (size_t)b->wpt);
-    b->result.alloc(1);
+    if (counted) {
+        build_row_lists(g, b->rows, s);
+        b->pop.alloc(nblk);
+        b->work.alloc(kWorkWords);
+    }
     hipLaunchKernelGGL(narrow_u64_to_u32, dim3((unsigned)((n_rb + 1 + 255) / 256)), dim3(256), 0, s, offs.p,
                        b->indptr.p, (size_t)n_rb + 1);
     BTC_CHECK_LAUNCH("narrow_u64_to_u32");
     if (grid && nblk) {
         hipLaunchKernelGGL((build_kernel<K, true>), dim3(grid), dim3(256), 0, s, n, n_rb, g->d_rowptr.p,
-                           g->d_col.p, nullptr, offs.p, b->indices.p, b->row_indices.p, b->tiles.p);
+                           g->d_col.p, nullptr, offs.p, b->indices.p, b->row_indices.p, b->tiles.p,
+                           counted ? b->pop.p : nullptr, b->rows.epop, counted ? b->rows.d_count + 3 : nullptr);
         BTC_CHECK_LAUNCH("build_kernel<fill>");
+    }
+    if (counted) {
+        BTC_HIP(hipMemcpyAsync(b->rows.count, b->rows.d_count, sizeof(b->rows.count), hipMemcpyDeviceToHost, s));
+        BTC_HIP(hipStreamSynchronize(s));
     }
 }
 
@@ -396,163 +420,6 @@ __device__ __forceinline__ v4i mfma_mac(const MfmaOp<K>& a, const MfmaOp<K>& b, 
                                                         0);
         return acc;
     }
-}
-
-template <int K>
-__device__ __forceinline__ v4i mfma_pair(const uint64_t* __restrict__ T, uint32_t pa, uint32_t pb, int i, int g,
-                                         v4i acc) {
-    if constexpr (K == 32) {
-        const uint32_t a = reinterpret_cast<const uint32_t*>(T + (size_t)pa * 8)[i];
-        const uint32_t b = reinterpret_cast<const uint32_t*>(T + (size_t)pb * 8)[i];
-        return __builtin_amdgcn_mfma_i32_16x16x32_i8(bytes8((a >> (8 * g)) & 0xFFu), bytes8((b >> (8 * g)) & 0xFFu),
-                                                     acc, 0, 0, 0);
-    } else {
-#pragma unroll
-        for (int h = 0; h < K / 64; ++h) {
-            const uint64_t a = T[(size_t)pa * (K / 4) + (K / 64) * i + h];
-            const uint64_t b = T[(size_t)pb * (K / 4) + (K / 64) * i + h];
-            acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(bytes16((uint32_t)(a >> (16 * g)) & 0xFFFFu),
-                                                        bytes16((uint32_t)(b >> (16 * g)) & 0xFFFFu), acc, 0, 0, 0);
-        }
-        return acc;
-    }
-}
-
-template <int K, bool BINSEARCH, bool PV, bool MFMA>
-__global__ __launch_bounds__(256) void tile_count_kernel(
-    int n, int n_rb, const uint32_t* __restrict__ indptr, const uint32_t* __restrict__ indices,
-    const uint32_t* __restrict__ row_indices, const uint64_t* __restrict__ tiles, uint32_t w0,
-    uint32_t w_end, const uint32_t* __restrict__ tile_list, uint32_t lstride, int tau,
-    unsigned long long* __restrict__ result, PvOut pv) {
-    constexpr int WPT = K / 4;
-    constexpr int SLABS = K / 16;
-    const int lane = threadIdx.x & 63;
-    const uint32_t w = uniform(w0 + blockIdx.x * 4 + (threadIdx.x >> 6));
-    if (w >= w_end) return;
-    const uint32_t t = tile_list ? uniform(tile_list[(size_t)w * lstride]) : w;
-    uint32_t I;
-    if (BINSEARCH) {  // row block of tile t by binary search over indptr (tc_16x128_mma_v4.h:29-38)
-        uint32_t lo = 0, hi = (uint32_t)n_rb;
-        while (lo < hi) {
-            uint32_t mid = (lo + hi) >> 1;
-            if (indptr[mid + 1] <= t) lo = mid + 1;
-            else hi = mid;
-        }
-        I = uniform(lo);
-    } else {
-        I = uniform(row_indices[t]);
-    }
-    const uint32_t JL = uniform(indices[t]);
-    const uint32_t a0 = uniform(indptr[I]), a1 = uniform(indptr[I + 1]);
-
-    uint32_t c = lane < WPT ? (uint32_t)__popcll(tiles[(size_t)t * WPT + lane]) : 0u;
-    const bool dense = (int)wave_sum_u32(c) > tau;
-
-    const int r = lane >> 2, q = lane & 3;
-    const RowBits<K> S = RowBits<K>::load(tiles, t, r);
-    uint32_t sum = 0;
-    if (MFMA && dense) {
-        // lane owns rows 4g + v (v < 4) of the mask tile and column c of each slab
-        const int g = lane >> 4, c = lane & 15;
-        RowBits<K> M[4];
-#pragma unroll
-        for (int v = 0; v < 4; ++v) M[v] = RowBits<K>::load(tiles, t, 4 * g + v);
-        uint32_t rs[4] = {0, 0, 0, 0};
-        for (int it = 0; it < SLABS; ++it) {
-            const uint32_t Jo = JL * SLABS + it;
-            if (Jo >= (uint32_t)n_rb) break;
-            const uint32_t b0 = uniform(indptr[Jo]), b1 = uniform(indptr[Jo + 1]);
-            v4i acc = {0, 0, 0, 0};
-            uint32_t pa = a0, pb = b0;
-            while (pa < a1 && pb < b1) {
-                const uint32_t ka = uniform(indices[pa]), kb = uniform(indices[pb]);
-                if (ka < kb) {
-                    ++pa;
-                } else if (ka > kb) {
-                    ++pb;
-                } else {
-                    acc = mfma_pair<K>(tiles, pa, pb, c, g, acc);
-                    ++pa;
-                    ++pb;
-                }
-            }
-            rs[0] += (M[0].bits(it * 16 + c) & 1u) ? (uint32_t)acc.x : 0u;
-            rs[1] += (M[1].bits(it * 16 + c) & 1u) ? (uint32_t)acc.y : 0u;
-            rs[2] += (M[2].bits(it * 16 + c) & 1u) ? (uint32_t)acc.z : 0u;
-            rs[3] += (M[3].bits(it * 16 + c) & 1u) ? (uint32_t)acc.w : 0u;
-        }
-        if (PV) {
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                uint32_t x = rs[v];
-                x += __shfl_xor(x, 1);
-                x += __shfl_xor(x, 2);
-                x += __shfl_xor(x, 4);
-                x += __shfl_xor(x, 8);
-                const int64_t vtx = (int64_t)I * 16 + 4 * g + v;
-                if (c == 0 && x && vtx < n) pv_add(pv, vtx, x);
-            }
-        }
-        const uint64_t tot = wave_sum_u64((uint64_t)(rs[0] + rs[1] + rs[2] + rs[3]));
-        if (lane == 0 && tot) atomicAdd(result, (unsigned long long)tot);
-        return;
-    }
-    for (int it = 0; it < SLABS; ++it) {
-        const uint32_t Jo = JL * SLABS + it;
-        if (Jo >= (uint32_t)n_rb) break;
-        const uint32_t b0 = uniform(indptr[Jo]), b1 = uniform(indptr[Jo + 1]);
-        const uint32_t m4 = S.bits(it * 16 + 4 * q) & 0xFu;
-        if (dense) {
-            uint32_t acc0 = 0, acc1 = 0, acc2 = 0, acc3 = 0;
-            uint32_t pa = a0, pb = b0;
-            while (pa < a1 && pb < b1) {
-                const uint32_t ka = uniform(indices[pa]), kb = uniform(indices[pb]);
-                if (ka < kb) {
-                    ++pa;
-                } else if (ka > kb) {
-                    ++pb;
-                } else {
-                    const RowBits<K> A = RowBits<K>::load(tiles, pa, r);
-                    acc0 += A.and_popc(RowBits<K>::load(tiles, pb, 4 * q + 0));
-                    acc1 += A.and_popc(RowBits<K>::load(tiles, pb, 4 * q + 1));
-                    acc2 += A.and_popc(RowBits<K>::load(tiles, pb, 4 * q + 2));
-                    acc3 += A.and_popc(RowBits<K>::load(tiles, pb, 4 * q + 3));
-                    ++pa;
-                    ++pb;
-                }
-            }
-            sum += ((m4 & 1u) ? acc0 : 0u) + ((m4 & 2u) ? acc1 : 0u) + ((m4 & 4u) ? acc2 : 0u) +
-                   ((m4 & 8u) ? acc3 : 0u);
-        } else if (m4) {
-            uint32_t pa = a0, pb = b0;
-            while (pa < a1 && pb < b1) {
-                const uint32_t ka = indices[pa], kb = indices[pb];
-                if (ka < kb) {
-                    ++pa;
-                } else if (ka > kb) {
-                    ++pb;
-                } else {
-                    const RowBits<K> A = RowBits<K>::load(tiles, pa, r);
-                    uint32_t mm = m4;
-                    while (mm) {
-                        const int cc = __ffs(mm) - 1;
-                        sum += A.and_popc(RowBits<K>::load(tiles, pb, 4 * q + cc));
-                        mm &= mm - 1;
-                    }
-                    ++pa;
-                    ++pb;
-                }
-            }
-        }
-    }
-    if (PV) {
-        uint32_t rs = sum + __shfl_xor(sum, 1);
-        rs += __shfl_xor(rs, 2);
-        const int64_t v = (int64_t)I * 16 + r;
-        if (q == 0 && rs && v < n) pv_add(pv, v, rs);
-    }
-    const uint64_t tot = wave_sum_u64((uint64_t)sum);
-    if (lane == 0 && tot) atomicAdd(result, (unsigned long long)tot);
 }
 
 // Calls f(pa, pb) for every tile column present in both sorted lists
@@ -756,6 +623,94 @@ __global__ __launch_bounds__(256) void dense_units_kernel(const uint32_t* __rest
     }
 }
 
+// Dense tiles of one count (pop > tau): their units, in any order but each
+// tile's together, at units[0, *n_units).  A workgroup looks at kSelTiles tiles and takes the
+// dense ones 16 lanes each (a lane per tile row, then per slab).  Its units
+// get their places with one atomic: one per dense tile on the same address
+// took 54 of planted 2^17's 284 us.
+constexpr uint32_t kSelTiles = 1024;
+template <int K>
+__global__ __launch_bounds__(256) void select_dense_kernel(
+    const uint32_t* __restrict__ pop, uint32_t nblk, int tau, int n_rb, const uint32_t* __restrict__ indptr,
+    const uint32_t* __restrict__ indices, const uint32_t* __restrict__ row_indices,
+    const uint64_t* __restrict__ tiles, uint4* __restrict__ units, uint32_t* __restrict__ n_units) {
+    constexpr int SLABS = K / 16;
+    __shared__ uint32_t tile[kSelTiles];  // the workgroup's dense tiles
+    __shared__ uint16_t have[kSelTiles];  // their slabs with a unit
+    __shared__ uint32_t nd_s, wsum[4], base_s;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, r = tid & 15, grp = tid >> 4;
+    if (tid == 0) nd_s = 0;
+    __syncthreads();
+    for (uint32_t x = tid; x < kSelTiles; x += 256) {
+        const uint64_t t = (uint64_t)blockIdx.x * kSelTiles + x;
+        if (t < nblk && (int)pop[t] > tau) tile[atomicAdd(&nd_s, 1u)] = (uint32_t)t;
+    }
+    __syncthreads();
+    const uint32_t nd = nd_s;
+    if (nd == 0) return;
+    // lane sl < SLABS: row block under slab sl and its tile columns
+    auto under = [&](uint32_t t, uint64_t& Jo, uint32_t& b0, uint32_t& b1) {
+        Jo = (uint64_t)indices[t] * SLABS + (uint64_t)r;
+        b0 = b1 = 0;
+        if (r < (uint32_t)SLABS && Jo < (uint64_t)n_rb) {
+            b0 = indptr[Jo];
+            b1 = indptr[Jo + 1];
+        }
+    };
+    for (uint32_t x = grp; x < nd; x += 16) {
+        const uint32_t t = tile[x];
+        const uint16_t* h = reinterpret_cast<const uint16_t*>(tiles + (size_t)t * (K / 4)) + r * SLABS;
+        uint32_t occ = 0;  // lane r: the slabs in which row r has bits
+#pragma unroll
+        for (int sl = 0; sl < SLABS; ++sl)
+            if (h[sl]) occ |= 1u << sl;
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1) occ |= (uint32_t)__shfl_xor((int)occ, o, 16);
+        uint64_t Jo;
+        uint32_t b0, b1;
+        under(t, Jo, b0, b1);
+        uint32_t hv = ((occ >> r) & 1u) && b1 != b0 ? 1u << r : 0u;
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1) hv |= (uint32_t)__shfl_xor((int)hv, o, 16);
+        if (r == 0) have[x] = (uint16_t)hv;
+    }
+    __syncthreads();
+    // places of the tiles' units: thread tid owns tiles [4 tid, 4 tid + 4)
+    uint32_t c[kSelTiles / 256], sum = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kSelTiles / 256; ++k) {
+        const uint32_t x = tid * (kSelTiles / 256) + k;
+        c[k] = sum;
+        sum += x < nd ? (uint32_t)__popc(have[x]) : 0u;
+    }
+    uint32_t inc = sum;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = (uint32_t)__shfl_up((int)inc, o);
+        if ((int)lane >= o) inc += y;
+    }
+    if (lane == 63) wsum[tid >> 6] = inc;
+    __syncthreads();
+    if (tid == 0) base_s = atomicAdd(n_units, wsum[0] + wsum[1] + wsum[2] + wsum[3]);
+    __shared__ uint32_t place[kSelTiles];
+    uint32_t at = inc - sum;
+    for (uint32_t w = 0; w < (tid >> 6); ++w) at += wsum[w];
+#pragma unroll
+    for (uint32_t k = 0; k < kSelTiles / 256; ++k) place[tid * (kSelTiles / 256) + k] = at + c[k];
+    __syncthreads();
+    for (uint32_t x = grp; x < nd; x += 16) {
+        const uint32_t t = tile[x], hv = have[x];
+        if (!((hv >> r) & 1u)) continue;
+        uint64_t Jo;
+        uint32_t b0, b1;
+        under(t, Jo, b0, b1);
+        const uint32_t I = row_indices[t];
+        const size_t u = (size_t)base_s + place[x] + (size_t)__popc(hv & ((1u << r) - 1u));
+        units[2 * u] = make_uint4(t, I, indptr[I], indptr[I + 1]);
+        units[2 * u + 1] = make_uint4((uint32_t)Jo, b0, b1, r);
+    }
+}
+
 __global__ __launch_bounds__(256) void gather_u32_kernel(const uint32_t* __restrict__ in,
                                                          const uint32_t* __restrict__ order, uint32_t n,
                                                          uint32_t* __restrict__ out) {
@@ -800,9 +755,12 @@ template <int K, bool PV, bool MFMA>
 __global__ __launch_bounds__(256) void dense_unit_kernel(int n, const uint32_t* __restrict__ indices,
                                                          const uint64_t* __restrict__ tiles,
                                                          const uint4* __restrict__ units, uint32_t first,
-                                                         uint32_t count, uint32_t stride, uint32_t set_words,
-                                                         uint32_t run, unsigned long long* __restrict__ slots,
-                                                         PvOut pv) {
+                                                         uint32_t count, const uint32_t* __restrict__ d_count,
+                                                         uint32_t stride, uint32_t set_words, uint32_t run,
+                                                         unsigned long long* __restrict__ slots, PvOut pv) {
+    // d_count (stride 1 then): units listed in all, known on the device only
+    if (d_count) count = min(count, max(*d_count, first) - first);
+    if (blockIdx.x * 4 * run >= count) return;
     constexpr int SLABS = K / 16;
     constexpr uint32_t TB = kTileBytes<K>;
     constexpr uint32_t WB = kWaveDenseBytes<K>;
@@ -1075,59 +1033,15 @@ __global__ __launch_bounds__(256) void tile_popcount_kernel(const uint64_t* __re
 // into launches of kMaxTilesPerLaunch waves.
 constexpr uint32_t kMaxTilesPerLaunch = 1u << 24;
 
-template <int K, bool BS, bool MF>
-void launch_k(const btc_bitbsr_s* b, const uint32_t* list, uint32_t lstride, uint32_t nt, int tau,
-              unsigned long long* res, PvOut pv, hipStream_t s) {
-    for (uint32_t w0 = 0; w0 < nt; w0 += kMaxTilesPerLaunch) {
-        const uint32_t chunk = std::min(kMaxTilesPerLaunch, nt - w0);
-        const unsigned grid = (chunk + 3) / 4;
-        const uint32_t end = w0 + chunk;
-        if (pv.on())
-            hipLaunchKernelGGL((tile_count_kernel<K, BS, true, MF>), dim3(grid), dim3(256), 0, s, b->n, b->n_rb,
-                               b->indptr.p, b->indices.p, b->row_indices.p, b->tiles.p, w0, end, list, lstride, tau,
-                               res, pv);
-        else
-            hipLaunchKernelGGL((tile_count_kernel<K, BS, false, MF>), dim3(grid), dim3(256), 0, s, b->n, b->n_rb,
-                               b->indptr.p, b->indices.p, b->row_indices.p, b->tiles.p, w0, end, list, lstride, tau,
-                               res, pv);
-        BTC_CHECK_LAUNCH("tile_count_kernel");
-    }
-}
-
-template <int K>
-void launch_kk(const btc_bitbsr_s* b, const uint32_t* list, uint32_t lstride, uint32_t nt, bool bs, bool mfma,
-               int tau, unsigned long long* res, PvOut pv, hipStream_t s) {
-    if (bs) {
-        mfma ? launch_k<K, true, true>(b, list, lstride, nt, tau, res, pv, s)
-             : launch_k<K, true, false>(b, list, lstride, nt, tau, res, pv, s);
-    } else {
-        mfma ? launch_k<K, false, true>(b, list, lstride, nt, tau, res, pv, s)
-             : launch_k<K, false, false>(b, list, lstride, nt, tau, res, pv, s);
-    }
-}
-
 }  // namespace
 
-void bitbsr_build(btc_graph_s* g, int K, hipStream_t s, btc_bitbsr_s* b) {
+void bitbsr_build(btc_graph_s* g, int K, hipStream_t s, btc_bitbsr_s* b, bool counted) {
     ensure_device(g, s);
     switch (K) {
-        case 32: build_impl<32>(g, s, b); break;
-        case 64: build_impl<64>(g, s, b); break;
-        case 128: build_impl<128>(g, s, b); break;
+        case 32: build_impl<32>(g, s, b, counted); break;
+        case 64: build_impl<64>(g, s, b, counted); break;
+        case 128: build_impl<128>(g, s, b, counted); break;
         default: fail(BTC_ERR_ARG, "tile width K = %d (expected 32, 64 or 128)", K);
-    }
-}
-
-void launch_tile_count(const btc_bitbsr_s* b, const uint32_t* tile_list, uint32_t ntiles, bool binsearch,
-                       bool mfma, int tau, unsigned long long* d_result, PvOut d_pv, hipStream_t s,
-                       uint32_t lstride) {
-    if (ntiles == 0) return;
-    BTC_REQUIRE(lane_sums_fit(b->max_row, b->K), BTC_ERR_OVERFLOW,
-                "longest row %d: a lane's 32-bit sum over %d tile columns could overflow", b->max_row, b->K / 4);
-    switch (b->K) {
-        case 32: launch_kk<32>(b, tile_list, lstride, ntiles, binsearch, mfma, tau, d_result, d_pv, s); break;
-        case 64: launch_kk<64>(b, tile_list, lstride, ntiles, binsearch, mfma, tau, d_result, d_pv, s); break;
-        default: launch_kk<128>(b, tile_list, lstride, ntiles, binsearch, mfma, tau, d_result, d_pv, s); break;
     }
 }
 
@@ -1179,7 +1093,7 @@ uint32_t build_dense_units(const btc_bitbsr_s* b, const uint32_t* list, uint32_t
 namespace {
 template <int K, bool MF>
 void launch_units_k(const btc_bitbsr_s* b, const uint4* units, uint32_t first, uint32_t count, uint32_t stride,
-                    unsigned long long* res, PvOut pv, hipStream_t s) {
+                    unsigned long long* res, PvOut pv, hipStream_t s, const uint32_t* d_count) {
     // column blocks of the graph: ids of tile columns are below this
     const uint64_t ncb = ((uint64_t)b->n + K - 1) / K;
     const uint32_t set_words = ncb <= 32ull * kColSetWords ? (uint32_t)((ncb + 31) / 32) : 0u;
@@ -1192,28 +1106,46 @@ void launch_units_k(const btc_bitbsr_s* b, const uint4* units, uint32_t first, u
         const uint32_t f0 = first + w0 * stride;
         if (pv.on())
             hipLaunchKernelGGL((dense_unit_kernel<K, true, MF>), dim3(grid), dim3(256), lds, s, b->n, b->indices.p,
-                               b->tiles.p, units, f0, chunk, stride, set_words, run, res, pv);
+                               b->tiles.p, units, f0, chunk, d_count, stride, set_words, run, res, pv);
         else
             hipLaunchKernelGGL((dense_unit_kernel<K, false, MF>), dim3(grid), dim3(256), lds, s, b->n, b->indices.p,
-                               b->tiles.p, units, f0, chunk, stride, set_words, run, res, pv);
+                               b->tiles.p, units, f0, chunk, d_count, stride, set_words, run, res, pv);
         BTC_CHECK_LAUNCH("dense_unit_kernel");
     }
 }
 }  // namespace
 
 void launch_dense_units(const btc_bitbsr_s* b, const uint4* units, uint32_t first, uint32_t count, uint32_t stride,
-                        bool mfma, unsigned long long* d_slots, PvOut d_pv, hipStream_t s) {
+                        bool mfma, unsigned long long* d_slots, PvOut d_pv, hipStream_t s, const uint32_t* d_count) {
     if (count == 0) return;
     BTC_REQUIRE(lane_sums_fit(b->max_row, b->K), BTC_ERR_OVERFLOW,
                 "longest row %d: a lane's 32-bit sum over %d tile columns could overflow", b->max_row, b->K / 4);
     switch (b->K) {
-        case 32: mfma ? launch_units_k<32, true>(b, units, first, count, stride, d_slots, d_pv, s)
-                      : launch_units_k<32, false>(b, units, first, count, stride, d_slots, d_pv, s); break;
-        case 64: mfma ? launch_units_k<64, true>(b, units, first, count, stride, d_slots, d_pv, s)
-                      : launch_units_k<64, false>(b, units, first, count, stride, d_slots, d_pv, s); break;
-        default: mfma ? launch_units_k<128, true>(b, units, first, count, stride, d_slots, d_pv, s)
-                      : launch_units_k<128, false>(b, units, first, count, stride, d_slots, d_pv, s); break;
+        case 32: mfma ? launch_units_k<32, true>(b, units, first, count, stride, d_slots, d_pv, s, d_count)
+                      : launch_units_k<32, false>(b, units, first, count, stride, d_slots, d_pv, s, d_count); break;
+        case 64: mfma ? launch_units_k<64, true>(b, units, first, count, stride, d_slots, d_pv, s, d_count)
+                      : launch_units_k<64, false>(b, units, first, count, stride, d_slots, d_pv, s, d_count); break;
+        default: mfma ? launch_units_k<128, true>(b, units, first, count, stride, d_slots, d_pv, s, d_count)
+                      : launch_units_k<128, false>(b, units, first, count, stride, d_slots, d_pv, s, d_count); break;
     }
+}
+
+void launch_dense_part(const btc_bitbsr_s* b, int tau, bool mfma, uint4* units, uint64_t max_units, unsigned long long* d_slots, PvOut d_pv, hipStream_t s) {
+    BTC_REQUIRE(max_units < 0xFFFFFFFFull, BTC_ERR_OVERFLOW, "%llu dense units exceed a u32 index",
+                (unsigned long long)max_units);
+    uint32_t* n_units = reinterpret_cast<uint32_t*>(d_slots - kWorkSlots + 1);  // the work words' first counter
+    const unsigned grid = (unsigned)(((uint64_t)b->nblk + kSelTiles - 1) / kSelTiles);
+    auto launch = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, s, b->pop.p, b->nblk, tau, b->n_rb, b->indptr.p,
+                           b->indices.p, b->row_indices.p, b->tiles.p, units, n_units);
+        BTC_CHECK_LAUNCH("select_dense_kernel");
+    };
+    switch (b->K) {
+        case 32: launch(select_dense_kernel<32>); break;
+        case 64: launch(select_dense_kernel<64>); break;
+        default: launch(select_dense_kernel<128>); break;
+    }
+    launch_dense_units(b, units, 0, (uint32_t)max_units, 1, mfma, d_slots, d_pv, s, n_units);
 }
 
 namespace {
@@ -1270,7 +1202,7 @@ int btc_bitbsr_build(btc_graph g, int32_t tile_k, void* stream, btc_bitbsr* out)
         BTC_REQUIRE(tile_k == 32 || tile_k == 64 || tile_k == 128, BTC_ERR_ARG,
                     "tile width K = %d (expected 32, 64 or 128)", tile_k);
         auto b = std::make_unique<btc_bitbsr_s>();
-        btcx::bitbsr_build(g, tile_k, btcx::as_stream(stream), b.get());
+        btcx::bitbsr_build(g, tile_k, btcx::as_stream(stream), b.get(), true);
         BTC_HIP(hipStreamSynchronize(btcx::as_stream(stream)));
         *out = b.release();
     });
@@ -1311,6 +1243,15 @@ void btc_bitbsr_free(btc_bitbsr b) { delete b; }
 
 namespace {
 
+// With no threshold given, graphs whose merge work (the sum of d(i) + d(j)
+// over the edges) is below this count every tile row by row: the dense part
+// is two more kernels and an allocation in front of the rows.  Planted
+// communities (16 x 32 / 16 x 128 tiles, us with the dense part against rows
+// only): work 19 M 112 / 123 against 72, 75 M 155 / 152 against 105, 151 M
+// 203 / 175 against 165, 301 M 246 / 242 against 239 / 266, 874 M 279 / 312
+// against 423.
+constexpr int64_t kDenseMinWork = int64_t(1) << 28;
+
 // btc_bitbsr_count with per-vertex output to int32 (pv32) or int64 (pv64).
 void bitbsr_count(btc_bitbsr b, int32_t variant, int32_t threshold_blocks, int32_t tau, void* stream,
                   uint64_t* total, int32_t* pv32, int64_t* pv64, float* kernel_ms) {
@@ -1320,22 +1261,34 @@ void bitbsr_count(btc_bitbsr b, int32_t variant, int32_t threshold_blocks, int32
     BTC_REQUIRE(variant >= BTC_VARIANT_AUTO && variant <= BTC_VARIANT_DIRECT, BTC_ERR_ARG,
                 "unknown variant %d", variant);
     hipStream_t s = btcx::as_stream(stream);
-    if (tau < 0) tau = btc_default_tau(b->K);
-    if (threshold_blocks <= 0) threshold_blocks = b->K == 128 ? 2048 : 40000;
-    const bool bs = variant == BTC_VARIANT_BINSEARCH ||
-                    (variant == BTC_VARIANT_AUTO && b->nblk < (uint32_t)threshold_blocks);
+    if (tau < 0)
+        tau = mfma || b->rows.merge_work >= kDenseMinWork ? btc_default_tau(b->K) : 16 * b->K;
+    (void)threshold_blocks;  // both variants find a tile's row block the same way here
+    BTC_REQUIRE(b->nblk == 0 || btcx::lane_sums_fit(b->max_row, b->K), BTC_ERR_OVERFLOW,
+                "longest row %d: a lane's 32-bit sum over %d tile columns could overflow", b->max_row, b->K / 4);
     btcx::PvBuf pv;
     if (pv32 || pv64) {
         pv.alloc((size_t)b->n, b->max_row);
         BTC_HIP(hipMemsetAsync(pv.data(), 0, pv.bytes(), s));
     }
-    BTC_HIP(hipMemsetAsync(b->result.p, 0, 8, s));
+    btcx::TmpBuf<uint4> units;
+    uint64_t max_units = 0;
+    if (b->rows.count[3] > (uint32_t)tau) {
+        // every dense tile holds more than tau entries, every unit one
+        const uint64_t m = (uint64_t)b->rows.m;
+        max_units = std::min<uint64_t>(std::min<uint64_t>(b->nblk, m / ((uint64_t)tau + 1)) * (uint64_t)(b->K / 16), m);
+        units.alloc(2 * max_units, s);
+    }
     btcx::EventTimer tm(kernel_ms != nullptr);
+    btcx::launch_zero_u32(reinterpret_cast<uint32_t*>(b->work.p), 2 * btcx::kWorkWords, s);
     tm.start(s);
-    btcx::launch_tile_count(b, nullptr, b->nblk, bs, mfma, tau, b->result.p, pv.out(), s);
+    unsigned long long* slots = b->work.p + btcx::kWorkSlots;
+    if (units.p) btcx::launch_dense_part(b, tau, mfma, units.p, max_units, slots, pv.out(), s);
+    btcx::launch_rows(b->rows, tau, slots, pv.out(), s);
+    btcx::launch_slot_sum(slots, b->work.p, s);
     tm.stop(s);
     unsigned long long h = 0;
-    BTC_HIP(hipMemcpyAsync(&h, b->result.p, 8, hipMemcpyDeviceToHost, s));
+    BTC_HIP(hipMemcpyAsync(&h, b->work.p, 8, hipMemcpyDeviceToHost, s));
     pv.copy_out(pv32, pv64, s);  // synchronises s
     if (kernel_ms) *kernel_ms = tm.ms();
     *total = h;

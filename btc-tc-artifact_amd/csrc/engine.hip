@@ -3,8 +3,8 @@
 // sum over (i, j) in L of |N_L(i) & N_L(j)| is split by edge:
 //
 //  * edges inside dense 16 x K mask tiles (popcount > tau) go through the
-//    Bit-BSR tile path (launch_tile_count with a list of dense tiles, every
-//    tile on the dense AND+popcount path);
+//    Bit-BSR tile path (launch_dense_units: AND + popcount or i8 MFMA
+//    over matched tile pairs);
 //
 //  * every other edge (i, j) is evaluated as the wedges (i; j, k) with k a
 //    neighbour of i below j: k is in N_L(j) exactly when (i, j, k) is a

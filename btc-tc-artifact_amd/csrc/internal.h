@@ -6,6 +6,24 @@
 #include "common.h"
 #include "prim.h"
 
+namespace btcx {
+
+// The rows of L beside a Bit-BSR's tiles (rowcount.hip): a copy of its CSR
+// and the work items of the rows, by class (light, wave, workgroup).
+struct RowLists {
+    DevBuf<unsigned char> block;  // everything below
+    uint4* items = nullptr;       // {t0, t1, first list, row}; classes at 0, cap0, cap0 + cap1
+    uint64_t cap0 = 0, cap1 = 0;
+    uint32_t* rowptr = nullptr;   // n + 1
+    int32_t* col = nullptr;       // m + kColPad
+    uint16_t* epop = nullptr;     // m: set bits of the entry's tile (16 x 128 at most)
+    uint32_t* d_count = nullptr;  // items per class, then the largest tile popcount
+    uint32_t count[4] = {0, 0, 0, 0};  // d_count once it has been read back
+    int64_t m = 0, merge_work = 0;
+};
+
+}  // namespace btcx
+
 // Bit-BSR of L with 16 x K tiles (K in {32, 64, 128}); see btc_amd.h.
 struct btc_bitbsr_s {
     int32_t n = 0;
@@ -18,7 +36,10 @@ struct btc_bitbsr_s {
     btcx::DevBuf<uint32_t> indices;      // nblk
     btcx::DevBuf<uint32_t> row_indices;  // nblk
     btcx::DevBuf<uint64_t> tiles;        // nblk * wpt
-    btcx::DevBuf<unsigned long long> result;
+    // handles made for counting only (btc_bitbsr_build)
+    btcx::RowLists rows;
+    btcx::DevBuf<uint32_t> pop;  // nblk: set bits of every tile
+    btcx::DevBuf<unsigned long long> work;  // kWorkWords: [0] total, slots
 };
 
 struct btc_pipeline_s;
@@ -325,8 +346,9 @@ void ensure_device(btc_graph_s* g, hipStream_t s);
 // out[0..n) = exclusive prefix sum of in[0..n), out[n] = total (u64).
 void scan_u32_to_u64(const uint32_t* in, uint64_t* out, size_t n, hipStream_t s);
 
-// Builds the 16 x K Bit-BSR of g on `s` into b (b's buffers are replaced).
-void bitbsr_build(btc_graph_s* g, int K, hipStream_t s, btc_bitbsr_s* b);
+// Builds the 16 x K Bit-BSR of g on `s` into b (b's buffers are replaced);
+// with `counted`, what btc_bitbsr_count reads beside the tiles as well.
+void bitbsr_build(btc_graph_s* g, int K, hipStream_t s, btc_bitbsr_s* b, bool counted = false);
 
 // Sets p->bsr to the plan's Bit-BSR of width K: the caller's when the plan
 // was made on one, else one built on s.  drop_plan_bsr releases it.
@@ -345,14 +367,14 @@ inline void drop_plan_bsr(btc_plan_s* p) {
     p->bsr = nullptr;
 }
 
-// Count over mask tiles of b.  tile_list (device) selects ntiles mask tiles,
-// or all tiles when NULL (list entries lstride apart: tile_list[w * lstride]).
-// tau < 0 sends every tile down the dense path; mfma selects the i8 MFMA
-// form of the dense path over AND + popcount.  Adds the total to *d_result
-// and per-row sums to d_pv (when it is on).
-void launch_tile_count(const btc_bitbsr_s* b, const uint32_t* tile_list, uint32_t ntiles,
-                       bool binsearch, bool mfma, int tau, unsigned long long* d_result, PvOut d_pv,
-                       hipStream_t s, uint32_t lstride = 1);
+// Enqueues the copy of g's CSR and the row items on s; r.count is valid once
+// d_count has been read back.
+void build_row_lists(const btc_graph_s* g, RowLists& r, hipStream_t s);
+
+// Counts the mask bits outside dense tiles (those of more than tau bits) row
+// by row, adding into the kSlots slots at d_slots and per-vertex sums into pv
+// when it is on.
+void launch_rows(const RowLists& r, int tau, unsigned long long* d_slots, PvOut pv, hipStream_t s);
 
 // Units of the dense tiles list[0, nt) of Bit-BSR b (one per tile slab with
 // mask bits over a row block that has tile columns) into `units`; returns
@@ -362,9 +384,17 @@ uint32_t build_dense_units(const btc_bitbsr_s* b, const uint32_t* list, uint32_t
 
 // Counts dense units first + w * stride, w in [0, count), of Bit-BSR b: the
 // engine's dense-tile path (i8 MFMA or AND + popcount), adding into the
-// kSlots slots at d_slots and per-vertex sums into d_pv when it is on.
+// kSlots slots at d_slots and per-vertex sums into d_pv when it is on.  With
+// d_count (stride 1), only the units below *d_count.
 void launch_dense_units(const btc_bitbsr_s* b, const uint4* units, uint32_t first, uint32_t count, uint32_t stride,
-                        bool mfma, unsigned long long* d_slots, PvOut d_pv, hipStream_t s);
+                        bool mfma, unsigned long long* d_slots, PvOut d_pv, hipStream_t s,
+                        const uint32_t* d_count = nullptr);
+
+// The dense part of one count of a Bit-BSR handle: tiles of more than tau
+// bits as units (room for max_units in `units`), counted into the slots that
+// lie kWorkSlots words into the count's cleared work words.
+void launch_dense_part(const btc_bitbsr_s* b, int tau, bool mfma, uint4* units, uint64_t max_units,
+                       unsigned long long* d_slots, PvOut d_pv, hipStream_t s);
 
 // *d_result += sum of the kSlots slots at d_slots, which are cleared.
 void launch_slot_sum(unsigned long long* d_slots, unsigned long long* d_result, hipStream_t s);
