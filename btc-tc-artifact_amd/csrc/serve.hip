@@ -6,6 +6,7 @@
 //             them as one block-diagonal unit (a single graph is planned on
 //             its own); admission keeps the resident set under the HBM
 //             budget, evicting idle units least recently used first
+//             (kResidentGrace after they became resident at the earliest)
 //          -> [GPU worker] every ready request joins the next launch: the
 //             single-graph units in one persistent wedge-kernel launch over
 //             all of their plans, each multi-graph unit in one launch that
@@ -59,6 +60,11 @@ constexpr int64_t kPipeCacheBytes = int64_t(4) << 30;
 // Captured preparation turns to groups beyond this many queued graphs per
 // prep thread.
 constexpr size_t kBacklogPerThread = 8;
+// A unit stays resident this long at least, so that a request by key right
+// behind the graph's submission finds it however fast units are prepared.
+// It delays only budgets that preparation turns over within that time (1 GiB
+// in 10 ms is several times its rate).
+constexpr std::chrono::milliseconds kResidentGrace{10};
 
 int64_t pow2_at_least(int64_t x, int64_t lo) {
     int64_t c = lo;
@@ -131,6 +137,7 @@ struct Unit {  // what is prepared, resident and evicted together
     int64_t bytes = 0;
     std::list<Unit*>::iterator lru;
     bool in_lru = false;
+    Clock::time_point published{};
     Unit() = default;
     Unit(const Unit&) = delete;
     Unit& operator=(const Unit&) = delete;
@@ -202,14 +209,15 @@ struct btc_server_s {
         return true;
     }
 
-    // Caller holds mu.  Evicts idle resident units (LRU first) until `need`
+    // Caller holds mu.  Evicts idle resident units past their grace (LRU
+    // first) until `need`
     // more bytes fit; returns whether they fit.
     bool make_room(int64_t need) {
         auto it = lru.end();
         while (resident_bytes + need > opts.hbm_budget_bytes && it != lru.begin()) {
             --it;
             Unit* u = *it;
-            if (!unit_idle(u)) continue;
+            if (!unit_idle(u) || Clock::now() - u->published < kResidentGrace) continue;
             resident_bytes -= u->bytes;
             it = lru.erase(it);
             const std::vector<uint64_t> keys = u->keys;
@@ -254,6 +262,7 @@ struct btc_server_s {
         lru.push_front(u.get());
         u->lru = lru.begin();
         u->in_lru = true;
+        u->published = Clock::now();
         for (size_t k = 0; k < u->keys.size(); ++k) {
             const uint64_t key = u->keys[k];
             Entry& e = cache[key];
@@ -527,7 +536,8 @@ struct btc_server_s {
     // them; false when the server stops meanwhile.
     bool admit(int64_t est) {
         std::unique_lock<std::mutex> lk(mu);
-        cv_prep.wait(lk, [&] { return stop || make_room(est) || resident_bytes == 0; });
+        // woken by unpinned units; a unit's grace ends without a signal
+        while (!(stop || make_room(est) || resident_bytes == 0)) cv_prep.wait_for(lk, std::chrono::milliseconds(1));
         if (stop) return false;
         resident_bytes += est;  // reserved until the unit's real size is known
         return true;
