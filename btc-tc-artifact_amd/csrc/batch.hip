@@ -95,7 +95,7 @@ __global__ void item_graphs_kernel(uint4* __restrict__ items, uint32_t nitems, c
 // the zeroed sums the wedge and tiny kernels add to.
 void batch_item_graphs(btc_batch_s* b, hipStream_t s) {
     btc_plan_s* p = b->plan;
-    b->d_gsum.alloc((size_t)b->count);
+    b->d_gsum.alloc_on((size_t)b->count, s);
     BTC_HIP(hipMemsetAsync(b->d_gsum.p, 0, (size_t)b->count * 8, s));
     if (p->nitems) {
         TmpBuf<uint32_t> lseg;
@@ -148,9 +148,9 @@ void batch_finish(btc_batch_s* b, const btc_count_opts* opts, hipStream_t s) {
     const btc_count_opts o = batch_opts(opts);
     check_status(btc_plan_create(&b->graph, &o, s, &b->plan));
     std::vector<uint32_t> vo32(b->voff.begin(), b->voff.end());
-    b->d_voff.alloc(vo32.size());
-    b->d_pv.alloc((size_t)b->graph.n, b->graph.max_row);
-    b->d_pg.alloc((size_t)b->count);
+    b->d_voff.alloc_on(vo32.size(), s);
+    b->d_pv.alloc_on((size_t)b->graph.n, b->graph.max_row, s);
+    b->d_pg.alloc_on((size_t)b->count, s);
     b->h_pg.assign((size_t)b->count, 0);
     BTC_HIP(hipMemcpyAsync(b->d_voff.p, vo32.data(), vo32.size() * 4, hipMemcpyHostToDevice, s));
     batch_item_graphs(b, s);
@@ -178,9 +178,9 @@ btc_batch_s* batch_from_plan(btc_graph_s&& g, btc_plan_s* plan, const std::vecto
     b->plan = own.release();
     b->plan->g = &b->graph;
     std::vector<uint32_t> vo32(voff.begin(), voff.end());
-    b->d_voff.alloc(vo32.size());
-    b->d_pv.alloc((size_t)b->graph.n, b->graph.max_row);
-    b->d_pg.alloc((size_t)b->count);
+    b->d_voff.alloc_on(vo32.size(), s);
+    b->d_pv.alloc_on((size_t)b->graph.n, b->graph.max_row, s);
+    b->d_pg.alloc_on((size_t)b->count, s);
     b->h_pg.assign((size_t)b->count, 0);
     BTC_HIP(hipMemcpyAsync(b->d_voff.p, vo32.data(), vo32.size() * 4, hipMemcpyHostToDevice, s));
     batch_item_graphs(b.get(), s);

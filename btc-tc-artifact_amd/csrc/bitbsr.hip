@@ -34,8 +34,8 @@ void ensure_device(btc_graph_s* g, hipStream_t s) {
                 "nnz(L) = %lld needs 64-bit row offsets (limit 2^32 - 1)", (long long)g->m);
     std::vector<uint32_t> rp32((size_t)g->n + 1);
     for (size_t i = 0; i < rp32.size(); ++i) rp32[i] = (uint32_t)g->rowptr[i];
-    g->d_rowptr.alloc(rp32.size());
-    g->d_col.alloc((size_t)g->m + kColPad);
+    g->d_rowptr.alloc_on(rp32.size(), s);
+    g->d_col.alloc_on((size_t)g->m + kColPad, s);
     BTC_HIP(hipMemsetAsync(g->d_col.p + g->m, 0, kColPad * 4, s));
     BTC_HIP(hipMemcpyAsync(g->d_rowptr.p, rp32.data(), rp32.size() * 4, hipMemcpyHostToDevice, s));
     if (g->m)
@@ -335,14 +335,14 @@ void build_impl(btc_graph_s* g, hipStream_t s, btc_bitbsr_s* b, bool counted) {
     BTC_REQUIRE(nblk < 0xFFFFFFFFull, BTC_ERR_OVERFLOW, "%llu tiles exceed the u32 tile index",
                 (unsigned long long)nblk);
     b->nblk = (uint32_t)nblk;
-    b->indptr.alloc((size_t)n_rb + 1);
-    b->indices.alloc(nblk);
-    b->row_indices.alloc(nblk);
-    b->tiles.alloc(nblk * (size_t)b->wpt);
+    b->indptr.alloc_on((size_t)n_rb + 1, s);
+    b->indices.alloc_on(nblk, s);
+    b->row_indices.alloc_on(nblk, s);
+    b->tiles.alloc_on(nblk * (size_t)b->wpt, s);
     if (counted) {
         build_row_lists(g, b->rows, s);
-        b->pop.alloc(nblk);
-        b->work.alloc(kWorkWords);
+        b->pop.alloc_on(nblk, s);
+        b->work.alloc_on(kWorkWords, s);
     }
     hipLaunchKernelGGL(narrow_u64_to_u32, dim3((unsigned)((n_rb + 1 + 255) / 256)), dim3(256), 0, s, offs.p,
                        b->indptr.p, (size_t)n_rb + 1);
@@ -1081,7 +1081,7 @@ uint32_t build_dense_units(const btc_bitbsr_s* b, const uint32_t* list, uint32_t
     BTC_HIP(hipStreamSynchronize(s));
     BTC_REQUIRE(nu < 0xFFFFFFFFull, BTC_ERR_OVERFLOW, "%llu dense units exceed a u32 index", (unsigned long long)nu);
     if (nu == 0) return 0;
-    units.alloc(2 * nu);
+    units.alloc_on(2 * nu, s);
     switch (b->K) {
         case 32: launch(dense_units_kernel<32, true>, order, units.p); break;
         case 64: launch(dense_units_kernel<64, true>, order, units.p); break;
@@ -1268,7 +1268,7 @@ void bitbsr_count(btc_bitbsr b, int32_t variant, int32_t threshold_blocks, int32
                 "longest row %d: a lane's 32-bit sum over %d tile columns could overflow", b->max_row, b->K / 4);
     btcx::PvBuf pv;
     if (pv32 || pv64) {
-        pv.alloc((size_t)b->n, b->max_row);
+        pv.alloc_on((size_t)b->n, b->max_row, s);
         BTC_HIP(hipMemsetAsync(pv.data(), 0, pv.bytes(), s));
     }
     btcx::TmpBuf<uint4> units;
@@ -1290,6 +1290,7 @@ void bitbsr_count(btc_bitbsr b, int32_t variant, int32_t threshold_blocks, int32
     unsigned long long h = 0;
     BTC_HIP(hipMemcpyAsync(&h, b->work.p, 8, hipMemcpyDeviceToHost, s));
     pv.copy_out(pv32, pv64, s);  // synchronises s
+    pv.release_on(s);
     if (kernel_ms) *kernel_ms = tm.ms();
     *total = h;
 }

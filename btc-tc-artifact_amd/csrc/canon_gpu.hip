@@ -465,10 +465,10 @@ void canonicalise_device(const int32_t* src, const int32_t* dst, int64_t nnz, in
         BTC_HIP(hipMemcpyAsync(&hn, newid.p + n, 4, hipMemcpyDeviceToHost, s));
         BTC_HIP(hipStreamSynchronize(s));
         nc = (int32_t)hn;
-        labels.alloc((size_t)nc);
+        labels.alloc_on((size_t)nc, s);
         BTC_LAUNCH(labels_kernel, n, s, used.p, newid.p, n, labels.p);
     } else {
-        labels.alloc((size_t)n);
+        labels.alloc_on((size_t)n, s);
         BTC_LAUNCH(iota_kernel, n, s, labels.p, (int64_t)n);
     }
     const int bn = id_bits(nc);
@@ -502,7 +502,7 @@ void canonicalise_device(const int32_t* src, const int32_t* dst, int64_t nnz, in
         k1.alloc((size_t)nc, s);
         v1.alloc((size_t)nc, s);
         rank.alloc((size_t)nc, s);
-        lab2.alloc((size_t)nc);
+        lab2.alloc_on((size_t)nc, s);
         BTC_HIP(hipMemsetAsync(deg.p, 0, (size_t)nc * 4, s));
         if (m) {
             hipLaunchKernelGGL(degree_kernel, dim3(std::min(grid_for(m), kRedBlocks)), dim3(kT), 0, s, keys, m, bn, deg.p);
@@ -532,8 +532,8 @@ void canonicalise_device(const int32_t* src, const int32_t* dst, int64_t nnz, in
     // CSR of L
     g->n = nc;
     g->m = m;
-    g->d_rowptr.alloc((size_t)nc + 1);
-    g->d_col.alloc((size_t)m + kColPad);
+    g->d_rowptr.alloc_on((size_t)nc + 1, s);
+    g->d_col.alloc_on((size_t)m + kColPad, s);
     BTC_LAUNCH(csr_kernel, std::max<int64_t>((int64_t)nc + 1, m + (int64_t)kColPad), s, keys, m, bn, nc,
                g->d_rowptr.p, g->d_col.p, (uint16_t*)nullptr);
     g->d_labels = std::move(labels);

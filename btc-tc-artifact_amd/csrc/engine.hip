@@ -667,7 +667,7 @@ __global__ void narrow_col_kernel(const int32_t* __restrict__ col, Cnt n_, uint1
 
 void build_col16(btc_plan_s* p, hipStream_t s) {
     const uint32_t n = (uint32_t)p->g->m + (uint32_t)kColPad;
-    p->col16.alloc(n);
+    p->col16.alloc_on(n, s);
     const unsigned grid = std::min<unsigned>((n + kThreads - 1) / kThreads, 1u << 16);
     hipLaunchKernelGGL(narrow_col_kernel, dim3(grid), dim3(kThreads), 0, s, p->g->d_col.p, n, p->col16.p);
     BTC_CHECK_LAUNCH("narrow_col_kernel");
@@ -722,7 +722,7 @@ void classify_dense_host(btc_plan_s* p, hipStream_t s, std::vector<uint8_t>& den
     plan_bsr(p, s);
     BTC_REQUIRE(p->bsr->nblk == ntiles[n_rb], BTC_ERR_STATE, "tile count mismatch (%u vs %u)", p->bsr->nblk,
                 ntiles[n_rb]);
-    p->dense_list.alloc(list.size());
+    p->dense_list.alloc_on(list.size(), s);
     BTC_HIP(hipMemcpyAsync(p->dense_list.p, list.data(), list.size() * 4, hipMemcpyHostToDevice, s));
     BTC_HIP(hipStreamSynchronize(s));
 }
@@ -737,7 +737,7 @@ void classify_dense(btc_plan_s* p, hipStream_t s, std::vector<uint8_t>& dense) {
     }
     const btc_bitbsr_s* b = plan_bsr(p, s);
     DevBuf<uint32_t> d_pop;
-    d_pop.alloc(b->nblk);
+    d_pop.alloc_on(b->nblk, s);
     launch_tile_popcount(b, d_pop.p, s);
     std::vector<uint32_t> pop(b->nblk), indptr((size_t)b->n_rb + 1), indices(b->nblk);
     BTC_HIP(hipMemcpyAsync(pop.data(), d_pop.p, (size_t)b->nblk * 4, hipMemcpyDeviceToHost, s));
@@ -770,7 +770,7 @@ void classify_dense(btc_plan_s* p, hipStream_t s, std::vector<uint8_t>& dense) {
             dense[q] = (int)pop[f - indices.data()] > p->tau;
         }
     }
-    p->dense_list.alloc(list.size());
+    p->dense_list.alloc_on(list.size(), s);
     BTC_HIP(hipMemcpyAsync(p->dense_list.p, list.data(), list.size() * 4, hipMemcpyHostToDevice, s));
     BTC_HIP(hipStreamSynchronize(s));
 }
@@ -923,7 +923,7 @@ void build_wedge_lists(btc_plan_s* p, const std::vector<uint8_t>& dense, int64_t
     std::memcpy(host.data() + ib, lst.data(), lb);
     std::memcpy(host.data() + ib + lb, rowbits.data(), bb);
     std::memcpy(host.data() + ib + lb + bb, ur.data(), rb);
-    p->lists.alloc(host.size());
+    p->lists.alloc_on(host.size(), s);
     if (!host.empty())
         BTC_HIP(hipMemcpyAsync(p->lists.p, host.data(), host.size(), hipMemcpyHostToDevice, s));
     p->items_p = reinterpret_cast<const uint4*>(p->lists.p);
@@ -1129,8 +1129,8 @@ void pipeline_count_enqueue(const PlanCap& c, const uint16_t* col16, const btc_c
 
 void plans_count(btc_plan_s* const* P, int k, hipStream_t s, uint64_t* totals, MultiWorkspace& ws) {
     if (k <= 0) return;
-    if (ws.totals.n < (size_t)k) ws.totals.alloc((size_t)k);
-    if (ws.counters.n < 2) ws.counters.alloc(2);
+    if (ws.totals.n < (size_t)k) ws.totals.alloc_on((size_t)k, s);
+    if (ws.counters.n < 2) ws.counters.alloc_on(2, s);
     BTC_HIP(hipMemsetAsync(ws.totals.p, 0, (size_t)k * 8, s));
     BTC_HIP(hipMemsetAsync(ws.counters.p, 0, 8, s));
     std::vector<PlanDev> pd((size_t)k);
@@ -1162,8 +1162,8 @@ void plans_count(btc_plan_s* const* P, int k, hipStream_t s, uint64_t* totals, M
                 for (uint32_t li = P[j]->n_block_items; li < P[j]->nitems; ++li)
                     ws.h_map.push_back(make_uint2((uint32_t)j, li));
             const size_t pbytes = pd.size() * sizeof(PlanDev);
-            if (ws.plans.n < pbytes) ws.plans.alloc(pbytes);
-            if (ws.map.n < ni) ws.map.alloc(ni);
+            if (ws.plans.n < pbytes) ws.plans.alloc_on(pbytes, s);
+            if (ws.map.n < ni) ws.map.alloc_on(ni, s);
             BTC_HIP(hipMemcpyAsync(ws.plans.p, pd.data(), pbytes, hipMemcpyHostToDevice, s));
             BTC_HIP(hipMemcpyAsync(ws.map.p, ws.h_map.data(), (size_t)ni * sizeof(uint2), hipMemcpyHostToDevice, s));
             a.plans = reinterpret_cast<const PlanDev*>(ws.plans.p);
@@ -1262,7 +1262,7 @@ void plan_count(btc_plan_s* p, hipStream_t s, uint64_t* total, int32_t* pv32, in
     }
     PvBuf pv;
     if (per_vertex) {
-        pv.alloc((size_t)g->n, g->max_row);
+        pv.alloc_on((size_t)g->n, g->max_row, s);
         BTC_HIP(hipMemsetAsync(pv.data(), 0, pv.bytes(), s));
     }
     EventTimer tm(kernel_ms != nullptr), tw(kernel_ms != nullptr);
@@ -1270,6 +1270,7 @@ void plan_count(btc_plan_s* p, hipStream_t s, uint64_t* total, int32_t* pv32, in
     unsigned long long h = 0;
     BTC_HIP(hipMemcpyAsync(&h, p->scratch.p, 8, hipMemcpyDeviceToHost, s));
     pv.copy_out(pv32, pv64, s);  // synchronises s
+    pv.release_on(s);
     if (kernel_ms) {
         *kernel_ms = tm.ms();
         p->last_wedge_ms = tw.ms();
@@ -1349,7 +1350,7 @@ btc_plan_s* plan_create(btc_graph g, const btc_count_opts* opts, hipStream_t s, 
         btcx::build_wedge_lists(p.get(), dense, chunk, s);
     }
     if (p->n_dense) p->n_units = btcx::build_dense_units(p->bsr, p->dense_list.p, p->n_dense, p->dense_units, s);
-    p->scratch.alloc(btcx::kWorkWords);
+    p->scratch.alloc_on(btcx::kWorkWords, s);
     BTC_HIP(hipMemsetAsync(p->scratch.p, 0, p->scratch.bytes(), s));
     BTC_HIP(hipStreamSynchronize(s));  // counts may run on other streams (every count clears these words again)
     p->info.tile_k = p->K;

@@ -175,7 +175,7 @@ void layout(btc_pipeline_s* p, Carve& c) {
 void pipeline_build(btc_pipeline_s* p, hipStream_t s) {
     Carve sizing;
     layout(p, sizing);
-    p->mem.alloc(sizing.top);
+    p->mem.alloc_on(sizing.top, s);
     Carve real;
     real.base = p->mem.p;
     layout(p, real);
@@ -391,7 +391,7 @@ void pipeline_copy_locked(btc_pipeline_s* p, hipStream_t s, bool with_plan, btc_
     };
     Carve sizing;
     carve(sizing);
-    g->block.alloc(sizing.top);
+    g->block.alloc_on(sizing.top, s);
     Carve real;
     real.base = g->block.p;
     carve(real);

@@ -392,7 +392,7 @@ void plan_device(btc_plan_s* p, int64_t chunk, hipStream_t s) {
         exclusive_scan_u32(flag.p, pos.p, b->nblk, s);
         const uint32_t nd = read_dev(pos.p + b->nblk, s);
         if (nd) {
-            p->dense_list.alloc(nd);
+            p->dense_list.alloc_on(nd, s);
             BTC_LAUNCH(select_kernel, b->nblk, s, flag.p, pos.p, (int64_t)b->nblk, p->dense_list.p);
             dense.alloc((size_t)m, s);
             BTC_LAUNCH(dense_edges_kernel, m, s, col, erow.p, m, p->K, b->indptr.p, b->indices.p, pop.p, p->tau,
@@ -440,7 +440,7 @@ void plan_device(btc_plan_s* p, int64_t chunk, hipStream_t s) {
 
     // one allocation: list records, row bitmaps, list rows; items apart
     const size_t lb = (size_t)ne * sizeof(uint4), bb = (size_t)nbm * (C / 32) * 4, rb = (size_t)ne * 4;
-    p->lists.alloc(lb + bb + rb);
+    p->lists.alloc_on(lb + bb + rb, s);
     uint4* lst = reinterpret_cast<uint4*>(p->lists.p);
     uint32_t* rowbits = reinterpret_cast<uint32_t*>(p->lists.p + lb);
     int32_t* ur = reinterpret_cast<int32_t*>(p->lists.p + lb + bb);
@@ -478,7 +478,7 @@ void plan_device(btc_plan_s* p, int64_t chunk, hipStream_t s) {
         BTC_LAUNCH_RED(items_kernel, nitems, s, rowptr, col, key, off.p, P.p, first.p, nitems, ne,
                    p->use_tiny, p->tiny_all, false, tmp.p, sk0.p, sv0.p, st.p + 4);
     const bool ialt = sort_pairs_u32(sk0.p, sv0.p, sk1.p, sv1.p, nitems, 32, s);
-    p->items_dev.alloc((size_t)nitems * 2);
+    p->items_dev.alloc_on((size_t)nitems * 2, s);
     if (nitems)
         BTC_LAUNCH(place_items_kernel, nitems, s, tmp.p, ialt ? sv1.p : sv0.p, nitems, p->items_dev.p, nullptr,
                    nullptr);

@@ -564,7 +564,7 @@ void build_row_lists(const btc_graph_s* g, RowLists& r, hipStream_t s) {
     r.cap1 = cap1;
     const size_t ib = (size_t)(cap0 + cap1 + cap2) * sizeof(uint4);
     const size_t rb = ((n + 1) * 4 + 255) & ~size_t(255);
-    r.block.alloc(ib + rb + (m + kColPad) * 4 + 16 + m * 2);
+    r.block.alloc_on(ib + rb + (m + kColPad) * 4 + 16 + m * 2, s);
     r.items = reinterpret_cast<uint4*>(r.block.p);
     r.rowptr = reinterpret_cast<uint32_t*>(r.block.p + ib);
     r.col = reinterpret_cast<int32_t*>(r.block.p + ib + rb);

@@ -2,8 +2,12 @@
 // dispatch rules shared by every path.
 #include <algorithm>
 #include <cstdarg>
+#include <chrono>
 #include <cstring>
+#include <exception>
 #include <mutex>
+#include <unordered_map>
+#include <vector>
 
 #include "common.h"
 
@@ -57,7 +61,198 @@ float EventTimer::ms() {
 
 }  // namespace btcx
 
+// ------------------------------------------------------------ device pool
 namespace btcx {
+namespace {
+
+constexpr int kPoolDevices = 64;
+
+// A freed block.  It may be handed out
+//  * for work on the stream its last use was on (stream order), or
+//  * for any work once the device has been synchronised after its release
+//    (released <= the pool's synced count).
+struct FreeBlock {
+    void* p;
+    size_t bytes;
+    hipStream_t s;
+    bool ordered;
+    uint64_t released;  // position among the pool's releases
+    std::chrono::steady_clock::time_point at;
+};
+
+// Bounded three ways: at most kPoolKeep cached bytes per device (3 % of its
+// memory; the oldest blocks go first), blocks that nothing took for
+// kPoolIdle are returned at the next call, and a failing allocation returns
+// every cached block before it is tried once more.
+constexpr size_t kPoolKeep = size_t(8) << 30;
+constexpr std::chrono::seconds kPoolIdle{10};
+
+struct Pool {
+    std::mutex mu;
+    std::vector<FreeBlock> cached;             // oldest release first
+    std::unordered_map<void*, size_t> live;    // bytes of every block handed out
+    size_t cached_bytes = 0;
+    uint64_t releases = 0, synced = 0;
+};
+
+// Never destroyed: buffers of static objects may outlive any order of
+// destruction, and the driver takes the memory back with the process.
+Pool* const g_pools = new Pool[kPoolDevices];
+
+int pool_device() {
+    int dev = 0;
+    BTC_HIP(hipGetDevice(&dev));
+    BTC_REQUIRE(dev >= 0 && dev < kPoolDevices, BTC_ERR_ARG, "device %d: memory is kept for devices 0-%d", dev,
+                kPoolDevices - 1);
+    return dev;
+}
+
+// Sizes are rounded up to eighths of a power of two (at least 512 bytes), up
+// to 64 MiB, so that inputs of about one size share blocks; larger ones to
+// 2 MiB.
+size_t pool_round(size_t bytes) {
+    if (bytes <= 512) return 512;
+    if (bytes > (size_t(64) << 20)) return (bytes + (size_t(2) << 20) - 1) & ~((size_t(2) << 20) - 1);
+    size_t p2 = 512;
+    while (p2 * 2 < bytes) p2 *= 2;
+    const size_t step = std::max<size_t>(p2 / 8, 256);
+    return (bytes + step - 1) / step * step;
+}
+
+// Waits for the device.  In the relaxed capture mode, since the thread may
+// not refuse the wait because of a capture elsewhere in the process.
+bool device_wait() {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool swapped = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    const hipError_t e = hipDeviceSynchronize();
+    if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e == hipSuccess;
+}
+
+// Takes the best cached block for `want` bytes (at most an eighth larger,
+// or twice up to 64 KiB), or NULL.  *waits: a block would fit if the device
+// were synchronised.
+void* pool_take(Pool& q, size_t want, bool ordered, hipStream_t s, bool* waits) {
+    const size_t most = want <= (size_t(64) << 10) ? 2 * want : want + want / 8;
+    size_t best = q.cached.size();
+    int best_rank = 3;
+    *waits = false;
+    for (size_t k = q.cached.size(); k-- > 0;) {
+        const FreeBlock& b = q.cached[k];
+        if (b.bytes < want || b.bytes > most) continue;
+        const bool same = ordered && b.ordered && b.s == s;
+        const bool idle = b.released <= q.synced;
+        if (!same && !idle) {
+            *waits = true;
+            continue;
+        }
+        const int rank = b.bytes == want ? 0 : 1;
+        if (rank < best_rank) {
+            best = k;
+            best_rank = rank;
+            if (rank == 0) break;
+        }
+    }
+    if (best == q.cached.size()) return nullptr;
+    const FreeBlock b = q.cached[best];
+    q.cached.erase(q.cached.begin() + (std::ptrdiff_t)best);
+    q.cached_bytes -= b.bytes;
+    q.live[b.p] = b.bytes;
+    return b.p;
+}
+
+// Blocks to give back now: idle for kPoolIdle, or the oldest beyond keep
+// bytes.
+std::vector<void*> pool_trim(Pool& q, size_t keep) {
+    std::vector<void*> out;
+    const auto now = std::chrono::steady_clock::now();
+    size_t k = 0;
+    while (k < q.cached.size() && (q.cached_bytes > keep || now - q.cached[k].at > kPoolIdle)) {
+        out.push_back(q.cached[k].p);
+        q.cached_bytes -= q.cached[k].bytes;
+        ++k;
+    }
+    q.cached.erase(q.cached.begin(), q.cached.begin() + (std::ptrdiff_t)k);
+    return out;
+}
+
+void give_back(const std::vector<void*>& blocks) {
+    for (void* p : blocks) (void)hipFree(p);  // waits for work that still uses it
+}
+
+}  // namespace
+
+void* pool_alloc(size_t bytes, bool ordered, hipStream_t s) {
+    const size_t want = pool_round(bytes);
+    Pool& q = g_pools[pool_device()];
+    std::vector<void*> old;
+    void* p = nullptr;
+    {
+        std::unique_lock<std::mutex> lk(q.mu);
+        bool waits = false;
+        p = pool_take(q, want, ordered, s, &waits);
+        if (!p && waits) {
+            const uint64_t upto = q.releases;
+            lk.unlock();
+            const bool ok = device_wait();
+            lk.lock();
+            if (ok) {
+                q.synced = std::max(q.synced, upto);
+                p = pool_take(q, want, ordered, s, &waits);
+            }
+        }
+        old = pool_trim(q, kPoolKeep);
+    }
+    give_back(old);
+    if (p) return p;
+    hipError_t e = hipMalloc(&p, want);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        {
+            std::lock_guard<std::mutex> lk(q.mu);
+            old = pool_trim(q, 0);
+        }
+        give_back(old);
+        e = hipMalloc(&p, bytes);
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            fail(BTC_ERR_NOMEM, "hipMalloc of %zu bytes failed: %s", bytes, hipGetErrorString(e));
+        }
+        std::lock_guard<std::mutex> lk(q.mu);
+        q.live[p] = bytes;
+        return p;
+    }
+    std::lock_guard<std::mutex> lk(q.mu);
+    q.live[p] = want;
+    return p;
+}
+
+void pool_free(void* p, bool ordered, hipStream_t s) {
+    if (!p) return;
+    // a buffer of a call that failed half-way: work may be left on any stream
+    if (std::uncaught_exceptions() > 0) ordered = false;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) dev = 0;
+    std::vector<void*> old;
+    for (int k = 0; k < kPoolDevices; ++k) {
+        Pool& q = g_pools[(dev + k) % kPoolDevices];  // the current device's almost always
+        std::lock_guard<std::mutex> lk(q.mu);
+        const auto it = q.live.find(p);
+        if (it == q.live.end()) continue;
+        const size_t bytes = it->second;
+        q.live.erase(it);
+        if (bytes > kPoolKeep / 4) {  // one block does not crowd out the rest
+            old.push_back(p);
+        } else {
+            q.cached.push_back({p, bytes, s, ordered, ++q.releases, std::chrono::steady_clock::now()});
+            q.cached_bytes += bytes;
+            old = pool_trim(q, kPoolKeep);
+        }
+        break;
+    }
+    give_back(old);
+}
 
 void mem_pool_init() {
     static std::once_flag once[64];
