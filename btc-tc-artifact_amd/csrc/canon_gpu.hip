@@ -11,9 +11,8 @@
 // made only when a host consumer asks (ensure_host).
 #include <climits>
 
-#include "device_util.h"
+#include "devtile.h"
 #include "internal.h"
-#include "prim.h"
 
 namespace btcx {
 namespace {
@@ -133,36 +132,58 @@ __global__ void relabel_kernel(uint64_t* __restrict__ keys, Cnt m_, int b, const
 // column c = k & mask).  Rows come in runs, so a wave adds each run of its
 // 64 keys with one atomic; columns of ids below kDegWindow (where hub
 // vertices of skewed graphs concentrate) are counted in LDS first, so a hub
-// gets one global atomic per workgroup rather than one per edge.
+// gets one global atomic per workgroup rather than one per edge.  The sums
+// are kept in kDegCopies copies (`stride` words apart), one per XCD as
+// workgroups are dealt to them in turn, since a line that eight L2 caches
+// want moves between them.  Bound: the L2's atomic rate on scattered words
+// (some 19 G/s).  One copy and one run of 64 keys at a time against this:
+// R-MAT 2^20 (14 M edges) 873 -> 541 us, 24 graphs (3.3 M) 280 -> 159 us.
 constexpr uint32_t kDegWindow = 8192;
 
-__global__ __launch_bounds__(kT) void degree_kernel(const uint64_t* __restrict__ keys, Cnt m_, int b,
-                                                    uint32_t* __restrict__ deg) {
-    __shared__ uint32_t h[kDegWindow];
+// deg[v] over the copies
+__device__ __forceinline__ uint32_t degree_sum(const uint32_t* __restrict__ deg, size_t stride, int64_t v) {
+    uint32_t d = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kDegCopies; ++k) d += deg[k * stride + (size_t)v];
+    return d;
+}
+
+// key_at(e): key e, e < m; every thread of the workgroup calls it with its
+// own window h and degree copy.
+constexpr int kDegPer = 4;  // runs of 64 keys a wave loads together
+template <class KeyAt>
+__device__ __forceinline__ void count_degrees(KeyAt&& key_at, int64_t m, int b, uint32_t* h, uint32_t* deg) {
     for (uint32_t i = threadIdx.x; i < kDegWindow; i += kT) h[i] = 0;
     __syncthreads();
-    const int64_t m = m_.get();
     const uint64_t mask = (1ull << b) - 1;
     const uint32_t lane = threadIdx.x & 63;
-    for (int64_t base = blockIdx.x * (int64_t)kT + (threadIdx.x & ~63u); base < m; base += (int64_t)gridDim.x * kT) {
-        const int64_t e = base + lane;
-        const bool ok = e < m;
-        const uint64_t k = ok ? keys[e] : ~0ull;
-        const uint32_t r = (uint32_t)(k >> b);
-        const uint32_t prev = __shfl_up(r, 1), next = __shfl_down(r, 1);
-        const bool first = lane == 0 || prev != r;
-        const bool last = lane == 63 || next != r;
-        const uint64_t starts = __ballot(first);
-        const uint32_t run0 = 63 - __clzll(starts & ((2ull << lane) - 1));  // first lane of my run
-        if (ok && last) {
-            const uint32_t cnt = lane - run0 + 1;
-            if (r < kDegWindow) atomicAdd(&h[r], cnt);
-            else atomicAdd(&deg[r], cnt);
+    for (int64_t base = (blockIdx.x * (int64_t)kT + (threadIdx.x & ~63u)) * kDegPer; base < m;
+         base += (int64_t)gridDim.x * kT * kDegPer) {
+        uint64_t key[kDegPer];
+#pragma unroll
+        for (int x = 0; x < kDegPer; ++x) {
+            const int64_t e = base + x * 64 + lane;
+            key[x] = e < m ? key_at(e) : ~0ull;
         }
-        if (ok) {
-            const uint32_t c = (uint32_t)(k & mask);
-            if (c < kDegWindow) atomicAdd(&h[c], 1u);
-            else atomicAdd(&deg[c], 1u);
+#pragma unroll
+        for (int x = 0; x < kDegPer; ++x) {
+            const bool ok = base + x * 64 + lane < m;
+            const uint32_t r = (uint32_t)(key[x] >> b);
+            const uint32_t prev = __shfl_up(r, 1);
+            const uint64_t starts = __ballot(lane == 0 || prev != r);
+            // a run's first lane adds its length: up to the next run, the
+            // last key or the wave's end
+            const uint64_t ends = (starts | __ballot(!ok)) >> lane >> 1;
+            if (ok) {
+                if (starts >> lane & 1) {
+                    const uint32_t cnt = ends ? (uint32_t)__builtin_ctzll(ends) + 1u : 64u - lane;
+                    if (r < kDegWindow) atomicAdd(&h[r], cnt);
+                    else atomicAdd(&deg[r], cnt);
+                }
+                const uint32_t c = (uint32_t)(key[x] & mask);
+                if (c < kDegWindow) atomicAdd(&h[c], 1u);
+                else atomicAdd(&deg[c], 1u);
+            }
         }
     }
     __syncthreads();
@@ -170,13 +191,19 @@ __global__ __launch_bounds__(kT) void degree_kernel(const uint64_t* __restrict__
         if (h[i]) atomicAdd(&deg[i], h[i]);
 }
 
+__global__ __launch_bounds__(kT) void degree_kernel(const uint64_t* __restrict__ keys, int64_t m, int b,
+                                                    uint32_t* __restrict__ deg, size_t stride_deg) {
+    __shared__ uint32_t h[kDegWindow];
+    count_degrees([&](int64_t e) { return keys[e]; }, m, b, h, deg + (blockIdx.x % kDegCopies) * stride_deg);
+}
+
 // key = top - degree (ascending = descending degree; top is at least the
 // largest degree), value = vertex
-__global__ void rank_keys_kernel(const uint32_t* __restrict__ deg, Cnt n_, uint32_t top, uint32_t* __restrict__ key,
-                                 uint32_t* __restrict__ val) {
+__global__ void rank_keys_kernel(const uint32_t* __restrict__ deg, size_t stride_deg, Cnt n_, uint32_t top,
+                                 uint32_t* __restrict__ key, uint32_t* __restrict__ val) {
     const int64_t n = n_.get();
     for (int64_t v = blockIdx.x * (int64_t)kT + threadIdx.x; v < n; v += (int64_t)gridDim.x * kT) {
-        key[v] = top - deg[v];
+        key[v] = top - degree_sum(deg, stride_deg, v);
         val[v] = (uint32_t)v;
     }
 }
@@ -218,9 +245,10 @@ __global__ void rank_scatter_kernel(const uint32_t* __restrict__ order, Cnt n_, 
 
 // L from the ascending keys: rowptr[r] = first e with keys[e] >= r << b
 // (r = 0..n), col[e] = the key's low b bits, col[m, m + kColPad) = 0; col16
-// (when set) gets the low 16 bits of col over the same m + kColPad entries.
+// (when set) gets the low 16 bits of col over the same m + kColPad entries,
+// erow (when set) every entry's row.
 __global__ void csr_kernel(const uint64_t* __restrict__ keys, Cnt m_, int b, Cnt n_, uint32_t* __restrict__ rowptr,
-                           int32_t* __restrict__ col, uint16_t* __restrict__ col16) {
+                           int32_t* __restrict__ col, uint16_t* __restrict__ col16, uint32_t* __restrict__ erow) {
     const int64_t m = m_.get();
     const int64_t n = n_.get();
     const uint64_t mask = (1ull << b) - 1;
@@ -237,9 +265,11 @@ __global__ void csr_kernel(const uint64_t* __restrict__ keys, Cnt m_, int b, Cnt
         rowptr[r] = (uint32_t)lo;
     }
     for (int64_t e = t0; e < m + (int64_t)kColPad; e += stride) {
-        const int32_t c = e < m ? (int32_t)(keys[e] & mask) : 0;
+        const uint64_t k = e < m ? keys[e] : 0;
+        const int32_t c = (int32_t)(k & mask);
         col[e] = c;
         if (col16) col16[e] = (uint16_t)c;
+        if (erow && e < m) erow[e] = (uint32_t)(k >> b);
     }
 }
 
@@ -278,108 +308,267 @@ __global__ __launch_bounds__(kT) void stats_kernel(const uint32_t* __restrict__ 
 }
 
 // ------------------------------------------------- capturable form kernels
-// Clears a run's words (keeping the ones the host wrote) and opens the id
-// range.
-__global__ void pipe_reset_kernel(PipeCtl* __restrict__ c) {
+// First kernel of a run: clears the run's words (keeping the ones the host
+// wrote), the sorts' and scans' words and the graphs' sums.
+__global__ __launch_bounds__(kT) void pipe_begin_kernel(PipeCtl* __restrict__ c, uint32_t* __restrict__ seq,
+                                                        uint64_t seq_words, unsigned long long* __restrict__ work,
+                                                        unsigned long long* __restrict__ per_graph,
+                                                        uint32_t max_graphs) {
+    const uint64_t t = blockIdx.x * (uint64_t)kT + threadIdx.x, stride = (uint64_t)gridDim.x * kT;
+    for (uint64_t i = t; i < seq_words; i += stride)
+        if (i != kSeqErr) seq[i] = 0;
+    if (per_graph)
+        for (uint64_t g = t; g < max_graphs; g += stride) per_graph[g] = 0;
+    if (blockIdx.x != 0) return;
     constexpr uint32_t kWords = sizeof(PipeCtl) / 4;
     uint32_t* w = reinterpret_cast<uint32_t*>(c);
-    for (uint32_t i = threadIdx.x + kPipeHostWords; i < kWords; i += blockDim.x) w[i] = 0;
+    for (uint32_t i = threadIdx.x + kPipeHostWords; i < kWords; i += kT) w[i] = 0;
     __syncthreads();
     if (threadIdx.x == 0) {
         c->lo = INT_MAX;
         c->hi = -1;
+        work[0] = 0;  // the count's total and cursors
+        work[1] = 0;
     }
 }
 
-// orient_kernel for unchecked input.  Every workgroup resolves n itself (the
-// given count, or the largest id + 1) and workgroup 0 records it with the
-// refusal bits; pairs with an id outside [0, n) become the sentinel too (the
-// run is refused then, but its kernels stay in bounds).
-__global__ void orient_checked_kernel(const int32_t* __restrict__ src, const int32_t* __restrict__ dst,
-                                      PipeCtl* __restrict__ c, int32_t n_cap, int b, uint64_t sentinel,
-                                      uint64_t* __restrict__ keys) {
-    const int64_t nnz = c->nnz;
-    const int32_t lo = nnz ? c->lo : 0, hi = c->hi;
-    int64_t nn = c->n_in > 0 ? (int64_t)c->n_in : (int64_t)hi + 1;
-    uint32_t st = 0;
-    if (lo < 0) st |= kPipeNegativeId;
-    if (hi >= nn) st |= kPipeIdRange;
-    if (nn > n_cap) {
-        st |= kPipeTooManyIds;
-        nn = n_cap;
+// The oriented keys of unchecked pairs (ids that no vertex count admits
+// become the sentinel: the run is refused then, but its kernels stay in
+// bounds), the id range and the sort's digits, in one read of the pairs.
+__global__ __launch_bounds__(kT) void orient_checked_kernel(const int32_t* __restrict__ src,
+                                                            const int32_t* __restrict__ dst, PipeCtl* __restrict__ c,
+                                                            int32_t n_cap, int b, uint64_t sentinel,
+                                                            uint64_t* __restrict__ keys, SortUse u) {
+    __shared__ DigitHist h;
+    __shared__ int32_t s_lo[kT / 64], s_hi[kT / 64];
+    const uint32_t nnz = c->nnz, limit = (uint32_t)(c->n_in > 0 ? min(c->n_in, n_cap) : n_cap);
+    sort_status_clear(u, nnz);
+    int32_t lo = INT_MAX, hi = -1;
+    hist_clear(h, u.passes);
+    auto one = [&](int32_t x, int32_t y) {
+        lo = min(lo, min(x, y));
+        hi = max(hi, max(x, y));
+        const uint32_t a = (uint32_t)x, e = (uint32_t)y;
+        const uint64_t k = (a == e || a >= limit || e >= limit) ? sentinel : ((uint64_t)max(a, e) << b) | min(a, e);
+        hist_add(h, u.passes, k);
+        return k;
+    };
+    const uint32_t quads = nnz / 4;  // the arrays are 256-byte aligned
+    for (uint64_t q = blockIdx.x * (uint64_t)kT + threadIdx.x; q < quads; q += (uint64_t)gridDim.x * kT) {
+        const int4 a = reinterpret_cast<const int4*>(src)[q], e = reinterpret_cast<const int4*>(dst)[q];
+        const ulonglong2 k0 = make_ulonglong2(one(a.x, e.x), one(a.y, e.y));
+        const ulonglong2 k1 = make_ulonglong2(one(a.z, e.z), one(a.w, e.w));
+        reinterpret_cast<ulonglong2*>(keys)[2 * q] = k0;
+        reinterpret_cast<ulonglong2*>(keys)[2 * q + 1] = k1;
     }
+    if (blockIdx.x == 0 && threadIdx.x < (nnz & 3u)) {
+        const uint32_t e = 4 * quads + threadIdx.x;
+        keys[e] = one(src[e], dst[e]);
+    }
+    hist_flush(h, u);
+    for (int o = 32; o > 0; o >>= 1) {
+        lo = min(lo, __shfl_xor(lo, o));
+        hi = max(hi, __shfl_xor(hi, o));
+    }
+    if ((threadIdx.x & 63) == 0) {
+        s_lo[threadIdx.x >> 6] = lo;
+        s_hi[threadIdx.x >> 6] = hi;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < kT / 64; ++w) {
+            lo = min(lo, s_lo[w]);
+            hi = max(hi, s_hi[w]);
+        }
+        if (lo != INT_MAX) {
+            atomicMin(&c->lo, lo);
+            atomicMax(&c->hi, hi);
+        }
+    }
+}
+
+// The first of every run of equal sorted keys (the sentinel apart) to out,
+// in order; m = their number; with used set, used[v] = 1 for their ids.
+// Workgroup 0 also resolves n (the given count, or the largest id + 1) and
+// the refusal bits.
+template <int PER>
+__global__ __launch_bounds__(kT) void unique_kernel(const uint64_t* __restrict__ keys, PipeCtl* __restrict__ c,
+                                                    int32_t n_cap, int b, uint64_t sentinel,
+                                                    uint64_t* __restrict__ out, uint32_t* __restrict__ used,
+                                                    ScanUse u) {
+    __shared__ uint32_t lds[4 * PER + 2];
+    __shared__ uint32_t s_tile;
+    const uint32_t nnz = c->nnz;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
+        const int32_t lo = nnz ? c->lo : 0, hi = c->hi;
+        int64_t nn = c->n_in > 0 ? (int64_t)c->n_in : (int64_t)hi + 1;
+        uint32_t st = 0;
+        if (lo < 0) st |= kPipeNegativeId;
+        if (hi >= nn) st |= kPipeIdRange;
+        if (nn > n_cap) {
+            st |= kPipeTooManyIds;
+            nn = n_cap;
+        }
         c->n = (uint32_t)nn;
         c->status = st;
     }
-    const uint32_t n = (uint32_t)nn;
-    for (int64_t e = blockIdx.x * (int64_t)kT + threadIdx.x; e < nnz; e += (int64_t)gridDim.x * kT) {
-        const uint32_t u = (uint32_t)src[e], v = (uint32_t)dst[e];
-        keys[e] = (u == v || u >= n || v >= n) ? sentinel : ((uint64_t)max(u, v) << b) | (uint64_t)min(u, v);
+    constexpr uint32_t kTile = kT * PER;
+    const uint32_t nt = (uint32_t)(((uint64_t)nnz + kTile - 1) / kTile);
+    const uint64_t mask = (1ull << b) - 1;
+    for (TileLoop l(u.ticket, nt, &s_tile); l.next();) {
+        uint64_t k[PER];
+        uint32_t f[PER], pos[PER];
+#pragma unroll
+        for (int x = 0; x < PER; ++x) {
+            const uint64_t e = (uint64_t)l.t * kTile + x * kT + threadIdx.x;
+            k[x] = e < nnz ? keys[e] : sentinel;
+            f[x] = k[x] != sentinel && (e == 0 || keys[e - 1] != k[x]);
+        }
+        const uint64_t tot = tile_offsets<uint32_t, PER>(f, pos, lds, u, l.t);
+        if (l.t == nt - 1 && threadIdx.x == 0) c->m = (uint32_t)tot;
+#pragma unroll
+        for (int x = 0; x < PER; ++x)
+            if (f[x]) {
+                out[pos[x]] = k[x];
+                if (used) {
+                    used[k[x] >> b] = 1u;
+                    used[k[x] & mask] = 1u;
+                }
+            }
     }
 }
 
-__global__ void fill_u32_kernel(uint32_t* __restrict__ p, Cnt n_, uint32_t v) {
-    const int64_t n = n_.get();
-    for (int64_t i = blockIdx.x * (int64_t)kT + threadIdx.x; i < n; i += (int64_t)gridDim.x * kT) p[i] = v;
-}
-
-// The compacted ids: labels (labels[newid[v]] = v for used v) and the keys
-// rewritten through newid (monotone, so they stay sorted).  With no edge
+// The used ids in order: newid = exclusive scan of used, labels[newid[v]] =
+// v, nc = their number; used is left cleared for the next run.  With no edge
 // nothing is compacted (labels = identity, nc = n), as in
 // canonicalise_device.
-__global__ void pipe_compact_ids_kernel(const uint32_t* __restrict__ used, const uint32_t* __restrict__ newid,
-                                        PipeCtl* __restrict__ c, int32_t* __restrict__ labels,
-                                        uint64_t* __restrict__ keys, int b) {
-    const int64_t n = c->n, m = c->m;
-    const int64_t stride = (int64_t)gridDim.x * kT, t0 = blockIdx.x * (int64_t)kT + threadIdx.x;
-    const bool none = m == 0;
-    for (int64_t v = t0; v < n; v += stride) {
-        if (none) labels[v] = (int32_t)v;
-        else if (used[v]) labels[newid[v]] = (int32_t)v;
-    }
-    if (none && t0 == 0) c->nc = (uint32_t)n;
-    const uint64_t mask = (1ull << b) - 1;
-    for (int64_t e = t0; e < m; e += stride) {
-        const uint64_t k = keys[e];
-        keys[e] = ((uint64_t)newid[k >> b] << b) | (uint64_t)newid[k & mask];
-    }
-}
-
-// First vertex of L of every graph: its first input id through newid
-// (none: no compaction, as when there is no edge).
-__global__ void pipe_csegs_kernel(const uint32_t* __restrict__ segs, const uint32_t* __restrict__ newid,
-                                  const PipeCtl* __restrict__ c, uint32_t* __restrict__ csegs) {
-    const uint32_t k = c->graphs;
-    const bool map = newid && c->m != 0;
-    for (uint32_t g = threadIdx.x; g <= k; g += blockDim.x) csegs[g] = map ? newid[segs[g]] : segs[g];
-}
-
-// rank_keys_kernel within graphs: key = graph << b | (top - degree), so one
-// sort orders by (graph, descending degree, id).
-__global__ void pipe_rank_keys_kernel(const uint32_t* __restrict__ deg, const PipeCtl* __restrict__ c,
-                                      const uint32_t* __restrict__ csegs, uint32_t top, int b,
-                                      uint32_t* __restrict__ key, uint32_t* __restrict__ val) {
-    const int64_t n = c->nc;
-    const uint32_t k = c->graphs;
-    for (int64_t v = blockIdx.x * (int64_t)kT + threadIdx.x; v < n; v += (int64_t)gridDim.x * kT) {
-        uint32_t lo = 0, hi = k;  // the last graph whose first vertex is <= v
-        while (hi - lo > 1) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (csegs[mid] <= (uint32_t)v) lo = mid;
-            else hi = mid;
+template <int PER>
+__global__ __launch_bounds__(kT) void newid_kernel(uint32_t* __restrict__ used, PipeCtl* __restrict__ c,
+                                                   uint32_t* __restrict__ newid, int32_t* __restrict__ labels,
+                                                   ScanUse u) {
+    __shared__ uint32_t lds[4 * PER + 2];
+    __shared__ uint32_t s_tile;
+    const uint32_t n = c->n;
+    const bool none = c->m == 0;
+    constexpr uint32_t kTile = kT * PER;
+    const uint32_t nt = (uint32_t)(((uint64_t)n + kTile - 1) / kTile);
+    for (TileLoop l(u.ticket, nt, &s_tile); l.next();) {
+        uint32_t f[PER], pos[PER];
+#pragma unroll
+        for (int x = 0; x < PER; ++x) {
+            const uint64_t v = (uint64_t)l.t * kTile + x * kT + threadIdx.x;
+            f[x] = 0;
+            if (v < n) {
+                f[x] = used[v];
+                if (f[x]) used[v] = 0;
+            }
         }
-        key[v] = (lo << b) | (top - deg[v]);
-        val[v] = (uint32_t)v;
+        const uint64_t tot = tile_offsets<uint32_t, PER>(f, pos, lds, u, l.t);
+        if (l.t == nt - 1 && threadIdx.x == 0) {
+            newid[n] = (uint32_t)tot;
+            c->nc = none ? n : (uint32_t)tot;
+        }
+#pragma unroll
+        for (int x = 0; x < PER; ++x) {
+            const uint64_t v = (uint64_t)l.t * kTile + x * kT + threadIdx.x;
+            if (v < n) newid[v] = pos[x];
+            if (f[x]) labels[pos[x]] = (int32_t)v;
+            else if (none && v < n) labels[v] = (int32_t)v;
+        }
     }
 }
 
-// No compaction: labels = identity and nc = n.
-__global__ void pipe_identity_kernel(PipeCtl* __restrict__ c, int32_t* __restrict__ labels) {
-    const int64_t n = c->n;
-    const int64_t t0 = blockIdx.x * (int64_t)kT + threadIdx.x;
-    for (int64_t v = t0; v < n; v += (int64_t)gridDim.x * kT) labels[v] = (int32_t)v;
-    if (t0 == 0) c->nc = (uint32_t)n;
+// Between the ids' compaction and the relabel: keys rewritten through newid
+// (monotone, so they stay sorted; NULL: no compaction, labels = identity and
+// nc = n), the graphs' first vertices of L (csegs), and with deg set the
+// degrees, as degree_kernel.
+__global__ __launch_bounds__(kT) void pipe_rekey_kernel(uint64_t* __restrict__ keys, PipeCtl* __restrict__ c, int b,
+                                                        const uint32_t* __restrict__ newid,
+                                                        int32_t* __restrict__ labels,
+                                                        const uint32_t* __restrict__ segs,
+                                                        uint32_t* __restrict__ csegs, uint32_t* __restrict__ deg,
+                                                        size_t stride_deg) {
+    __shared__ uint32_t h[kDegWindow];
+    const int64_t m = c->m, n = c->n;
+    if (csegs && blockIdx.x == 0)
+        for (uint32_t g = threadIdx.x; g <= c->graphs; g += kT) csegs[g] = newid && m ? newid[segs[g]] : segs[g];
+    if (!newid) {
+        const int64_t t0 = blockIdx.x * (int64_t)kT + threadIdx.x;
+        for (int64_t v = t0; v < n; v += (int64_t)gridDim.x * kT) labels[v] = (int32_t)v;
+        if (t0 == 0) c->nc = (uint32_t)n;
+    }
+    const uint64_t mask = (1ull << b) - 1;
+    auto rekey = [&](int64_t e) -> uint64_t {
+        const uint64_t k = keys[e];
+        if (!newid) return k;
+        const uint64_t x = ((uint64_t)newid[k >> b] << b) | (uint64_t)newid[k & mask];
+        keys[e] = x;
+        return x;
+    };
+    if (!deg) {
+        if (newid)
+            for (int64_t e = blockIdx.x * (int64_t)kT + threadIdx.x; e < m; e += (int64_t)gridDim.x * kT) rekey(e);
+        return;
+    }
+    if (blockIdx.x * (int64_t)kT * kDegPer >= m) return;  // workgroup-uniform: no keys of its own
+    count_degrees(rekey, m, b, h, deg + (blockIdx.x % kDegCopies) * stride_deg);
+}
+
+// rank_keys_kernel within graphs (csegs set): key = graph << b | (top -
+// degree), so one sort orders by (graph, descending degree, id).  The degree
+// copies are left cleared for the next run; the sort's digits are taken.
+__global__ __launch_bounds__(kT) void pipe_rank_keys_kernel(uint32_t* __restrict__ deg, size_t stride_deg,
+                                                            const PipeCtl* __restrict__ c,
+                                                            const uint32_t* __restrict__ csegs, uint32_t top, int b,
+                                                            uint32_t* __restrict__ key, uint32_t* __restrict__ val,
+                                                            SortUse u) {
+    __shared__ DigitHist h;
+    const int64_t n = c->nc;
+    sort_status_clear(u, (uint64_t)n);
+    hist_clear(h, u.passes);
+    for (int64_t v = blockIdx.x * (int64_t)kT + threadIdx.x; v < n; v += (int64_t)gridDim.x * kT) {
+        uint32_t lo = 0;
+        if (csegs) {
+            uint32_t hi = c->graphs;  // the last graph whose first vertex is <= v
+            while (hi - lo > 1) {
+                const uint32_t mid = (lo + hi) >> 1;
+                if (csegs[mid] <= (uint32_t)v) lo = mid;
+                else hi = mid;
+            }
+        }
+        uint32_t part[kDegCopies], d = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < kDegCopies; ++k) part[k] = deg[k * stride_deg + (size_t)v];
+#pragma unroll
+        for (uint32_t k = 0; k < kDegCopies; ++k) {
+            d += part[k];
+            if (part[k]) deg[k * stride_deg + (size_t)v] = 0;
+        }
+        const uint32_t x = (csegs ? lo << b : 0u) | (top - d);
+        key[v] = x;
+        val[v] = (uint32_t)v;
+        hist_add(h, u.passes, x);
+    }
+    hist_flush(h, u);
+}
+
+// relabel_kernel through rank, with the next sort's digits.
+__global__ __launch_bounds__(kT) void pipe_relabel_kernel(uint64_t* __restrict__ keys, const PipeCtl* __restrict__ c,
+                                                          int b, const uint32_t* __restrict__ rank, SortUse u) {
+    __shared__ DigitHist h;
+    const int64_t m = c->m;
+    sort_status_clear(u, (uint64_t)m);
+    if (blockIdx.x * (int64_t)kT >= m) return;  // workgroup-uniform
+    const uint64_t mask = (1ull << b) - 1;
+    hist_clear(h, u.passes);
+    for (int64_t e = blockIdx.x * (int64_t)kT + threadIdx.x; e < m; e += (int64_t)gridDim.x * kT) {
+        const uint64_t k = keys[e];
+        const uint32_t r = rank[k >> b], q = rank[k & mask];
+        const uint64_t x = ((uint64_t)max(r, q) << b) | (uint64_t)min(r, q);
+        keys[e] = x;
+        hist_add(h, u.passes, x);
+    }
+    hist_flush(h, u);
 }
 
 #define BTC_LAUNCH(kernel, n, s, ...)                                                   \
@@ -496,19 +685,20 @@ void canonicalise_device(const int32_t* src, const int32_t* dst, int64_t nnz, in
     if (flags & BTC_CANON_DEGREE_ORDER) {
         TmpBuf<uint32_t> deg, k0, v0, k1, v1, rank;
         DevBuf<int32_t> lab2;
-        deg.alloc((size_t)nc, s);
+        deg.alloc((size_t)nc * kDegCopies, s);
         k0.alloc((size_t)nc, s);
         v0.alloc((size_t)nc, s);
         k1.alloc((size_t)nc, s);
         v1.alloc((size_t)nc, s);
         rank.alloc((size_t)nc, s);
         lab2.alloc_on((size_t)nc, s);
-        BTC_HIP(hipMemsetAsync(deg.p, 0, (size_t)nc * 4, s));
+        BTC_HIP(hipMemsetAsync(deg.p, 0, (size_t)nc * kDegCopies * 4, s));
         if (m) {
-            hipLaunchKernelGGL(degree_kernel, dim3(std::min(grid_for(m), kRedBlocks)), dim3(kT), 0, s, keys, m, bn, deg.p);
+            hipLaunchKernelGGL(degree_kernel, dim3(std::min(grid_for(m), kRedBlocks)), dim3(kT), 0, s, keys, m, bn, deg.p,
+                               (size_t)nc);
             BTC_CHECK_LAUNCH("degree_kernel");
         }
-        BTC_LAUNCH(rank_keys_kernel, nc, s, deg.p, nc, 0xFFFFFFFFu, k0.p, v0.p);
+        BTC_LAUNCH(rank_keys_kernel, nc, s, deg.p, (size_t)nc, nc, 0xFFFFFFFFu, k0.p, v0.p);
         bool alt = sort_pairs_u32(k0.p, v0.p, k1.p, v1.p, (size_t)nc, 32, s);
         if (segs) {
             // then a stable sort by segment: (segment, -degree, id)
@@ -535,7 +725,7 @@ void canonicalise_device(const int32_t* src, const int32_t* dst, int64_t nnz, in
     g->d_rowptr.alloc_on((size_t)nc + 1, s);
     g->d_col.alloc_on((size_t)m + kColPad, s);
     BTC_LAUNCH(csr_kernel, std::max<int64_t>((int64_t)nc + 1, m + (int64_t)kColPad), s, keys, m, bn, nc,
-               g->d_rowptr.p, g->d_col.p, (uint16_t*)nullptr);
+               g->d_rowptr.p, g->d_col.p, (uint16_t*)nullptr, (uint32_t*)nullptr);
     g->d_labels = std::move(labels);
 
     // derived statistics (graph_finalize on the device)
@@ -568,10 +758,11 @@ unsigned cap_grid(int64_t cap) {
         BTC_CHECK_LAUNCH(#kernel);                                                     \
     } while (0)
 
+// Kernels that end in atomics on a few addresses (reductions, digit totals).
 #define CAP_LAUNCH_RED(kernel, cap, s, ...)                                                \
-    do {                                                                               \
-        hipLaunchKernelGGL(kernel, dim3(std::min(cap_grid(cap), kCapRedBlocks)), dim3(kT), 0, s, __VA_ARGS__);  \
-        BTC_CHECK_LAUNCH(#kernel);                                                     \
+    do {                                                                                   \
+        hipLaunchKernelGGL(kernel, dim3(std::min(cap_grid(cap), 2 * kCapRedBlocks)), dim3(kT), 0, s, __VA_ARGS__);  \
+        BTC_CHECK_LAUNCH(#kernel);                                                         \
     } while (0)
 
 int32_t* canonicalise_capacity(const CanonCap& c, hipStream_t s) {
@@ -579,64 +770,66 @@ int32_t* canonicalise_capacity(const CanonCap& c, hipStream_t s) {
     const int64_t E = c.nnz_cap, N = c.n_cap;
     const int b = id_bits(N);
     const uint64_t sentinel = (1ull << (2 * b)) - 1;
-    const Cnt nnz = Cnt::dev(&ctl->nnz), n = Cnt::dev(&ctl->n), m = Cnt::dev(&ctl->m), nc = Cnt::dev(&ctl->nc);
-    hipLaunchKernelGGL(pipe_reset_kernel, dim3(1), dim3(64), 0, s, ctl);
-    BTC_CHECK_LAUNCH("pipe_reset_kernel");
-    CAP_LAUNCH_RED(id_range_kernel, E, s, c.src, c.dst, nnz, &ctl->lo);
+    const Cnt m = Cnt::dev(&ctl->m), nc = Cnt::dev(&ctl->nc);
+    const bool compact = (c.flags & BTC_CANON_COMPACT) != 0, groups = c.max_graphs > 1;
+    const uint64_t seq_words = dseq_clear_words(c.seq->cap);
+    hipLaunchKernelGGL(pipe_begin_kernel, dim3(std::min(cap_grid((int64_t)seq_words), kCapRedBlocks)), dim3(kT), 0, s,
+                       ctl, static_cast<uint32_t*>(c.seq->p), seq_words, c.work, groups ? c.per_graph : nullptr,
+                       (uint32_t)c.max_graphs);
+    BTC_CHECK_LAUNCH("pipe_begin_kernel");
 
     // oriented keys, sorted, deduplicated
-    CAP_LAUNCH(orient_checked_kernel, E, s, c.src, c.dst, ctl, c.n_cap, b, sentinel, c.ka);
-    uint64_t* sorted = dsort_u64(c.ka, c.kb, (size_t)E, &ctl->nnz, 2 * b, c.ws, s);
+    const SortUse su = dseq_sort(*c.seq, 2 * b);
+    CAP_LAUNCH_RED(orient_checked_kernel, E / 4 + 1, s, c.src, c.dst, ctl, c.n_cap, b, sentinel, c.ka, su);
+    uint64_t* sorted = dsort_u64(c.ka, c.kb, (size_t)E, &ctl->nnz, su, s);
     uint64_t* keys = sorted == c.ka ? c.kb : c.ka;
     uint64_t* spare = sorted;
-    CAP_LAUNCH(first_flag_kernel, E, s, sorted, nnz, sentinel, c.flag);
-    dscan_u32(c.flag, c.pos, (size_t)E, &ctl->nnz, &ctl->m, c.ws, s);
-    CAP_LAUNCH(compact_kernel, E, s, sorted, c.flag, c.pos, nnz, keys);
+    with_tile_per(E, [&](auto per) {
+        constexpr int PER = decltype(per)::value;
+        CAP_LAUNCH(unique_kernel<PER>, E / PER + 1, s, sorted, ctl, c.n_cap, b, sentinel, keys,
+                   compact ? c.used : nullptr, dseq_scan(*c.seq));
+    });
 
     // order-preserving compaction of the used ids (ids keep b bits); the
-    // graphs' ranges follow it
-    const bool groups = c.max_graphs > 1;
+    // graphs' ranges follow it; degrees
     int32_t* labels = c.lab0;
-    if (c.flags & BTC_CANON_COMPACT) {
-        CAP_LAUNCH(fill_u32_kernel, N, s, c.used, n, 0u);
-        CAP_LAUNCH(mark_used_kernel, E, s, keys, m, b, c.used);
-        dscan_u32(c.used, c.newid, (size_t)N, &ctl->n, &ctl->nc, c.ws, s);
-        CAP_LAUNCH(pipe_compact_ids_kernel, std::max(N, E), s, c.used, c.newid, ctl, labels, keys, b);
-    } else {
-        CAP_LAUNCH(pipe_identity_kernel, N, s, ctl, labels);
-    }
-    if (groups) {
-        hipLaunchKernelGGL(pipe_csegs_kernel, dim3(1), dim3(64), 0, s, c.segs,
-                           (c.flags & BTC_CANON_COMPACT) ? c.newid : nullptr, ctl, c.csegs);
-        BTC_CHECK_LAUNCH("pipe_csegs_kernel");
-    }
+    if (compact)
+        with_tile_per(N, [&](auto per) {
+            constexpr int PER = decltype(per)::value;
+            CAP_LAUNCH(newid_kernel<PER>, N / PER + 1, s, c.used, ctl, c.newid, labels, dseq_scan(*c.seq));
+        });
+    const bool by_degree = (c.flags & BTC_CANON_DEGREE_ORDER) != 0;
+    hipLaunchKernelGGL(pipe_rekey_kernel, dim3(std::min(cap_grid(std::max(N, E)), 4 * kCapRedBlocks)), dim3(kT), 0, s,
+                       keys, ctl, b, compact ? c.newid : nullptr, labels, c.segs, groups ? c.csegs : nullptr,
+                       by_degree ? c.deg : nullptr, (size_t)N);
+    BTC_CHECK_LAUNCH("pipe_rekey_kernel");
 
-    if (c.flags & BTC_CANON_DEGREE_ORDER) {
+    if (by_degree) {
         // keys N - 1 - degree < 2^b: descending degree, ties by id
-        CAP_LAUNCH(fill_u32_kernel, N, s, c.deg, nc, 0u);
-        hipLaunchKernelGGL(degree_kernel, dim3(std::min(cap_grid(E), kCapRedBlocks)), dim3(kT), 0, s, keys, m, b, c.deg);
-        BTC_CHECK_LAUNCH("degree_kernel");
         int kb = b;  // key bits: degree rank, then (several graphs) the graph
         if (groups) {
             int gb = 1;
             while ((1 << gb) < c.max_graphs) ++gb;
             BTC_REQUIRE(b + gb <= 32, BTC_ERR_OVERFLOW, "%d ids and %d graphs exceed 32-bit relabel keys", c.n_cap,
                         c.max_graphs);
-            CAP_LAUNCH(pipe_rank_keys_kernel, N, s, c.deg, ctl, c.csegs, (uint32_t)(N - 1), b, c.k0, c.v0);
             kb = b + gb;
-        } else {
-            CAP_LAUNCH(rank_keys_kernel, N, s, c.deg, nc, (uint32_t)(N - 1), c.k0, c.v0);
         }
-        const bool alt = dsort_pairs_u32(c.k0, c.v0, c.k1, c.v1, (size_t)N, &ctl->nc, kb, c.ws, s);
+        const SortUse ru = dseq_sort(*c.seq, kb);
+        CAP_LAUNCH_RED(pipe_rank_keys_kernel, N, s, c.deg, (size_t)N, ctl, groups ? c.csegs : nullptr,
+                       (uint32_t)(N - 1), b, c.k0, c.v0, ru);
+        const bool alt = dsort_pairs_u32(c.k0, c.v0, c.k1, c.v1, (size_t)N, &ctl->nc, ru, s);
         CAP_LAUNCH(rank_scatter_kernel, N, s, alt ? c.v1 : c.v0, nc, c.rank, labels, c.lab1);
-        CAP_LAUNCH(relabel_kernel, E, s, keys, m, b, c.rank, b);
-        keys = dsort_u64(keys, spare, (size_t)E, &ctl->m, 2 * b, c.ws, s);
+        const SortUse ku = dseq_sort(*c.seq, 2 * b);
+        CAP_LAUNCH_RED(pipe_relabel_kernel, E, s, keys, ctl, b, c.rank, ku);
+        keys = dsort_u64(keys, spare, (size_t)E, &ctl->m, ku, s);
         labels = c.lab1;
     }
 
-    // CSR of L (with its 16-bit copy) and its statistics
-    CAP_LAUNCH(csr_kernel, std::max(N + 1, E + (int64_t)kColPad), s, keys, m, b, nc, c.rowptr, c.col, c.col16);
-    CAP_LAUNCH_RED(stats_kernel, std::max(N, E), s, c.rowptr, c.col, nc, m, ctl->rs);
+    // CSR of L (with its 16-bit copy and every entry's row) and its statistics
+    CAP_LAUNCH(csr_kernel, std::max(N + 1, E + (int64_t)kColPad), s, keys, m, b, nc, c.rowptr, c.col, c.col16, c.erow);
+    hipLaunchKernelGGL(stats_kernel, dim3(std::min(cap_grid(std::max(N, E)), kCapRedBlocks)), dim3(kT), 0, s, c.rowptr,
+                       c.col, nc, m, ctl->rs);
+    BTC_CHECK_LAUNCH("stats_kernel");
     return labels;
 }
 

@@ -222,10 +222,15 @@ struct PipeCtl {
     unsigned long long st[8];  // planner statistics (as plan_device's)
     unsigned long long chunk;  // wedge checks per work item
     unsigned long long checks; // wedge checks in all
+    unsigned long long total;  // triangles of the run
+    unsigned long long err;    // the sorts' and scans' error word
 };
 constexpr uint32_t kPipeNegativeId = 1, kPipeIdRange = 2, kPipeTooManyIds = 4;
 constexpr uint32_t kPipeHostWords = 4;  // words of PipeCtl the host writes before a run
 static_assert(sizeof(PipeCtl) % 8 == 0, "u64 fields aligned");
+
+// Copies of the degree counters (canon_gpu.hip).
+constexpr uint32_t kDegCopies = 8;
 
 // Buffers of a capturable canonicalisation of up to nnz_cap pairs over up
 // to n_cap ids (element counts in brackets).
@@ -238,11 +243,9 @@ struct CanonCap {
     PipeCtl* ctl;
     uint64_t* ka;
     uint64_t* kb;        // [nnz_cap] each
-    uint32_t* flag;      // [nnz_cap]
-    uint32_t* pos;       // [nnz_cap + 1]
-    uint32_t* used;      // [n_cap]
+    uint32_t* used;      // [n_cap], zeroed once: every run leaves it cleared
     uint32_t* newid;     // [n_cap + 1]
-    uint32_t* deg;
+    uint32_t* deg;       // [kDegCopies * n_cap], zeroed once likewise
     uint32_t* k0;
     uint32_t* v0;
     uint32_t* k1;
@@ -253,13 +256,16 @@ struct CanonCap {
     uint32_t* rowptr;    // [n_cap + 1]
     int32_t* col;        // [nnz_cap + kColPad]
     uint16_t* col16;     // [nnz_cap + kColPad]: low 16 bits of col
-    DevWs ws;            // dsort / dscan workspace for max(nnz_cap, n_cap)
+    DevSeq* seq;         // the run's sorts and scans (workspace for max(nnz_cap, n_cap))
+    unsigned long long* work;  // the count's words (kWorkWords): total and cursors cleared by the first kernel
+    uint32_t* erow;      // [nnz_cap]: row of every entry of L, for the planner
     // several graphs (max_graphs > 1): graph g's ids are segs[g] ..
     // segs[g + 1] - 1 of the input (host-written), csegs[g] its first vertex
     // of L; the degree relabel keeps every graph a contiguous range
     int32_t max_graphs = 1;
     const uint32_t* segs = nullptr;  // [max_graphs + 1]
     uint32_t* csegs = nullptr;       // [max_graphs + 1]
+    unsigned long long* per_graph = nullptr;  // [max_graphs]: cleared by the first kernel
 };
 
 // Enqueues the canonicalisation of ctl->nnz pairs (the same CSR as
@@ -277,34 +283,27 @@ struct PlanCap {
     uint32_t core_ids;       // C (0 = no hub-core bitmaps)
     int cus;                 // compute units (items of about 64 per CU)
     PipeCtl* ctl;
-    uint32_t* erow;
-    uint32_t* lflag;         // [m_cap] each
-    uint32_t* lpos;          // [m_cap + 1]
+    const uint32_t* erow;    // [m_cap]: row of every entry
+    uint32_t* cend;          // [n_cap]: end of the row's ids below C
+    uint32_t* rbi;           // [n_cap]: the row's core bitmap or kNoBitmap
     uint32_t* k0;
     uint32_t* v0;
     uint32_t* k1;
     uint32_t* v1;            // [m_cap] each
-    uint32_t* off;           // [n_cap + 1]
-    uint32_t* cend;
-    uint32_t* has;           // [n_cap] each
-    uint32_t* rbi;           // [n_cap + 1]
+    uint4* rec;              // [m_cap]: list records in entry order
+    uint32_t* off;
+    uint32_t* oend;          // [n_cap] each: lists of every pivot that has any
     uint4* lists;            // [m_cap]
     uint32_t* rowbits;       // [nbm_cap * C / 32]
     int32_t* ur;             // [m_cap]
-    uint64_t* cost;          // [m_cap]
     uint64_t* P;             // [m_cap + 1]
-    uint32_t* start;         // [m_cap]
-    uint32_t* spos;          // [m_cap + 1]
     size_t items_cap;        // m_cap (every work item opens at a distinct list)
     uint32_t* first;         // [items_cap]
-    uint4* tmp_items;        // [2 * items_cap]
-    uint32_t* sk0;
-    uint32_t* sv0;
-    uint32_t* sk1;
-    uint32_t* sv1;           // [items_cap] each
+    uint32_t* skey;          // [items_cap]
     uint4* items;            // [2 * items_cap]
-    unsigned long long* work;  // the count's words (kWorkWords): total and cursors cleared with the items
-    DevWs ws;                // dsort / dscan workspace for max(m_cap, items_cap)
+    DevSeq* seq;             // the run's sorts and scans (workspace for max(m_cap, n_cap))
+    // several graphs: their vertex ranges in L, whose index every item gets
+    const uint32_t* csegs = nullptr;
 };
 
 // Rows that can hold a hub-core bitmap: at least kCoreRowMin entries each.
@@ -324,21 +323,22 @@ void pipeline_count_checked(btc_pipeline_s* p, int32_t count, const int32_t* con
                             const int64_t* sizes, const int64_t* nv, hipStream_t s, uint64_t* per_graph,
                             uint64_t* total);
 
+// Enqueues the count of a plan_capacity plan: the wedge kernel on the item
+// counts in ctl, then the slot sum into work[0] and ctl->total (work: the
+// count's kWorkWords words, total and cursors cleared by the run's first
+// kernel, the slots left cleared by every count).  col16 is L's 16-bit copy.
+// With pv set (several graphs), per_graph[g] (cleared by the run's first
+// kernel) gets graph g's count: the wedge kernel adds each item's count at
+// the graph its record holds; with 64-bit offsets the per-vertex sums go to
+// pv (cleared over ctl->nc vertices) and are summed per graph over its
+// vertices [csegs[g], csegs[g + 1]) instead.
+void pipeline_count_enqueue(const PlanCap& c, const uint16_t* col16, const btc_count_opts& o, hipStream_t s,
+                            unsigned long long* work, unsigned long long* pv = nullptr,
+                            const uint32_t* csegs = nullptr, unsigned long long* per_graph = nullptr,
+                            int max_graphs = 1);
+
 // Checks the launch-shape fields of o (BTC_ERR_ARG on a bad value).
 void check_launch_opts(const btc_count_opts& o);
-
-// Enqueues the count of a plan_capacity plan (whose last kernel cleared the
-// total and cursors at c.work; the slots are left cleared by every count):
-// the wedge kernel on the item counts in ctl, then the slot sum into
-// c.work[0].  col16 is L's 16-bit copy.  With pv set (several graphs),
-// per_graph[g] (g < max_graphs, cleared first) gets graph g's count: each
-// work item records its graph (the graph whose vertices [csegs[g],
-// csegs[g + 1]) hold its pivot) and the wedge kernel adds the item's count
-// there; with 64-bit offsets the per-vertex sums go to pv (cleared over
-// ctl->nc vertices) and are summed per graph instead.
-void pipeline_count_enqueue(const PlanCap& c, const uint16_t* col16, const btc_count_opts& o, hipStream_t s,
-                            unsigned long long* pv = nullptr, const uint32_t* csegs = nullptr,
-                            unsigned long long* per_graph = nullptr, int max_graphs = 1);
 
 // Uploads L (rowptr narrowed to u32) to HBM on first use.
 void ensure_device(btc_graph_s* g, hipStream_t s);

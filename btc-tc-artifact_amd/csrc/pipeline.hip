@@ -43,7 +43,7 @@ struct btc_pipeline_s {
     int32_t graph_nodes = 0;
     btcx::PinnedBuf pin;  // [0, 4 KiB): control block and total; then staged pairs
     btcx::PipeCtl last{};
-    size_t ws_bytes = 0;  // the sorts' and scans' workspace (zeroed at creation)
+    btcx::DevSeq seq;     // the captured run's sorts and scans
     // a run's end is awaited on this event, which blocks the host thread
     // instead of spinning (threads that run pipelines side by side leave
     // their cores to each other meanwhile)
@@ -58,12 +58,12 @@ struct btc_pipeline_s {
 namespace btcx {
 namespace {
 
-// Pinned staging: control block, total and error word from 0, the graphs'
+// Pinned staging: control block from 0, the graphs'
 // ranges at kPinSegs, per-graph sums at kPinPerGraph, pairs from kPinHeader.
 constexpr size_t kPinHeader = 4096;
 constexpr size_t kPinSegs = 1024, kPinPerGraph = 2048;
 constexpr int kMaxPipelineGraphs = 64;
-static_assert(sizeof(PipeCtl) + 16 <= kPinSegs && kPinSegs + 4 * (kMaxPipelineGraphs + 1) <= kPinPerGraph &&
+static_assert(sizeof(PipeCtl) <= kPinSegs && kPinSegs + 4 * (kMaxPipelineGraphs + 1) <= kPinPerGraph &&
                   kPinPerGraph + 8 * kMaxPipelineGraphs <= kPinHeader,
               "pinned header layout");
 
@@ -101,11 +101,9 @@ void layout(btc_pipeline_s* p, Carve& c) {
     k.ctl = p->ctl;
     k.ka = c.take<uint64_t>(E);
     k.kb = c.take<uint64_t>(E);
-    k.flag = c.take<uint32_t>(E);
-    k.pos = c.take<uint32_t>(E + 1);
     k.used = c.take<uint32_t>(N);
     k.newid = c.take<uint32_t>(N + 1);
-    k.deg = c.take<uint32_t>(N);
+    k.deg = c.take<uint32_t>(kDegCopies * N);
     k.k0 = c.take<uint32_t>(N);
     k.v0 = c.take<uint32_t>(N);
     k.k1 = c.take<uint32_t>(N);
@@ -125,40 +123,32 @@ void layout(btc_pipeline_s* p, Carve& c) {
     q.core_ids = C;
     q.cus = device_cu_count();
     q.ctl = p->ctl;
-    // the canonicalisation's keys and flags are dead once L is written:
-    // the planner's list keys and flags reuse them
+    // the canonicalisation's keys are dead once L is written: the planner's
+    // list keys reuse them
     q.k0 = reinterpret_cast<uint32_t*>(k.ka);
     q.v0 = q.k0 ? q.k0 + M : nullptr;
     q.k1 = reinterpret_cast<uint32_t*>(k.kb);
     q.v1 = q.k1 ? q.k1 + M : nullptr;
-    q.lflag = k.flag;
-    q.lpos = k.pos;
-    q.erow = c.take<uint32_t>(M);
-    q.off = c.take<uint32_t>(N + 1);
+    k.erow = c.take<uint32_t>(M);
+    q.erow = k.erow;
     q.cend = c.take<uint32_t>(N);
-    q.has = c.take<uint32_t>(N);
-    q.rbi = c.take<uint32_t>(N + 1);
+    q.rbi = c.take<uint32_t>(N);
+    q.off = c.take<uint32_t>(N);
+    q.oend = c.take<uint32_t>(N);
+    q.rec = c.take<uint4>(M);
     q.lists = c.take<uint4>(M);
     q.rowbits = c.take<uint32_t>(C ? pipe_bitmap_rows((int64_t)M, p->n_cap) * (C / 32) : 1);
     q.ur = c.take<int32_t>(M);
-    q.cost = c.take<uint64_t>(M);
     q.P = c.take<uint64_t>(M + 1);
-    q.start = c.take<uint32_t>(M);
-    q.spos = c.take<uint32_t>(M + 1);
     q.items_cap = M;
     q.first = c.take<uint32_t>(M);
-    q.tmp_items = c.take<uint4>(2 * M);
-    q.sk0 = c.take<uint32_t>(M);
-    q.sv0 = c.take<uint32_t>(M);
-    q.sk1 = c.take<uint32_t>(M);
-    q.sv1 = c.take<uint32_t>(M);
+    q.skey = c.take<uint32_t>(M);
     q.items = c.take<uint4>(2 * M);
-    q.work = p->work;
-    const size_t big = std::max(E, N);
-    p->ws_bytes = dprim_ws_bytes(big);
-    const DevWs ws{c.take<unsigned char>(p->ws_bytes), big};
-    k.ws = ws;
-    q.ws = ws;
+    k.work = p->work;
+    p->seq = DevSeq{};
+    p->seq.cap = std::max(E, N);
+    p->seq.p = c.take<unsigned char>(dseq_bytes(p->seq.cap));
+    k.seq = q.seq = &p->seq;
     if (p->max_graphs > 1) {
         const size_t G = (size_t)p->max_graphs;
         p->segs = c.take<uint32_t>(G + 1);
@@ -168,6 +158,8 @@ void layout(btc_pipeline_s* p, Carve& c) {
         k.max_graphs = p->max_graphs;
         k.segs = p->segs;
         k.csegs = p->csegs;
+        k.per_graph = p->per_graph;
+        q.csegs = p->csegs;
     }
 }
 
@@ -179,15 +171,17 @@ void pipeline_build(btc_pipeline_s* p, hipStream_t s) {
     Carve real;
     real.base = p->mem.p;
     layout(p, real);
-    // the count's words and the sorts' and scans' workspace start cleared;
-    // every replay leaves them cleared again
+    // the count's words, the id marks and the degree copies start cleared and
+    // every replay leaves them cleared again; the error word starts cleared
     BTC_HIP(hipMemsetAsync(p->work, 0, kWorkWords * 8, s));
-    BTC_HIP(hipMemsetAsync(p->canon.ws.p, 0, p->ws_bytes, s));
+    BTC_HIP(hipMemsetAsync(p->canon.used, 0, (size_t)p->n_cap * 4, s));
+    BTC_HIP(hipMemsetAsync(p->canon.deg, 0, (size_t)p->n_cap * 4 * kDegCopies, s));
+    BTC_HIP(hipMemsetAsync(p->seq.p, 0, dseq_clear_words(p->seq.cap) * 4, s));
     BTC_HIP(hipStreamSynchronize(s));
     p->graph.capture([&](hipStream_t cs) {
         p->labels = canonicalise_capacity(p->canon, cs);
         plan_capacity(p->plan, cs);
-        pipeline_count_enqueue(p->plan, p->col16, p->opts, cs, p->pv, p->csegs, p->per_graph, p->max_graphs);
+        pipeline_count_enqueue(p->plan, p->col16, p->opts, cs, p->work, p->pv, p->csegs, p->per_graph, p->max_graphs);
     });
     BTC_HIP(hipEventCreateWithFlags(&p->done, hipEventBlockingSync | hipEventDisableTiming));
     size_t nodes = 0;
@@ -213,27 +207,23 @@ void replay(btc_pipeline_s* p, char* pin, uint32_t nnz, int32_t n_in, uint32_t g
     tm.start(s);
     p->graph.launch(s);
     tm.stop(s);
-    unsigned long long* htotal = reinterpret_cast<unsigned long long*>(pin + sizeof(PipeCtl));
-    uint32_t* herr = reinterpret_cast<uint32_t*>(htotal + 1);
     unsigned long long* hpg = reinterpret_cast<unsigned long long*>(pin + kPinPerGraph);
     BTC_HIP(hipMemcpyAsync(h, p->ctl, sizeof(PipeCtl), hipMemcpyDeviceToHost, s));
-    BTC_HIP(hipMemcpyAsync(htotal, p->work, 8, hipMemcpyDeviceToHost, s));
-    BTC_HIP(hipMemcpyAsync(herr, dsort_error_word(p->canon.ws), 4, hipMemcpyDeviceToHost, s));
     if (p->max_graphs > 1)
         BTC_HIP(hipMemcpyAsync(hpg, p->per_graph, (size_t)graphs * 8, hipMemcpyDeviceToHost, s));
     BTC_HIP(hipEventRecord(p->done, s));
     BTC_HIP(hipEventSynchronize(p->done));
-    BTC_REQUIRE(*herr == 0, BTC_ERR_HIP, "a device sort of the pipeline failed (look-back spin limit)");
     const PipeCtl c = *h;
+    BTC_REQUIRE(c.err == 0, BTC_ERR_HIP, "a device sort of the pipeline failed (look-back spin limit)");
     BTC_REQUIRE(!(c.status & kPipeNegativeId), BTC_ERR_ARG, "negative vertex id %d", c.lo);
     BTC_REQUIRE(!(c.status & kPipeIdRange), BTC_ERR_ARG, "vertex id %d >= n = %d", c.hi, n_in);
     BTC_REQUIRE(!(c.status & kPipeTooManyIds), BTC_ERR_ARG, "vertex id %d: more than the pipeline's %d ids", c.hi,
                 p->n_cap);
     if (kernel_ms) *kernel_ms = tm.ms();
-    *total = *htotal;
+    *total = c.total;
     if (per_graph) {
         if (p->max_graphs > 1) std::memcpy(per_graph, hpg, (size_t)graphs * 8);
-        else per_graph[0] = *htotal;
+        else per_graph[0] = c.total;
     }
     p->last = c;
     p->ran = true;
@@ -432,8 +422,8 @@ void pipeline_copy_locked(btc_pipeline_s* p, hipStream_t s, bool with_plan, btc_
         q->n_block_items = c.item_counts[0];
         q->n_tiny_items = 0;
         btc_plan_info& in = q->info;
-        in.sparse_edges = (int64_t)c.st[1];
-        in.sparse_merge_work = (int64_t)c.st[2];
+        in.sparse_edges = (int64_t)c.m;
+        in.sparse_merge_work = (int64_t)c.rs[2];
         in.core_lists = (int64_t)c.st[3];
         in.core_rows = c.nbm;
         in.wedge_checks = (int64_t)c.checks;

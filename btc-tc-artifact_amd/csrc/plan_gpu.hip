@@ -11,9 +11,8 @@
 // edge order (a stable radix sort by pivot), and a pivot's lists are cut
 // where the running cost crosses a multiple of `chunk` rather than
 // greedily.
-#include "device_util.h"
+#include "devtile.h"
 #include "internal.h"
-#include "prim.h"
 
 namespace btcx {
 namespace {
@@ -121,6 +120,31 @@ __device__ __forceinline__ bool clip(const uint32_t* __restrict__ rowptr, const 
     s0 = lower_bound_dev(col, r0, q, lo);
     s1 = upper_bound_dev(col, s0, q, hi);
     return s1 > s0;
+}
+
+// The list of entry q (row i, whose ids below C end at ce and whose core
+// bitmap is rb): its record {s0, s_noncore, s1, bitmap} and the core words it
+// ANDs; false when it is empty.
+__device__ __forceinline__ bool list_record(const uint32_t* __restrict__ rowptr, const int32_t* __restrict__ col,
+                                            uint32_t i, uint32_t q, uint32_t ce, uint32_t rb, uint32_t C, uint4& r,
+                                            uint32_t& words) {
+    uint32_t s0, s1;
+    words = 0;
+    if (!clip(rowptr, col, i, q, s0, s1)) return false;
+    r = make_uint4(s0, s0, s1, kNoBitmap);
+    if (rb != kNoBitmap) {
+        const uint32_t j = (uint32_t)col[q];
+        const uint32_t lo = (uint32_t)col[rowptr[j]], hi = (uint32_t)col[rowptr[j + 1] - 1];
+        if ((lo & ~127u) < C) {
+            const uint32_t c1 = min(s1, ce), ids = c1 > s0 ? c1 - s0 : 0u, w = core_words(lo, hi, C);
+            if (take_core_bitmap(ids, w)) {
+                r.y = max(s0, ce);
+                r.w = rb;
+                words = w;
+            }
+        }
+    }
+    return true;
 }
 
 // Pass over the edges: list flag per edge, sparse edge count and merge work.
@@ -330,27 +354,342 @@ __global__ void place_items_kernel(const uint4* __restrict__ tmp_items, const ui
 }
 
 // ------------------------------------------------- capturable form kernels
-// pivot_offsets_kernel and core_rows_kernel in one launch.
-__global__ void pivot_core_kernel(const uint32_t* __restrict__ key, Cnt ne_, Cnt n_,
-                                  const uint32_t* __restrict__ rowptr, const int32_t* __restrict__ col, uint32_t C,
-                                  uint32_t* __restrict__ off, uint32_t* __restrict__ cend,
-                                  uint32_t* __restrict__ has) {
-    const uint32_t ne = (uint32_t)ne_.get();
-    const int64_t n = n_.get();
-    GS_LOOP(j, n + 1) off[j] = lower_bound_dev(key, 0u, ne, (uint32_t)j);
-    GS_LOOP(i, n) {
-        const uint32_t r0 = rowptr[i];
-        const uint32_t c = lower_bound_dev(col, r0, rowptr[i + 1], (int32_t)C);
-        cend[i] = c;
-        has[i] = c - r0 >= kCoreRowMin;
+// Rows of L: the end of their ids below C (cend) and the index of their core
+// bitmap (rbi; kNoBitmap for a row of fewer than kCoreRowMin of them; numbered
+// in no particular order, one atomic a workgroup).
+__global__ __launch_bounds__(kT) void pipe_rows_kernel(const uint32_t* __restrict__ rowptr,
+                                                       const int32_t* __restrict__ col, PipeCtl* __restrict__ c,
+                                                       uint32_t C, uint32_t* __restrict__ cend,
+                                                       uint32_t* __restrict__ rbi) {
+    __shared__ uint32_t s_has[kT / 64], s_base;
+    const uint32_t lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int64_t n = c->nc;
+    for (int64_t base = blockIdx.x * (int64_t)kT; base < n; base += (int64_t)gridDim.x * kT) {
+        const int64_t r = base + threadIdx.x;
+        bool has = false;
+        if (r < n) {
+            const uint32_t r0 = rowptr[r], ce = lower_bound_dev(col, r0, rowptr[r + 1], (int32_t)C);
+            cend[r] = ce;
+            has = ce - r0 >= kCoreRowMin;
+        }
+        const uint64_t some = __ballot(has);
+        if (lane == 0) s_has[wid] = (uint32_t)__popcll(some);
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            uint32_t t = 0;
+            for (int k = 0; k < kT / 64; ++k) t += s_has[k];
+            s_base = t ? atomicAdd(&c->nbm, t) : 0u;
+        }
+        __syncthreads();
+        if (r < n) {
+            uint32_t at = s_base + (uint32_t)__popcll(some & ((1ull << lane) - 1));
+            for (uint32_t k = 0; k < wid; ++k) at += s_has[k];
+            rbi[r] = has ? at : kNoBitmap;
+        }
+        __syncthreads();
     }
 }
 
-// rowbits[0, nbm * CW) = 0
-__global__ void rowbits_clear_kernel(uint32_t* __restrict__ rowbits, const uint32_t* __restrict__ d_nbm,
-                                     uint32_t CW) {
-    const int64_t n = (int64_t)*d_nbm * CW;
-    GS_LOOP(i, n) rowbits[i] = 0;
+// Entries of L in tiles: those with a list (a non-empty clipped prefix) go
+// to (pivot, entry) pairs in entry order, the list's record to rec[entry],
+// where the entries of a row share its cache lines; the sort by pivot then
+// moves 8 bytes a list and the records are fetched once, instead of every
+// list's two searches of a random row (24 R-MAT graphs, 3.3 M entries: this
+// kernel and the next 270 us against 490 us for flags, scan, pairs, records,
+// costs and their scan as kernels of their own).  ne = lists.
+template <int PER>
+__global__ __launch_bounds__(kT) void pipe_clip_kernel(const uint32_t* __restrict__ rowptr,
+                                                       const int32_t* __restrict__ col,
+                                                       const uint32_t* __restrict__ erow,
+                                                       const uint32_t* __restrict__ cend,
+                                                       const uint32_t* __restrict__ rbi, uint32_t C,
+                                                       PipeCtl* __restrict__ c, uint32_t* __restrict__ key,
+                                                       uint32_t* __restrict__ val, uint4* __restrict__ rec, SortUse su,
+                                                       ScanUse u) {
+    __shared__ DigitHist h;
+    __shared__ uint32_t lds[4 * PER + 2];
+    __shared__ uint32_t s_tile;
+    const uint32_t m = c->m;
+    sort_status_clear(su, m);  // at most m lists
+    constexpr uint32_t kTile = kT * PER;
+    const uint32_t nt = (uint32_t)(((uint64_t)m + kTile - 1) / kTile);
+    if (blockIdx.x >= nt) return;  // workgroup-uniform
+    hist_clear(h, su.passes);
+    for (TileLoop l(u.ticket, nt, &s_tile); l.next();) {
+        uint32_t f[PER], pos[PER];
+#pragma unroll
+        for (int x = 0; x < PER; ++x) {
+            const uint64_t q = (uint64_t)l.t * kTile + x * kT + threadIdx.x;
+            f[x] = 0;
+            if (q >= m) continue;
+            const uint32_t i = erow[q];
+            uint4 r;
+            uint32_t words;
+            f[x] = list_record(rowptr, col, i, (uint32_t)q, cend[i], rbi[i], C, r, words);
+            if (f[x]) rec[q] = r;
+        }
+        const uint64_t tot = tile_offsets<uint32_t, PER>(f, pos, lds, u, l.t);
+        if (l.t == nt - 1 && threadIdx.x == 0) c->ne = (uint32_t)tot;
+#pragma unroll
+        for (int x = 0; x < PER; ++x) {
+            if (!f[x]) continue;
+            const uint32_t q = l.t * kTile + x * kT + threadIdx.x, j = (uint32_t)col[q];
+            key[pos[x]] = j;
+            val[pos[x]] = q;
+            hist_add(h, su.passes, j);
+        }
+    }
+    hist_flush(h, su);
+}
+
+// The lists by pivot: records, rows, the running cost P and the range of every
+// pivot that has lists.
+template <int PER>
+__global__ __launch_bounds__(kT) void pipe_lists_kernel(const uint32_t* __restrict__ rowptr,
+                                                        const int32_t* __restrict__ col,
+                                                        const uint32_t* __restrict__ erow, uint32_t C,
+                                                        PipeCtl* __restrict__ c, const uint32_t* __restrict__ key,
+                                                        const uint32_t* __restrict__ val,
+                                                        const uint4* __restrict__ rec, uint32_t* __restrict__ off,
+                                                        uint32_t* __restrict__ oend, uint4* __restrict__ lst,
+                                                        int32_t* __restrict__ ur, uint64_t* __restrict__ P,
+                                                        ScanUse u) {
+    __shared__ uint64_t lds[4 * PER + 2];
+    __shared__ uint64_t red[kT / 64];
+    __shared__ uint32_t s_tile;
+    const uint32_t ne = c->ne;
+    constexpr uint32_t kTile = kT * PER;
+    const uint32_t nt = (uint32_t)(((uint64_t)ne + kTile - 1) / kTile);
+    uint64_t nc = 0, nn = 0;
+    for (TileLoop l(u.ticket, nt, &s_tile); l.next();) {
+        uint64_t v[PER], at[PER];
+#pragma unroll
+        for (int x = 0; x < PER; ++x) {
+            const uint64_t e = (uint64_t)l.t * kTile + x * kT + threadIdx.x;
+            v[x] = 0;
+            if (e >= ne) continue;
+            const uint32_t j = key[e], q = val[e];
+            const uint4 r = rec[q];
+            const uint32_t lo = (uint32_t)col[rowptr[j]], hi = (uint32_t)col[rowptr[j + 1] - 1];
+            const uint32_t ids = r.z > r.y ? r.z - r.y : 0u;
+            lst[e] = r;
+            ur[e] = (int32_t)erow[q];
+            v[x] = (uint64_t)ids + (r.w != kNoBitmap ? core_words(lo, hi, C) : 0u);
+            nc += r.w != kNoBitmap;
+            nn += hi < kNarrowIds ? ids : 0u;
+            if (e == 0 || key[e - 1] != j) off[j] = (uint32_t)e;
+            if (e + 1 == ne || key[e + 1] != j) oend[j] = (uint32_t)e + 1;
+        }
+        const uint64_t tot = tile_offsets<uint64_t, PER>(v, at, lds, u, l.t);
+        if (l.t == nt - 1 && threadIdx.x == 0) {
+            P[ne] = tot;
+            c->checks = tot;
+        }
+#pragma unroll
+        for (int x = 0; x < PER; ++x) {
+            const uint64_t e = (uint64_t)l.t * kTile + x * kT + threadIdx.x;
+            if (e < ne) P[e] = at[x];
+        }
+    }
+    __syncthreads();
+    nc = block_sum_u64<kT>(nc, red);
+    nn = block_sum_u64<kT>(nn, red);
+    if (threadIdx.x == 0) {
+        if (nc) atomicAdd(&c->st[3], (unsigned long long)nc);
+        if (nn) atomicAdd(&c->st[6], (unsigned long long)nn);
+    }
+}
+
+// Core bitmaps, a wave per row that has one: lane w % 64 owns word w, taken
+// 64 words (2048 ids) at a time from the row's ids below C, so a bitmap is
+// cleared, set and written in one pass without atomics.
+__global__ __launch_bounds__(kT) void pipe_core_fill_kernel(const uint32_t* __restrict__ rowptr,
+                                                            const int32_t* __restrict__ col,
+                                                            const uint32_t* __restrict__ cend,
+                                                            const uint32_t* __restrict__ rbi, uint32_t C,
+                                                            const PipeCtl* __restrict__ c,
+                                                            uint32_t* __restrict__ rowbits) {
+    if (c->nbm == 0) return;
+    const int64_t n = c->nc, waves = ((int64_t)gridDim.x * kT) >> 6;
+    const uint32_t lane = threadIdx.x & 63, CW = C / 32;
+    for (int64_t i = (blockIdx.x * (int64_t)kT + threadIdx.x) >> 6; i < n; i += waves) {
+        if (rbi[i] == kNoBitmap) continue;
+        uint32_t* b = rowbits + (size_t)rbi[i] * CW;
+        const uint32_t p1 = cend[i];
+        uint32_t p = rowptr[i];
+        for (uint32_t w0 = 0; w0 < CW; w0 += 64) {
+            uint32_t word = 0;
+            // ids of this span, 64 at a time, each lane picking its word's
+            while (p < p1) {
+                const uint32_t at = p + lane;
+                const uint32_t id = at < p1 ? (uint32_t)col[at] : 0xFFFFFFFFu;
+                const uint64_t in = __ballot(id < (w0 + 64) * 32);
+                const int cnt = __popcll(in);
+                for (int k = 0; k < cnt; ++k) {
+                    const uint32_t kid = (uint32_t)__builtin_amdgcn_readlane((int)id, k);
+                    word |= (kid >> 5) - w0 == lane ? 1u << (kid & 31u) : 0u;
+                }
+                p += (uint32_t)cnt;
+                if (cnt < 64) break;
+            }
+            if (w0 + lane < CW) b[w0 + lane] = word;
+        }
+    }
+}
+
+// List e opens a work item: the pivot's first list, or (pivots of more than
+// a wave's worth) where the running cost crosses a multiple of the cut, about
+// target_items items in all and at least 8192 checks each.  first[k] = the
+// list that opens item k.
+template <int PER>
+__global__ __launch_bounds__(kT) void pipe_first_kernel(const uint32_t* __restrict__ rowptr,
+                                                        const int32_t* __restrict__ col, PipeCtl* __restrict__ c,
+                                                        const uint32_t* __restrict__ key,
+                                                        const uint32_t* __restrict__ off,
+                                                        const uint32_t* __restrict__ oend,
+                                                        const uint64_t* __restrict__ P, uint64_t target_items,
+                                                        uint32_t* __restrict__ first, ScanUse u) {
+    __shared__ uint32_t lds[4 * PER + 2];
+    __shared__ uint32_t s_tile;
+    const uint32_t ne = c->ne;
+    const uint64_t chunk = max((uint64_t)8192, ((uint64_t)c->checks + target_items - 1) / target_items);
+    constexpr uint32_t kTile = kT * PER;
+    const uint32_t nt = (uint32_t)(((uint64_t)ne + kTile - 1) / kTile);
+    for (TileLoop l(u.ticket, nt, &s_tile); l.next();) {
+        uint32_t f[PER], pos[PER];
+#pragma unroll
+        for (int x = 0; x < PER; ++x) {
+            const uint64_t e = (uint64_t)l.t * kTile + x * kT + threadIdx.x;
+            f[x] = 0;
+            if (e >= ne) continue;
+            const uint32_t j = key[e], eb = off[j];
+            f[x] = e == eb;
+            if (!f[x]) {
+                const uint32_t t0 = rowptr[j], t1 = rowptr[j + 1];
+                if (!wave_pivot(oend[j] - eb, (uint32_t)col[t0], (uint32_t)col[t1 - 1], t1 - t0))
+                    f[x] = (P[e] - P[eb]) / chunk != (P[e - 1] - P[eb]) / chunk;
+            }
+        }
+        const uint64_t tot = tile_offsets<uint32_t, PER>(f, pos, lds, u, l.t);
+        if (l.t == nt - 1 && threadIdx.x == 0) c->nitems = (uint32_t)tot;
+#pragma unroll
+        for (int x = 0; x < PER; ++x)
+            if (f[x]) first[pos[x]] = l.t * kTile + x * kT + threadIdx.x;
+    }
+}
+
+// Bucket of an item's class and work: workgroup items before wave items, by
+// half octaves of work, heaviest first.
+__device__ __forceinline__ uint32_t item_bucket(bool small, uint64_t w) {
+    const uint32_t len = w ? 64 - __clzll(w) : 0u;
+    const uint32_t half = len >= 2 ? (uint32_t)(w >> (len - 2)) & 1u : 0u;
+    return ((small ? 1u : 0u) << 6) | (63u - min(63u, 2 * len + half));
+}
+
+// Items per bucket; pivot row words and wave items (st[4], st[5]).
+__global__ __launch_bounds__(kT) void pipe_item_keys_kernel(const uint32_t* __restrict__ rowptr,
+                                                            const int32_t* __restrict__ col, PipeCtl* __restrict__ c,
+                                                            const uint32_t* __restrict__ key,
+                                                            const uint32_t* __restrict__ off,
+                                                            const uint32_t* __restrict__ oend,
+                                                            const uint64_t* __restrict__ P,
+                                                            const uint32_t* __restrict__ first,
+                                                            uint32_t* __restrict__ skey,
+                                                            uint32_t* __restrict__ totals) {
+    __shared__ uint32_t h[kDigits];
+    __shared__ uint64_t red[kT / 64];
+    const uint32_t nitems = c->nitems, ne = c->ne;
+    if (blockIdx.x * kT >= nitems) return;  // workgroup-uniform
+    h[threadIdx.x] = 0;
+    __syncthreads();
+    uint64_t words = 0, small_items = 0;
+    GS_LOOP(k, nitems) {
+        const uint32_t eb = first[k], ee = k + 1 < nitems ? first[k + 1] : ne, j = key[eb];
+        const uint32_t t0 = rowptr[j], t1 = rowptr[j + 1];
+        const bool small = wave_pivot(oend[j] - off[j], (uint32_t)col[t0], (uint32_t)col[t1 - 1], t1 - t0);
+        const uint32_t s = item_bucket(small, P[ee] - P[eb]);
+        skey[k] = s;
+        atomicAdd(&h[s], 1u);
+        words += t1 - t0;
+        small_items += small;
+    }
+    __syncthreads();
+    const uint32_t cnt = h[threadIdx.x];
+    if (cnt) atomicAdd(&totals[threadIdx.x], cnt);
+    words = block_sum_u64<kT>(words, red);
+    small_items = block_sum_u64<kT>(small_items, red);
+    if (threadIdx.x == 0) {
+        if (words) atomicAdd(&c->st[4], (unsigned long long)words);
+        if (small_items) atomicAdd(&c->st[5], (unsigned long long)small_items);
+    }
+}
+
+// The items to their buckets (in no particular order within one), each with
+// its graph when csegs is set (the last one whose rows start at or before its
+// pivot row); workgroup 0 records the launch's item counts.
+__global__ __launch_bounds__(kT) void pipe_place_kernel(const uint32_t* __restrict__ rowptr,
+                                                        const int32_t* __restrict__ col, PipeCtl* __restrict__ c,
+                                                        const uint32_t* __restrict__ key,
+                                                        const uint64_t* __restrict__ P,
+                                                        const uint32_t* __restrict__ first,
+                                                        const uint32_t* __restrict__ skey,
+                                                        const uint32_t* __restrict__ totals,
+                                                        uint32_t* __restrict__ cursors,
+                                                        const uint32_t* __restrict__ csegs,
+                                                        uint4* __restrict__ items) {
+    __shared__ uint32_t start[kDigits], h[kDigits], wsum[kT / 64];
+    const uint32_t nitems = c->nitems, ne = c->ne, graphs = c->graphs;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        c->item_counts[0] = nitems - (uint32_t)c->st[5];
+        c->item_counts[1] = nitems;
+    }
+    if (blockIdx.x * kT >= nitems) return;  // workgroup-uniform
+    const uint32_t lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    uint32_t x = totals[threadIdx.x];
+    const uint32_t own = x;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = (uint32_t)__shfl_up((int)x, o);
+        if ((int)lane >= o) x += y;
+    }
+    if (lane == 63) wsum[wid] = x;
+    __syncthreads();
+    for (uint32_t k = 0; k < wid; ++k) x += wsum[k];
+    start[threadIdx.x] = x - own;
+    for (uint64_t k0 = (uint64_t)blockIdx.x * kT; k0 < nitems; k0 += (uint64_t)gridDim.x * kT) {
+        h[threadIdx.x] = 0;
+        __syncthreads();
+        const uint64_t k = k0 + threadIdx.x;
+        uint32_t s = 0, at = 0;
+        if (k < nitems) {
+            s = skey[k];
+            at = atomicAdd(&h[s], 1u);
+        }
+        __syncthreads();
+        const uint32_t cnt = h[threadIdx.x];
+        const uint32_t base = cnt ? atomicAdd(&cursors[threadIdx.x], cnt) : 0u;
+        __syncthreads();
+        h[threadIdx.x] = start[threadIdx.x] + base;
+        __syncthreads();
+        if (k < nitems) {
+            const uint32_t eb = first[k], ee = k + 1 < nitems ? first[k + 1] : ne, j = key[eb];
+            const uint32_t t0 = rowptr[j], t1 = rowptr[j + 1];
+            uint32_t g = 0;
+            if (csegs) {
+                uint32_t hi = graphs;  // rowptr[csegs[g]] <= t0 < rowptr[csegs[hi]]
+                while (hi - g > 1) {
+                    const uint32_t mid = (g + hi) >> 1;
+                    if (rowptr[csegs[mid]] <= t0) g = mid;
+                    else hi = mid;
+                }
+            }
+            const uint32_t r = h[s] + at;
+            items[2 * (size_t)r] = make_uint4(t0, t1, eb, ee);
+            items[2 * (size_t)r + 1] = make_uint4((uint32_t)col[t0], (uint32_t)col[t1 - 1],
+                                                  (uint32_t)min(P[ee] - P[eb], (uint64_t)0xFFFFFFFFu), g);
+        }
+        __syncthreads();
+    }
 }
 
 template <class T>
@@ -523,54 +862,41 @@ unsigned cap_grid(int64_t cap) {
         BTC_CHECK_LAUNCH(#kernel);                                                     \
     } while (0)
 
+// Kernels that end in atomics on a few addresses (reductions, digit totals).
 #define CAP_LAUNCH_RED(kernel, cap, s, ...)                                                \
-    do {                                                                               \
-        hipLaunchKernelGGL(kernel, dim3(std::min(cap_grid(cap), kCapRedBlocks)), dim3(kT), 0, s, __VA_ARGS__);  \
-        BTC_CHECK_LAUNCH(#kernel);                                                     \
+    do {                                                                                   \
+        hipLaunchKernelGGL(kernel, dim3(std::min(cap_grid(cap), 4 * kCapRedBlocks)), dim3(kT), 0, s, __VA_ARGS__);  \
+        BTC_CHECK_LAUNCH(#kernel);                                                         \
     } while (0)
-
 
 void plan_capacity(const PlanCap& c, hipStream_t s) {
     PipeCtl* ctl = c.ctl;
     const int64_t M = c.m_cap, N = c.n_cap, I = (int64_t)c.items_cap;
-    const Cnt m = Cnt::dev(&ctl->m), nc = Cnt::dev(&ctl->nc), ne = Cnt::dev(&ctl->ne),
-              nitems = Cnt::dev(&ctl->nitems);
-    const uint32_t* rowptr = c.rowptr;
-    const int32_t* col = c.col;
-    unsigned long long* st = ctl->st;  // cleared with the rest of *ctl
-
-    CAP_LAUNCH(edge_rows_kernel, N * 64, s, rowptr, nc, c.erow);
-    // prefix lists: flag, compact (pivot, edge), stable sort by pivot
-    CAP_LAUNCH_RED(clip_kernel, M, s, rowptr, col, c.erow, nullptr, m, c.lflag, st + 1);
-    dscan_u32(c.lflag, c.lpos, (size_t)M, &ctl->m, &ctl->ne, c.ws, s);
-    CAP_LAUNCH(list_keys_kernel, M, s, c.lflag, c.lpos, col, m, c.k0, c.v0);
-    const bool alt = dsort_pairs_u32(c.k0, c.v0, c.k1, c.v1, (size_t)M, &ctl->ne, id_bits(N), c.ws, s);
-    const uint32_t* key = alt ? c.k1 : c.k0;
-    const uint32_t* val = alt ? c.v1 : c.v0;
-
-    // pivot offsets and hub-core rows, bitmaps
     const uint32_t C = c.core_ids;
-    CAP_LAUNCH(pivot_core_kernel, N + 1, s, key, ne, nc, rowptr, col, C, c.off, c.cend, c.has);
-    dscan_u32(c.has, c.rbi, (size_t)N, &ctl->nc, &ctl->nbm, c.ws, s);
-    if (C) {
-        CAP_LAUNCH(rowbits_clear_kernel, (int64_t)pipe_bitmap_rows(M, c.n_cap) * (C / 32), s, c.rowbits, &ctl->nbm,
-                   C / 32);
-        CAP_LAUNCH(core_fill_kernel, N * 64, s, rowptr, col, c.cend, c.has, c.rbi, nc, C / 32, c.rowbits);
-    }
-    CAP_LAUNCH_RED(records_kernel, M, s, rowptr, col, c.erow, val, ne, c.cend, c.has, c.rbi, C, c.lists, c.ur, c.cost,
-               st + 3, st + 6);
-    dscan_u64(c.cost, c.P, (size_t)M, &ctl->ne, reinterpret_cast<uint64_t*>(&ctl->checks), c.ws, s);
-
-    // work items (each opens at a list, so there are at most ne of them):
-    // about 64 per CU, sorted by class and then work in half octaves
-    CAP_LAUNCH(item_start_kernel, M, s, rowptr, col, key, c.off, c.P, ne, (uint64_t)0, &ctl->checks,
-               (uint64_t)64 * (uint64_t)c.cus, c.start);
-    dscan_u32(c.start, c.spos, (size_t)M, &ctl->ne, &ctl->nitems, c.ws, s);
-    CAP_LAUNCH(select_kernel, M, s, c.start, c.spos, ne, c.first);
-    CAP_LAUNCH_RED(items_kernel, I, s, rowptr, col, key, c.off, c.P, c.first, nitems, ne, false, false, true, c.tmp_items,
-               c.sk0, c.sv0, st + 4);
-    const bool ialt = dsort_pairs_u32(c.sk0, c.sv0, c.sk1, c.sv1, (size_t)I, &ctl->nitems, 8, c.ws, s);
-    CAP_LAUNCH(place_items_kernel, I, s, c.tmp_items, ialt ? c.sv1 : c.sv0, nitems, c.items, ctl, c.work);
+    const SortUse su = dseq_sort(*c.seq, id_bits(c.n_cap));
+    CAP_LAUNCH(pipe_rows_kernel, N, s, c.rowptr, c.col, ctl, C, c.cend, c.rbi);
+    if (C) CAP_LAUNCH(pipe_core_fill_kernel, N * 64, s, c.rowptr, c.col, c.cend, c.rbi, C, ctl, c.rowbits);
+    with_tile_per(M, [&](auto per) {
+        constexpr int PER = decltype(per)::value;
+        // prefix lists: records by entry, (pivot, entry) pairs, stably sorted by pivot
+        CAP_LAUNCH_RED(pipe_clip_kernel<PER>, M / PER + 1, s, c.rowptr, c.col, c.erow, c.cend, c.rbi, C, ctl, c.k0, c.v0,
+                       c.rec, su, dseq_scan(*c.seq));
+        const bool alt = dsort_pairs_u32(c.k0, c.v0, c.k1, c.v1, (size_t)M, &ctl->ne, su, s);
+        const uint32_t* key = alt ? c.k1 : c.k0;
+        const uint32_t* val = alt ? c.v1 : c.v0;
+        // records, costs and pivots' ranges in list order
+        CAP_LAUNCH_RED(pipe_lists_kernel<PER>, M / PER + 1, s, c.rowptr, c.col, c.erow, C, ctl, key, val, c.rec, c.off,
+                       c.oend, c.lists, c.ur, c.P, dseq_scan(*c.seq));
+        // work items (each opens at a list, so there are at most ne of them):
+        // about 64 per CU, by class and then work in half octaves
+        CAP_LAUNCH(pipe_first_kernel<PER>, M / PER + 1, s, c.rowptr, c.col, ctl, key, c.off, c.oend, c.P,
+                   (uint64_t)64 * (uint64_t)c.cus, c.first, dseq_scan(*c.seq));
+        const SortUse iu = dseq_sort(*c.seq, kDigitBits);  // its words: bucket totals, then cursors
+        CAP_LAUNCH_RED(pipe_item_keys_kernel, I, s, c.rowptr, c.col, ctl, key, c.off, c.oend, c.P, c.first, c.skey,
+                       iu.totals);
+        CAP_LAUNCH_RED(pipe_place_kernel, I, s, c.rowptr, c.col, ctl, key, c.P, c.first, c.skey, iu.totals,
+                       iu.totals + kDigits, c.csegs, c.items);
+    });
 }
 
 }  // namespace btcx

@@ -25,39 +25,41 @@ bool sort_pairs_u32(uint32_t* keys, uint32_t* vals, uint32_t* kt, uint32_t* vt, 
 void exclusive_scan_u32(const uint32_t* in, uint32_t* out, size_t n, hipStream_t s);
 void exclusive_scan_u64(const uint64_t* in, uint64_t* out, size_t n, hipStream_t s);
 
-// Capturable forms (devprim.hip).  The element count n is read from device
-// memory (*d_n) when the kernels run, buffers hold `cap` elements (n <= cap),
-// and the caller's workspace `ws` (dprim_ws_bytes(cap) bytes, 256-byte
-// aligned, zeroed once before its first use) holds every temporary: the
-// kernels are the only work enqueued, so one stream capture serves every n
-// up to cap.  Each call leaves the workspace's tickets, totals and statuses
-// zeroed again for the next call on the same stream; calls sharing a
-// workspace must not overlap.
-
-size_t dprim_ws_bytes(size_t cap);
-
-// The workspace: its device address and the capacity it was sized for
-// (its layout follows from that, whatever the capacity of a call).
-struct DevWs {
+// Capturable forms (devprim.hip, devtile.h).  The element count n is read
+// from device memory (*d_n) when the kernels run, buffers hold `cap` elements
+// (n <= cap), and a workspace (dseq_bytes(cap) bytes, 256-byte aligned)
+// holds every temporary: kernels are the only work enqueued, so one stream
+// capture serves every n up to cap.
+//
+// A run of sorts and scans in stream order takes its uses from one DevSeq
+// when it is enqueued: each has tickets, totals and scan statuses of its
+// own, all of them in the words [0, dseq_clear_words) that the run's first
+// kernel clears (but for word kSeqErr, which stays).  A sort's statuses are
+// shared by all and cleared by the kernel that writes its keys.
+constexpr uint32_t kSortTile = 2048;  // keys of a sort's tile
+constexpr int kMaxSorts = 6, kMaxScans = 8;
+constexpr uint32_t kSeqErr = 0;
+struct SortUse;
+struct ScanUse;
+struct DevSeq {
     void* p = nullptr;
     size_t cap = 0;
+    int sorts = 0, scans = 0;
 };
+size_t dseq_bytes(size_t cap);
+size_t dseq_clear_words(size_t cap);
+SortUse dseq_sort(DevSeq& q, int end_bit);
+ScanUse dseq_scan(DevSeq& q);
 
-// out[i] = sum of in[0, i) for i <= n; out[n] and *d_total (when set) get
-// the total.
-void dscan_u32(const uint32_t* in, uint32_t* out, size_t cap, const uint32_t* d_n, uint32_t* d_total,
-               const DevWs& ws, hipStream_t s);
-void dscan_u64(const uint64_t* in, uint64_t* out, size_t cap, const uint32_t* d_n, uint64_t* d_total,
-               const DevWs& ws, hipStream_t s);
+// Word that a sort or scan sets (and nothing clears) if a look-back ever ran
+// past its spin limit -- a result that cannot be trusted.
+const uint32_t* dseq_error_word(const DevSeq& q);
 
-// Word of ws that a sort or scan sets (and nothing clears) if a look-back
-// ever ran past its spin limit -- a result that cannot be trusted.
-const uint32_t* dsort_error_word(const DevWs& ws);
-
-// Stable radix sorts on bits [0, end_bit), as sort_u64 / sort_pairs_u32.
-uint64_t* dsort_u64(uint64_t* keys, uint64_t* tmp, size_t cap, const uint32_t* d_n, int end_bit, const DevWs& ws,
-                    hipStream_t s);
+// The passes of a stable radix sort whose keys' writer filled in u.  u64
+// keys: returns the buffer that holds the result; pairs: whether the result
+// is in (kt, vt).
+uint64_t* dsort_u64(uint64_t* keys, uint64_t* tmp, size_t cap, const uint32_t* d_n, const SortUse& u, hipStream_t s);
 bool dsort_pairs_u32(uint32_t* keys, uint32_t* vals, uint32_t* kt, uint32_t* vt, size_t cap, const uint32_t* d_n,
-                     int end_bit, const DevWs& ws, hipStream_t s);
+                     const SortUse& u, hipStream_t s);
 
 }  // namespace btcx
