@@ -152,6 +152,7 @@ void batch_finish(btc_batch_s* b, const btc_count_opts* opts, hipStream_t s) {
     b->d_pv.alloc_on((size_t)b->graph.n, b->graph.max_row, s);
     b->d_pg.alloc_on((size_t)b->count, s);
     b->h_pg.assign((size_t)b->count, 0);
+    host_words(((size_t)b->count + 1) * 8);  // what a count returns through
     BTC_HIP(hipMemcpyAsync(b->d_voff.p, vo32.data(), vo32.size() * 4, hipMemcpyHostToDevice, s));
     batch_item_graphs(b, s);
     BTC_HIP(hipStreamSynchronize(s));
@@ -182,6 +183,7 @@ btc_batch_s* batch_from_plan(btc_graph_s&& g, btc_plan_s* plan, const std::vecto
     b->d_pv.alloc_on((size_t)b->graph.n, b->graph.max_row, s);
     b->d_pg.alloc_on((size_t)b->count, s);
     b->h_pg.assign((size_t)b->count, 0);
+    host_words(((size_t)b->count + 1) * 8);  // what a count returns through
     BTC_HIP(hipMemcpyAsync(b->d_voff.p, vo32.data(), vo32.size() * 4, hipMemcpyHostToDevice, s));
     batch_item_graphs(b.get(), s);
     BTC_HIP(hipStreamSynchronize(s));
@@ -374,10 +376,13 @@ int btc_batch_count(btc_batch b, void* stream, uint64_t* per_graph, uint64_t* to
             b->enqueue_count(s);
         }
         if (kernel_ms) tm.stop(s);  // both kernels and the per-graph sums
-        unsigned long long t = 0;
-        BTC_HIP(hipMemcpyAsync(&t, b->plan->scratch.p, 8, hipMemcpyDeviceToHost, s));
-        BTC_HIP(hipMemcpyAsync(b->h_pg.data(), b->d_pg.p, (size_t)b->count * 8, hipMemcpyDeviceToHost, s));
+        // through pinned memory: the total, then the graphs' sums
+        unsigned long long* const h = reinterpret_cast<unsigned long long*>(btcx::host_words(((size_t)b->count + 1) * 8));
+        BTC_HIP(hipMemcpyAsync(h, b->plan->scratch.p, 8, hipMemcpyDeviceToHost, s));
+        BTC_HIP(hipMemcpyAsync(h + 1, b->d_pg.p, (size_t)b->count * 8, hipMemcpyDeviceToHost, s));
         BTC_HIP(hipStreamSynchronize(s));
+        const unsigned long long t = h[0];
+        std::copy(h + 1, h + 1 + b->count, b->h_pg.begin());
         if (kernel_ms) *kernel_ms = tm.ms();
         uint64_t sum = 0;
         for (auto x : b->h_pg) sum += x;

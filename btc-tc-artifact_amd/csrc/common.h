@@ -232,6 +232,14 @@ struct PinnedBuf {
     char* reserve(size_t bytes);
 };
 
+// Pinned memory of the calling thread for what a call returns: the count
+// kernels write a total (and a batch its graphs' sums) there themselves, so
+// no copy to the host follows them.  host_words(bytes) may move the block
+// when it grows: a call asks for its words before it takes host_total().
+constexpr size_t kHostTotalBytes = 64;
+char* host_words(size_t bytes);
+unsigned long long* host_total();
+
 // Copies count host arrays of `bytes` each into device memory (dev[k]) on
 // stream s and waits: through a thread's cached pinned staging, two 16 MiB
 // chunks at a time for large arrays (host threads fill one chunk while the
@@ -287,6 +295,7 @@ struct CapturedGraph {
 // Kernel timing with HIP events recorded on the launch stream.
 struct EventTimer {
     hipEvent_t a = nullptr, b = nullptr;
+    int dev = 0;
     bool on = false;
     explicit EventTimer(bool enable);
     ~EventTimer();
@@ -356,6 +365,10 @@ struct PvBuf {
     bool wide() const { return b64.p != nullptr; }
     void* data() const { return b64.p ? (void*)b64.p : (void*)b32.p; }
     size_t bytes() const { return n * (b64.p ? 8 : 4); }
+    // what copy_out takes of the thread's pinned words: everything up to
+    // kStageMax, else nothing
+    static constexpr size_t kStageMax = size_t(16) << 20;
+    size_t staged() const { return bytes() <= kStageMax ? bytes() : 0; }
     // Copies the sums to host int32 (h32; BTC_ERR_OVERFLOW when a count
     // does not fit) or int64 (h64) after the work on s; synchronises s.
     void copy_out(int32_t* h32, int64_t* h64, hipStream_t s) const;

@@ -32,6 +32,7 @@
 #include <cstring>
 #include <mutex>
 #include <numeric>
+#include <unordered_map>
 
 #include "device_util.h"
 #include "internal.h"
@@ -959,6 +960,19 @@ void check_launch_opts(const btc_count_opts& o) {
 
 namespace {
 
+// Resident workgroups of a kernel per CU (at least 1), asked for once per
+// kernel: every device this builds for is a gfx950.
+int blocks_per_cu(const void* fn) {
+    static std::mutex mu;
+    static std::unordered_map<const void*, int> known;
+    std::lock_guard<std::mutex> lk(mu);
+    const auto it = known.find(fn);
+    if (it != known.end()) return it->second;
+    int per_cu = 0;
+    BTC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kThreads, 0));
+    return known[fn] = std::max(1, per_cu);
+}
+
 // W64: 64-bit byte offsets into L, in the default shape only (4 lanes per
 // list, one load in flight).
 WedgeFn wedge_fn(const btc_count_opts& o, bool pv, bool w64, unsigned* grid, bool gs = false) {
@@ -966,9 +980,7 @@ WedgeFn wedge_fn(const btc_count_opts& o, bool pv, bool w64, unsigned* grid, boo
     const int U = o.unroll ? o.unroll : 1;
     WedgeFn fn = w64 ? (pv ? wedge_kernel<4, 1, true, true, false> : wedge_kernel<4, 1, false, true, false>)
                      : pick_wedge(G, U, pv, gs);
-    int per_cu = 0;
-    BTC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(fn), kThreads, 0));
-    per_cu = std::max(1, per_cu);
+    int per_cu = blocks_per_cu(reinterpret_cast<const void*>(fn));
     if (o.waves_per_eu > 0) per_cu = std::min(per_cu, (int)o.waves_per_eu);
     *grid = (unsigned)(device_cu_count() * per_cu);
     return fn;
@@ -1019,11 +1031,10 @@ void launch_tiny(btc_plan_s* p, unsigned long long* d_total, PvOut d_pv, hipStre
     auto fn = wide_offsets(p) ? (d_pv.on() ? tiny_kernel<true, true, false> : tiny_kernel<false, true, false>)
                               : (d_pv.on() ? tiny_kernel<true, false, false>
                                            : (gs ? tiny_kernel<false, false, true> : tiny_kernel<false, false, false>));
-    int per_cu = 0;
-    BTC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(fn), kThreads, 0));
+    const int per_cu = blocks_per_cu(reinterpret_cast<const void*>(fn));
     constexpr uint32_t kGroups = kThreads / kTinyLanes;
     const unsigned grid =
-        (unsigned)std::min<int64_t>((int64_t)device_cu_count() * std::max(1, per_cu), (n + kGroups - 1) / kGroups);
+        (unsigned)std::min<int64_t>((int64_t)device_cu_count() * per_cu, (n + kGroups - 1) / kGroups);
     hipLaunchKernelGGL(fn, dim3(grid), dim3(kThreads), 0, s, plan_dev(p, d_total, d_pv), (int)p->launch.lookup,
                        p->nitems - p->n_tiny_items, n, share, shares, d_slots);
     BTC_CHECK_LAUNCH("tiny_kernel");
@@ -1129,6 +1140,7 @@ void plans_count(btc_plan_s* const* P, int k, hipStream_t s, uint64_t* totals, M
     }
     for (int j = 0; j < k; ++j)
         if (P[j]->n_dense) {
+            P[j]->scratch_clean = false;
             launch_zero_u32(reinterpret_cast<uint32_t*>(P[j]->scratch.p + kWorkSlots), 2 * kSlotWords, s);
             launch_plan_dense(P[j], P[j]->scratch.p + kWorkSlots, PvOut{}, s);
             launch_slot_sum(P[j]->scratch.p + kWorkSlots, ws.totals.p + j, s);
@@ -1176,14 +1188,21 @@ void ensure_side_stream(btc_plan_s* p) {
 }
 
 void plan_enqueue(btc_plan_s* p, hipStream_t s, PvOut d_pv, EventTimer* tm, EventTimer* tw,
-                  unsigned long long* d_work, bool make_streams) {
+                  unsigned long long* d_work, bool make_streams, unsigned long long* h_total) {
     BTC_REQUIRE(!d_pv.p32 || p->g->max_row <= kPv32MaxRow, BTC_ERR_STATE,
                 "longest row %d: per-vertex counts need 64-bit slots", p->g->max_row);
-    if (!d_work) d_work = p->scratch.p;
-    launch_zero_u32(reinterpret_cast<uint32_t*>(d_work), 2 * kWorkWords, s);  // total, counters and slots
+    const bool own = !d_work;
+    if (own) d_work = p->scratch.p;
+    if (!own || !h_total || !p->scratch_clean)  // total, counters and slots
+        launch_zero_u32(reinterpret_cast<uint32_t*>(d_work), 2 * kWorkWords, s);
+    if (own) p->scratch_clean = false;
     unsigned long long* d_total = d_work;
     uint32_t* d_counters = reinterpret_cast<uint32_t*>(d_work + 1);
     unsigned long long* d_slots = d_work + kWorkSlots;
+    auto finish = [&] {
+        if (h_total) launch_count_finish(d_work, h_total, s);
+        else launch_slot_sum(d_slots, d_total, s);
+    };
     if ((p->n_dense || p->n_tiny_items) && p->nitems && p->info.wedge_checks >= kOverlapChecks &&
         (make_streams || p->side)) {
         // the latency-bound tiny-pivot and dense-tile kernels run on two
@@ -1211,7 +1230,7 @@ void plan_enqueue(btc_plan_s* p, hipStream_t s, PvOut d_pv, EventTimer* tm, Even
             BTC_HIP(hipStreamWaitEvent(s, p->ev_join, 0));
         }
         if (p->n_tiny_items) BTC_HIP(hipStreamWaitEvent(s, p->ev_join2, 0));
-        launch_slot_sum(d_slots, d_total, s);
+        finish();
         if (tm) tm->stop(s);
         return;
     }
@@ -1221,7 +1240,7 @@ void plan_enqueue(btc_plan_s* p, hipStream_t s, PvOut d_pv, EventTimer* tm, Even
     if (p->nitems) launch_wedge(p, d_total, d_counters, d_pv, s, 0, 1, d_slots);
     if (tw) tw->stop(s);
     if (p->n_tiny_items) launch_tiny(p, d_total, d_pv, s, 0, 1, d_slots);
-    launch_slot_sum(d_slots, d_total, s);
+    finish();
     if (tm) tm->stop(s);
 }
 
@@ -1235,6 +1254,7 @@ void plan_count(btc_plan_s* p, hipStream_t s, uint64_t* total, int32_t* pv32, in
         // replay of the captured totals-only count
         EventTimer tm(kernel_ms != nullptr);
         tm.start(s);
+        p->scratch_clean = false;  // the replay clears its words first and leaves its total
         p->count_graph.launch(s);
         tm.stop(s);
         unsigned long long h = 0;
@@ -1252,15 +1272,19 @@ void plan_count(btc_plan_s* p, hipStream_t s, uint64_t* total, int32_t* pv32, in
         pv.alloc_on((size_t)g->n, g->max_row, s);
         BTC_HIP(hipMemsetAsync(pv.data(), 0, pv.bytes(), s));
     }
-    EventTimer tm(kernel_ms != nullptr), tw(kernel_ms != nullptr);
-    plan_enqueue(p, s, pv.out(), &tm, &tw);
-    unsigned long long h = 0;
-    BTC_HIP(hipMemcpyAsync(&h, p->scratch.p, 8, hipMemcpyDeviceToHost, s));
+    host_words(pv.staged());
+    unsigned long long* const h_total = host_total();
+    // the wedge kernel is timed apart only where others run beside it
+    const bool parts = p->n_dense || p->n_tiny_items;
+    EventTimer tm(kernel_ms != nullptr), tw(kernel_ms != nullptr && parts);
+    plan_enqueue(p, s, pv.out(), &tm, &tw, nullptr, true, h_total);
     pv.copy_out(pv32, pv64, s);  // synchronises s
+    p->scratch_clean = true;
+    const uint64_t h = *h_total;
     pv.release_on(s);
     if (kernel_ms) {
         *kernel_ms = tm.ms();
-        p->last_wedge_ms = tw.ms();
+        p->last_wedge_ms = parts ? tw.ms() : *kernel_ms;
         p->last_dense_ms = p->n_dense || p->n_tiny_items ? std::max(0.f, *kernel_ms - p->last_wedge_ms) : 0.f;
     }
     *total = h;
@@ -1339,7 +1363,8 @@ btc_plan_s* plan_create(btc_graph g, const btc_count_opts* opts, hipStream_t s, 
     if (p->n_dense) p->n_units = btcx::build_dense_units(p->bsr, p->dense_list.p, p->n_dense, p->dense_units, s);
     p->scratch.alloc_on(btcx::kWorkWords, s);
     BTC_HIP(hipMemsetAsync(p->scratch.p, 0, p->scratch.bytes(), s));
-    BTC_HIP(hipStreamSynchronize(s));  // counts may run on other streams (every count clears these words again)
+    BTC_HIP(hipStreamSynchronize(s));  // counts may run on other streams
+    p->scratch_clean = true;
     p->info.tile_k = p->K;
     p->info.tau = p->tau;
     p->info.core_ids = p->core_ids;
@@ -1392,6 +1417,7 @@ int btc_plan_count_share(btc_plan p, int32_t shares, int32_t share, void* stream
         BTC_REQUIRE(shares >= 1 && share >= 0 && share < shares, BTC_ERR_ARG, "share %d of %d", share, shares);
         hipStream_t s = btcx::as_stream(stream);
         const uint32_t k = (uint32_t)shares, j = (uint32_t)share;
+        p->scratch_clean = false;
         btcx::launch_zero_u32(reinterpret_cast<uint32_t*>(p->scratch.p), 2 * btcx::kWorkWords, s);
         btcx::EventTimer tm(kernel_ms != nullptr);
         tm.start(s);

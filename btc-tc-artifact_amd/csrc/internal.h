@@ -40,6 +40,7 @@ struct btc_bitbsr_s {
     btcx::RowLists rows;
     btcx::DevBuf<uint32_t> pop;  // nblk: set bits of every tile
     btcx::DevBuf<unsigned long long> work;  // kWorkWords: [0] total, slots
+    bool work_clean = false;  // the last count left work cleared
 };
 
 struct btc_pipeline_s;
@@ -76,6 +77,7 @@ struct btc_plan_s {
     uint32_t n_block_items = 0;
     uint32_t n_tiny_items = 0;  // the last items: tiny pivots (tiny_pivot)
     btcx::DevBuf<unsigned long long> scratch;  // kWorkWords: [0] total, [1] work-item counters, slots
+    bool scratch_clean = false;  // the last count left scratch cleared (plan_enqueue)
     btc_plan_info info{};
     float last_dense_ms = 0.f;
     float last_wedge_ms = 0.f;
@@ -399,6 +401,11 @@ void launch_dense_part(const btc_bitbsr_s* b, int tau, bool mfma, uint4* units, 
 // *d_result += sum of the kSlots slots at d_slots, which are cleared.
 void launch_slot_sum(unsigned long long* d_slots, unsigned long long* d_result, hipStream_t s);
 
+// The last kernel of a count whose result the host waits for: the sum of the
+// total and the slots to *h_total (pinned host memory), the count's work
+// words (kWorkWords at d_work) cleared for the next count.
+void launch_count_finish(unsigned long long* d_work, unsigned long long* h_total, hipStream_t s);
+
 // p[0, n) = 0 by a kernel (safe inside captured graphs).
 void launch_zero_u32(uint32_t* p, size_t n, hipStream_t s);
 
@@ -429,7 +436,11 @@ void plans_count(btc_plan_s* const* plans, int k, hipStream_t s, uint64_t* total
 // all kernels, tw the wedge kernel (either may be NULL).  With make_streams
 // false the dense-tile and tiny-pivot kernels run beside the wedge kernel
 // only when the plan's side streams exist already (no stream is created).
+// With h_total (pinned host memory; d_work NULL) the total goes there and the
+// work words are left cleared: the caller sets p->scratch_clean once it has
+// waited for the count, which saves the next one its clearing kernel.
 void plan_enqueue(btc_plan_s* p, hipStream_t s, PvOut d_pv, EventTimer* tm, EventTimer* tw,
-                  unsigned long long* d_work = nullptr, bool make_streams = true);
+                  unsigned long long* d_work = nullptr, bool make_streams = true,
+                  unsigned long long* h_total = nullptr);
 
 }  // namespace btcx

@@ -32,15 +32,40 @@ void fail(int code, const char* fmt, ...) {
     throw Error{code};
 }
 
+// Events of this thread that no timer holds, by device: creating and
+// destroying a pair took 3 us of a small count.
+struct TimerEvents {
+    std::vector<hipEvent_t> free[64];
+    ~TimerEvents() {
+        for (auto& v : free)
+            for (hipEvent_t e : v) (void)hipEventDestroy(e);
+    }
+};
+static thread_local TimerEvents tl_events;
+
 EventTimer::EventTimer(bool enable) : on(enable) {
     if (!on) return;
-    BTC_HIP(hipEventCreate(&a));
-    BTC_HIP(hipEventCreate(&b));
+    BTC_HIP(hipGetDevice(&dev));
+    auto take = [this] {
+        hipEvent_t e = nullptr;
+        if (dev < 64 && !tl_events.free[dev].empty()) {
+            e = tl_events.free[dev].back();
+            tl_events.free[dev].pop_back();
+        } else {
+            BTC_HIP(hipEventCreate(&e));
+        }
+        return e;
+    };
+    a = take();
+    b = take();
 }
 
 EventTimer::~EventTimer() {
-    if (a) (void)hipEventDestroy(a);
-    if (b) (void)hipEventDestroy(b);
+    for (hipEvent_t e : {a, b}) {
+        if (!e) continue;
+        if (dev < 64 && tl_events.free[dev].size() < 8) tl_events.free[dev].push_back(e);
+        else (void)hipEventDestroy(e);
+    }
 }
 
 void EventTimer::start(hipStream_t s) {
@@ -366,9 +391,43 @@ void upload_arrays(const void* const* host, void* const* dev, int count, size_t 
     BTC_HIP(e);
 }
 
+// 64-bit sums to int32, each checked.
+static void narrow_sums(const unsigned long long* t, size_t n, int32_t* h32) {
+    for (size_t v = 0; v < n; ++v) {
+        BTC_REQUIRE(t[v] <= (unsigned long long)INT32_MAX, BTC_ERR_OVERFLOW,
+                    "vertex %zu closes %llu triangles, beyond int32 per-vertex output (the int64 entry points "
+                    "return it)", v, t[v]);
+        h32[v] = (int32_t)t[v];
+    }
+}
+
+char* host_words(size_t bytes) {
+    static thread_local PinnedBuf words;
+    return words.reserve(bytes + kHostTotalBytes) + kHostTotalBytes;
+}
+
+unsigned long long* host_total() { return reinterpret_cast<unsigned long long*>(host_words(0) - kHostTotalBytes); }
+
 void PvBuf::copy_out(int32_t* h32, int64_t* h64, hipStream_t s) const {
     if (n == 0 || (!h32 && !h64)) {
         BTC_HIP(hipStreamSynchronize(s));
+        return;
+    }
+    // up to kStageMax bytes come through pinned memory of the thread (a copy
+    // to pageable memory is staged by the runtime at a third of the rate)
+    if (staged()) {
+        const void* d = b64.p ? (const void*)b64.p : (const void*)b32.p;
+        char* const pin = host_words(bytes());
+        BTC_HIP(hipMemcpyAsync(pin, d, bytes(), hipMemcpyDeviceToHost, s));
+        BTC_HIP(hipStreamSynchronize(s));
+        if (wide() == (h64 != nullptr)) {
+            std::memcpy(h64 ? (void*)h64 : (void*)h32, pin, bytes());
+        } else if (h64) {
+            const int32_t* t = reinterpret_cast<const int32_t*>(pin);
+            for (size_t v = 0; v < n; ++v) h64[v] = t[v];
+        } else {
+            narrow_sums(reinterpret_cast<const unsigned long long*>(pin), n, h32);
+        }
         return;
     }
     if (!wide() && h32) {
@@ -391,12 +450,7 @@ void PvBuf::copy_out(int32_t* h32, int64_t* h64, hipStream_t s) const {
     std::vector<unsigned long long> t(n);  // 64-bit slots narrowed, each checked
     BTC_HIP(hipMemcpyAsync(t.data(), b64.p, n * 8, hipMemcpyDeviceToHost, s));
     BTC_HIP(hipStreamSynchronize(s));
-    for (size_t v = 0; v < n; ++v) {
-        BTC_REQUIRE(t[v] <= (unsigned long long)INT32_MAX, BTC_ERR_OVERFLOW,
-                    "vertex %zu closes %llu triangles, beyond int32 per-vertex output (the int64 entry points "
-                    "return it)", v, t[v]);
-        h32[v] = (int32_t)t[v];
-    }
+    narrow_sums(t.data(), n, h32);
 }
 
 }  // namespace btcx
