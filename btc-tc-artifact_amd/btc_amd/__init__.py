@@ -170,6 +170,8 @@ _SIGS = {
                                      C.POINTER(C.c_float)]),
     "btc_pipeline_create_batch": (C.c_int, [C.c_int32, C.c_int64, C.c_int32, C.c_uint32, C.POINTER(CountOpts), vp,
                                             C.POINTER(vp)]),
+    "btc_pipeline_count_graphs": (C.c_int, [vp, vp, vp, vp, vp, C.c_int32, vp, vp, C.POINTER(C.c_uint64),
+                                            C.POINTER(C.c_float)]),
     "btc_pipeline_count_batch": (C.c_int, [vp, vp, vp, vp, vp, C.c_int32, vp, vp, C.POINTER(C.c_uint64),
                                            C.POINTER(C.c_float)]),
     "btc_pipeline_export_batch": (C.c_int, [vp, vp, C.POINTER(vp)]),
@@ -478,17 +480,19 @@ class Pipeline:
 
     def count_batch(self, graphs, stream=None):
         """(total, per-graph uint64 array, kernel_ms) of [(src, dst, n), ...]
-        in one run (btc_pipeline_count_batch)."""
+        in one run (btc_pipeline_count_graphs)."""
         k = len(graphs)
-        off = np.zeros(k + 1, np.int64)
-        off[1:] = np.cumsum([len(g[0]) for g in graphs])
-        src = np.ascontiguousarray(np.concatenate([np.asarray(g[0], np.int32) for g in graphs]), np.int32)
-        dst = np.ascontiguousarray(np.concatenate([np.asarray(g[1], np.int32) for g in graphs]), np.int32)
+        pairs = [(np.ascontiguousarray(g[0], np.int32), np.ascontiguousarray(g[1], np.int32)) for g in graphs]
+        if any(u.shape != v.shape for u, v in pairs):
+            raise ValueError("src and dst differ in length")
+        src = np.array([u.ctypes.data for u, _ in pairs], np.uint64)
+        dst = np.array([v.ctypes.data for _, v in pairs], np.uint64)
+        size = np.array([u.size for u, _ in pairs], np.int64)
         nv = np.ascontiguousarray([g[2] for g in graphs], np.int32)
         per = np.zeros(k, np.uint64)
         total, ms = C.c_uint64(0), C.c_float(0)
-        _check(lib().btc_pipeline_count_batch(self._h, _ptr(src), _ptr(dst), _ptr(off), _ptr(nv), k, stream,
-                                              _ptr(per), C.byref(total), C.byref(ms)))
+        _check(lib().btc_pipeline_count_graphs(self._h, _ptr(src), _ptr(dst), _ptr(size), _ptr(nv), k, stream,
+                                               _ptr(per), C.byref(total), C.byref(ms)))
         return total.value, per, ms.value
 
     def export_batch(self, stream=None):

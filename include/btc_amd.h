@@ -423,11 +423,16 @@ int btc_pipeline_count(btc_pipeline p, const int32_t* src, const int32_t* dst, i
                        int32_t device_pairs, void* stream, uint64_t* total, float* kernel_ms);
 /* count graphs in one run (host pairs, the layout of btc_batch_from_coo:
  * graph k's pairs are src/dst[edge_offsets[k], edge_offsets[k+1]) over ids
- * [0, n_per_graph[k]), n <= 0: its largest id + 1; ids are checked on the
- * host); per_graph[k] (may be NULL) = graph k's triangles, *total = all. */
+ * [0, n_per_graph[k]), n <= 0: its largest id + 1; an id out of
+ * range refuses the call and leaves the last run as it was); per_graph[k] (may be NULL) = graph k's triangles, *total = all. */
 int btc_pipeline_count_batch(btc_pipeline p, const int32_t* src, const int32_t* dst, const int64_t* edge_offsets,
                              const int32_t* n_per_graph, int32_t count, void* stream, uint64_t* per_graph,
                              uint64_t* total, float* kernel_ms);
+/* The same with every graph's pairs in arrays of its own: graph k's are
+ * src[k] / dst[k][0, pairs[k]). */
+int btc_pipeline_count_graphs(btc_pipeline p, const int32_t* const* src, const int32_t* const* dst,
+                              const int64_t* pairs, const int32_t* n_per_graph, int32_t count, void* stream,
+                              uint64_t* per_graph, uint64_t* total, float* kernel_ms);
 /* A copy of the last accepted run's canonical graph, in HBM: the same L and
  * labels as btc_graph_from_coo_device of the same pairs. */
 int btc_pipeline_graph(btc_pipeline p, void* stream, btc_graph* out);

@@ -36,3 +36,35 @@ def test_tile_edges(gpu, orc, e_cap, flags):
         assert np.array_equal(rp, rp2) and np.array_equal(col, col2), (e, n, kind)
         assert np.array_equal(host.labels(), q.labels()), (e, n, kind)
         assert total == orc.tc_merge(rp, col, threads=4), (e, n, kind)
+
+
+@pytest.mark.parametrize("k", [1, 2, 63, 64])
+def test_group_ranges_on_the_device(gpu, orc, k):
+    """Several graphs whose ids are checked and moved by the device: empty
+    graphs, ranges taken from the pairs (n <= 0), arrays on both sides of a
+    staging piece; a refused call names the first bad graph and leaves the
+    last run's batch exportable."""
+    rng = np.random.default_rng(k)
+    p = gpu.Pipeline(1 << 17, 1 << 19, 3, max_graphs=64)
+    gs = []
+    for g in range(k):
+        n = int(rng.integers(1, 1500))
+        e = 0 if g % 7 == 3 else int(rng.integers(1, 6 * n + 2))
+        if g == 1:
+            n, e = 4000, (1 << 16) + 5
+        s, d = (rng.integers(0, n, e).astype(np.int32) for _ in range(2))
+        gs.append((s, d, 0 if g % 5 == 4 else n))
+    want = []
+    for s, d, n in gs:
+        rp, col = gpu.Graph.from_coo(s, d, n or int(max(s.max(initial=0), d.max(initial=0))) + 1).csr()
+        want.append(orc.tc_merge(rp, col, threads=1))
+    total, per, _ = p.count_batch(gs)
+    assert list(per) == want and total == sum(want)
+    for bad in (-1, 1500):
+        worse = [(s.copy(), d, n) for s, d, n in gs] + [(np.array([0, bad], np.int32), np.array([1, 1], np.int32), 7)]
+        worse = worse[-64:]
+        with pytest.raises(gpu.BtcError, match="graph %d: vertex id" % (len(worse) - 1)):
+            p.count_batch(worse)
+        assert list(p.export_batch().count()[1]) == want
+    total, per, _ = p.count_batch(gs[::-1])
+    assert list(per) == want[::-1]
