@@ -48,6 +48,14 @@ int id_bits(int64_t n) {
         BTC_CHECK_LAUNCH(#kernel);                                                  \
     } while (0)
 
+// The passes over entries and lists: bound by the latency of their dependent
+// loads, so they fill the chip twice over.
+#define BTC_LAUNCH_CLIP(kernel, n, s, ...)                                                  \
+    do {                                                                                    \
+        hipLaunchKernelGGL(kernel, dim3(std::min(grid_for(n), 4 * kRedBlocks)), dim3(kT), 0, s, __VA_ARGS__); \
+        BTC_CHECK_LAUNCH(#kernel);                                                          \
+    } while (0)
+
 // First index in [lo, hi) of a[] with a[x] >= v (a ascending).
 template <class T>
 __device__ __forceinline__ uint32_t lower_bound_dev(const T* a, uint32_t lo, uint32_t hi, T v) {
@@ -123,13 +131,11 @@ __device__ __forceinline__ bool clip(const uint32_t* __restrict__ rowptr, const 
 }
 
 // The list of entry q (row i, whose ids below C end at ce and whose core
-// bitmap is rb): its record {s0, s_noncore, s1, bitmap} and the core words it
-// ANDs; false when it is empty.
+// bitmap is rb): its record {s0, s_noncore, s1, bitmap}; false when it is
+// empty.
 __device__ __forceinline__ bool list_record(const uint32_t* __restrict__ rowptr, const int32_t* __restrict__ col,
-                                            uint32_t i, uint32_t q, uint32_t ce, uint32_t rb, uint32_t C, uint4& r,
-                                            uint32_t& words) {
+                                            uint32_t i, uint32_t q, uint32_t ce, uint32_t rb, uint32_t C, uint4& r) {
     uint32_t s0, s1;
-    words = 0;
     if (!clip(rowptr, col, i, q, s0, s1)) return false;
     r = make_uint4(s0, s0, s1, kNoBitmap);
     if (rb != kNoBitmap) {
@@ -140,18 +146,23 @@ __device__ __forceinline__ bool list_record(const uint32_t* __restrict__ rowptr,
             if (take_core_bitmap(ids, w)) {
                 r.y = max(s0, ce);
                 r.w = rb;
-                words = w;
             }
         }
     }
     return true;
 }
 
-// Pass over the edges: list flag per edge, sparse edge count and merge work.
+// Pass over the entries of L: list flag and record of every entry (rec[q]
+// where flagged), sparse edge count and merge work.  Records are made here,
+// where neighbouring entries share a row's cache lines, and fetched once
+// after the sort by pivot: made in list order, each list searched a random
+// row twice (R-MAT 2^20, 12 M lists: 1666 us there; here 72 us more than the
+// flags alone, and 525 us to fetch them).
 __global__ void clip_kernel(const uint32_t* __restrict__ rowptr, const int32_t* __restrict__ col,
-                            const uint32_t* __restrict__ erow, const uint8_t* __restrict__ dense, Cnt m_,
-                            uint32_t* __restrict__ flag, unsigned long long* __restrict__ stats) {
-    const int64_t m = (int64_t)m_.get();
+                            const uint32_t* __restrict__ erow, const uint8_t* __restrict__ dense, int64_t m,
+                            const uint32_t* __restrict__ cend, const uint32_t* __restrict__ has,
+                            const uint32_t* __restrict__ rbi, uint32_t C, uint32_t* __restrict__ flag,
+                            uint4* __restrict__ rec, unsigned long long* __restrict__ stats) {
     uint64_t se = 0, sw = 0;
     GS_LOOP(q, m) {
         uint32_t f = 0;
@@ -159,8 +170,9 @@ __global__ void clip_kernel(const uint32_t* __restrict__ rowptr, const int32_t* 
             const uint32_t i = erow[q], j = (uint32_t)col[q];
             ++se;
             sw += (rowptr[i + 1] - rowptr[i]) + (rowptr[j + 1] - rowptr[j]);
-            uint32_t s0, s1;
-            f = clip(rowptr, col, i, (uint32_t)q, s0, s1);
+            uint4 r;
+            f = list_record(rowptr, col, i, (uint32_t)q, cend[i], has[i] ? rbi[i] : kNoBitmap, C, r);
+            if (f) rec[q] = r;
         }
         flag[q] = f;
     }
@@ -220,38 +232,24 @@ __global__ void core_fill_kernel(const uint32_t* __restrict__ rowptr, const int3
     }
 }
 
-// List record of every pivot-sorted list e (see the wedge kernel's
-// scan_lists), its row, and its cost (ids looked up + core words ANDed).
+// Record of every pivot-sorted list e (see the wedge kernel's scan_lists), its
+// row, and its cost (ids looked up + core words ANDed).
 __global__ void records_kernel(const uint32_t* __restrict__ rowptr, const int32_t* __restrict__ col,
-                               const uint32_t* __restrict__ erow, const uint32_t* __restrict__ val, Cnt ne_,
-                               const uint32_t* __restrict__ cend, const uint32_t* __restrict__ has,
-                               const uint32_t* __restrict__ rbi, uint32_t C, uint4* __restrict__ lst,
-                               int32_t* __restrict__ ur, uint64_t* __restrict__ cost,
+                               const uint32_t* __restrict__ erow, const uint32_t* __restrict__ key,
+                               const uint32_t* __restrict__ val, int64_t ne, const uint4* __restrict__ rec, uint32_t C,
+                               uint4* __restrict__ lst, int32_t* __restrict__ ur, uint64_t* __restrict__ cost,
                                unsigned long long* __restrict__ ncore, unsigned long long* __restrict__ nnarrow) {
-    const uint32_t ne = (uint32_t)ne_.get();
     uint64_t nc = 0, nn = 0;
     GS_LOOP(e, ne) {
-        const uint32_t q = val[e], i = erow[q], j = (uint32_t)col[q];
-        uint32_t s0 = 0, s1 = 0;
-        clip(rowptr, col, i, q, s0, s1);
+        const uint32_t q = val[e], j = key[e];
+        const uint4 r = rec[q];
         const uint32_t lo = (uint32_t)col[rowptr[j]], hi = (uint32_t)col[rowptr[j + 1] - 1];
-        const uint32_t base = lo & ~127u;
-        uint32_t sc = s0, rb = kNoBitmap, words = 0;
-        if (has[i] && base < C) {
-            const uint32_t ce = min(s1, cend[i]);
-            const uint32_t core_ids = ce > s0 ? ce - s0 : 0u;
-            const uint32_t w = core_words(lo, hi, C);
-            if (take_core_bitmap(core_ids, w)) {
-                sc = max(s0, cend[i]);
-                rb = rbi[i];
-                words = w;
-                ++nc;
-            }
-        }
-        lst[e] = make_uint4(s0, sc, s1, rb);
-        ur[e] = (int32_t)i;
-        cost[e] = (uint64_t)(s1 > sc ? s1 - sc : 0u) + words;
-        if (hi < kNarrowIds) nn += s1 > sc ? s1 - sc : 0u;
+        const uint32_t ids = r.z > r.y ? r.z - r.y : 0u;
+        lst[e] = r;
+        ur[e] = (int32_t)erow[q];
+        cost[e] = (uint64_t)ids + (r.w != kNoBitmap ? core_words(lo, hi, C) : 0u);
+        nc += r.w != kNoBitmap;
+        nn += hi < kNarrowIds ? ids : 0u;
     }
     __shared__ uint64_t lds[kT / 64];
     nc = block_sum_u64<kT>(nc, lds);
@@ -424,8 +422,7 @@ __global__ __launch_bounds__(kT) void pipe_clip_kernel(const uint32_t* __restric
             if (q >= m) continue;
             const uint32_t i = erow[q];
             uint4 r;
-            uint32_t words;
-            f[x] = list_record(rowptr, col, i, (uint32_t)q, cend[i], rbi[i], C, r, words);
+            f[x] = list_record(rowptr, col, i, (uint32_t)q, cend[i], rbi[i], C, r);
             if (f[x]) rec[q] = r;
         }
         const uint64_t tot = tile_offsets<uint32_t, PER>(f, pos, lds, u, l.t);
@@ -744,12 +741,26 @@ void plan_device(btc_plan_s* p, int64_t chunk, hipStream_t s) {
     p->info.dense_tiles = p->n_dense;
     p->info.dense_edges = (int64_t)read_dev(st.p + 0, s);
 
-    // prefix lists: flag, compact (pivot, edge), stable sort by pivot
+    // hub-core bitmaps
+    TmpBuf<uint32_t> cend, has, rbi;
+    cend.alloc((size_t)n, s);
+    has.alloc((size_t)n, s);
+    rbi.alloc((size_t)n + 1, s);
+    const uint32_t C = p->core_ids;
+    if (n) BTC_LAUNCH(core_rows_kernel, n, s, rowptr, col, n, C, cend.p, has.p);
+    exclusive_scan_u32(has.p, rbi.p, (size_t)n, s);
+
+    // prefix lists: flag and record, compact (pivot, edge), stable sort by pivot
+    TmpBuf<uint4> rec;
     TmpBuf<uint32_t> lflag, lpos;
+    rec.alloc((size_t)m, s);
     lflag.alloc((size_t)m, s);
     lpos.alloc((size_t)m + 1, s);
-    if (m) BTC_LAUNCH_RED(clip_kernel, m, s, rowptr, col, erow.p, p->n_dense ? dense.p : nullptr, m, lflag.p, st.p + 1);
+    if (m)
+        BTC_LAUNCH_CLIP(clip_kernel, m, s, rowptr, col, erow.p, p->n_dense ? dense.p : nullptr, m, cend.p, has.p, rbi.p, C,
+                        lflag.p, rec.p, st.p + 1);
     exclusive_scan_u32(lflag.p, lpos.p, (size_t)m, s);
+    const uint32_t nbm = read_dev(rbi.p + n, s);
     const uint32_t ne = read_dev(lpos.p + m, s);
     TmpBuf<uint32_t> k0, v0, k1, v1;
     k0.alloc(ne, s);
@@ -767,15 +778,6 @@ void plan_device(btc_plan_s* p, int64_t chunk, hipStream_t s) {
     off.alloc((size_t)n + 1, s);
     BTC_LAUNCH(pivot_offsets_kernel, (int64_t)n + 1, s, key, ne, n, off.p);
 
-    // hub-core bitmaps
-    TmpBuf<uint32_t> cend, has, rbi;
-    cend.alloc((size_t)n, s);
-    has.alloc((size_t)n, s);
-    rbi.alloc((size_t)n + 1, s);
-    const uint32_t C = p->core_ids;
-    if (n) BTC_LAUNCH(core_rows_kernel, n, s, rowptr, col, n, C, cend.p, has.p);
-    exclusive_scan_u32(has.p, rbi.p, (size_t)n, s);
-    const uint32_t nbm = read_dev(rbi.p + n, s);
 
     // one allocation: list records, row bitmaps, list rows; items apart
     const size_t lb = (size_t)ne * sizeof(uint4), bb = (size_t)nbm * (C / 32) * 4, rb = (size_t)ne * 4;
@@ -791,8 +793,9 @@ void plan_device(btc_plan_s* p, int64_t chunk, hipStream_t s) {
     cost.alloc(ne, s);
     P.alloc((size_t)ne + 1, s);
     if (ne)
-        BTC_LAUNCH_RED(records_kernel, ne, s, rowptr, col, erow.p, val, ne, cend.p, has.p, rbi.p, C, lst, ur, cost.p,
-                   st.p + 3, st.p + 6);
+        BTC_LAUNCH_CLIP(records_kernel, ne, s, rowptr, col, erow.p, key, val, (int64_t)ne, rec.p, C, lst, ur, cost.p,
+                        st.p + 3, st.p + 6);
+    rec.release();
     exclusive_scan_u64(cost.p, P.p, ne, s);
     erow.release();
 
