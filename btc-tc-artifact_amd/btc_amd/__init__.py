@@ -333,7 +333,7 @@ class Graph:
 def _count_out(n, per_vertex, wide=False):
     total = C.c_uint64(0)
     ms = C.c_float(0)
-    pv = np.zeros(n, np.int64 if wide else np.int32) if per_vertex else None
+    pv = np.empty(n, np.int64 if wide else np.int32) if per_vertex else None
     return total, ms, pv
 
 

@@ -421,7 +421,13 @@ void PvBuf::copy_out(int32_t* h32, int64_t* h64, hipStream_t s) const {
         BTC_HIP(hipMemcpyAsync(pin, d, bytes(), hipMemcpyDeviceToHost, s));
         BTC_HIP(hipStreamSynchronize(s));
         if (wide() == (h64 != nullptr)) {
-            std::memcpy(h64 ? (void*)h64 : (void*)h32, pin, bytes());
+            char* const out = h64 ? reinterpret_cast<char*>(h64) : reinterpret_cast<char*>(h32);
+            const size_t total = bytes(), parts = std::max<size_t>(1, std::min<size_t>(8, total >> 17));
+#pragma omp parallel for num_threads((int)parts) if (parts > 1) schedule(static)
+            for (size_t t = 0; t < parts; ++t) {
+                const size_t a = total * t / parts, z = total * (t + 1) / parts;
+                std::memcpy(out + a, pin + a, z - a);
+            }
         } else if (h64) {
             const int32_t* t = reinterpret_cast<const int32_t*>(pin);
             for (size_t v = 0; v < n; ++v) h64[v] = t[v];
