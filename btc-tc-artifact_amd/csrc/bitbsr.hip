@@ -223,10 +223,13 @@ struct RowBits<128> {
     }
 };
 
-// FILL = false: counts[I] = number of tiles of row block I.
+// FILL = false: counts[I] = number of tiles of row block I; with `needed`,
+// the row blocks that counting the dense tiles (more than tau bits) reads are
+// marked: a dense tile's own and those of its columns.
 // FILL = true: writes tile I's indices / row_indices / bits at offs[I] and,
 // with pop, every tile's set bits (pop) and, beside each entry of L, those
-// of its tile (epop); *max_pop becomes the largest of them.
+// of its tile (epop); *max_pop becomes the largest of them.  With `needed`
+// only the marked row blocks are written.
 template <int K, bool FILL>
 __global__ __launch_bounds__(256) void build_kernel(int n, int n_rb, const uint32_t* __restrict__ rowptr,
                                                      const int32_t* __restrict__ col,
@@ -235,11 +238,12 @@ __global__ __launch_bounds__(256) void build_kernel(int n, int n_rb, const uint3
                                                      uint32_t* __restrict__ indices,
                                                      uint32_t* __restrict__ row_indices,
                                                      uint64_t* __restrict__ tiles, uint32_t* __restrict__ pop,
-                                                     uint16_t* __restrict__ epop, uint32_t* __restrict__ max_pop) {
+                                                     uint16_t* __restrict__ epop, uint32_t* __restrict__ max_pop,
+                                                     uint32_t* __restrict__ needed, int tau) {
     const int lane = threadIdx.x & 63;
     const int r = lane & 15;
     const int64_t I = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * 4 + (lane >> 4);
-    const bool valid = I < n_rb;
+    const bool valid = I < n_rb && (!FILL || !needed || needed[I]);
     const int64_t row = I * 16 + r;
     uint32_t p = 0, e = 0;
     if (valid && row < n) {
@@ -293,6 +297,16 @@ __global__ __launch_bounds__(256) void build_kernel(int n, int n_rb, const uint3
                 }
                 ++t;
             }
+            if (!FILL && needed) {
+                uint32_t c = p - p0;
+#pragma unroll
+                for (int o = 8; o > 0; o >>= 1) c += (uint32_t)__shfl_xor((int)c, o, 16);
+                if (c > (uint32_t)tau) {
+                    const int64_t rb = (int64_t)cur * (K / 16) + r;
+                    if (r < K / 16 && rb < n_rb) needed[rb] = 1;
+                    if (r == 0) needed[I] = 1;
+                }
+            }
             ++cnt;
         }
     }
@@ -309,8 +323,14 @@ __global__ void narrow_u64_to_u32(const uint64_t* __restrict__ in, uint32_t* __r
     if (i < n) out[i] = (uint32_t)in[i];
 }
 
+// counts[I] = 0 for the row blocks that are not marked
+__global__ void drop_counts_kernel(uint32_t* __restrict__ counts, const uint32_t* __restrict__ needed, size_t n) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n && !needed[i]) counts[i] = 0;
+}
+
 template <int K>
-void build_impl(btc_graph_s* g, hipStream_t s, btc_bitbsr_s* b, bool counted) {
+void build_impl(btc_graph_s* g, hipStream_t s, btc_bitbsr_s* b, bool counted, int dense_tau) {
     const int n = g->n;
     const int n_rb = (n + 15) / 16;
     b->n = n;
@@ -323,10 +343,21 @@ void build_impl(btc_graph_s* g, hipStream_t s, btc_bitbsr_s* b, bool counted) {
     TmpBuf<uint64_t> offs;
     counts.alloc((size_t)n_rb, s);
     offs.alloc((size_t)n_rb + 1, s);
+    TmpBuf<uint32_t> needed;
+    if (dense_tau >= 0) {
+        needed.alloc((size_t)n_rb, s);
+        BTC_HIP(hipMemsetAsync(needed.p, 0, (size_t)n_rb * 4, s));
+    }
     if (grid) {
         hipLaunchKernelGGL((build_kernel<K, false>), dim3(grid), dim3(256), 0, s, n, n_rb, g->d_rowptr.p,
-                           g->d_col.p, counts.p, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
+                           g->d_col.p, counts.p, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, needed.p,
+                           dense_tau);
         BTC_CHECK_LAUNCH("build_kernel<count>");
+        if (needed.p) {
+            hipLaunchKernelGGL(drop_counts_kernel, dim3((unsigned)((n_rb + 255) / 256)), dim3(256), 0, s, counts.p,
+                               needed.p, (size_t)n_rb);
+            BTC_CHECK_LAUNCH("drop_counts_kernel");
+        }
     }
     scan_u32_to_u64(counts.p, offs.p, (size_t)n_rb, s);
     uint64_t nblk = 0;
@@ -350,7 +381,8 @@ void build_impl(btc_graph_s* g, hipStream_t s, btc_bitbsr_s* b, bool counted) {
     if (grid && nblk) {
         hipLaunchKernelGGL((build_kernel<K, true>), dim3(grid), dim3(256), 0, s, n, n_rb, g->d_rowptr.p,
                            g->d_col.p, nullptr, offs.p, b->indices.p, b->row_indices.p, b->tiles.p,
-                           counted ? b->pop.p : nullptr, b->rows.epop, counted ? b->rows.d_count + 3 : nullptr);
+                           counted ? b->pop.p : nullptr, b->rows.epop, counted ? b->rows.d_count + 3 : nullptr,
+                           needed.p, dense_tau);
         BTC_CHECK_LAUNCH("build_kernel<fill>");
     }
     if (counted) {
@@ -1035,12 +1067,12 @@ constexpr uint32_t kMaxTilesPerLaunch = 1u << 24;
 
 }  // namespace
 
-void bitbsr_build(btc_graph_s* g, int K, hipStream_t s, btc_bitbsr_s* b, bool counted) {
+void bitbsr_build(btc_graph_s* g, int K, hipStream_t s, btc_bitbsr_s* b, bool counted, int dense_tau) {
     ensure_device(g, s);
     switch (K) {
-        case 32: build_impl<32>(g, s, b, counted); break;
-        case 64: build_impl<64>(g, s, b, counted); break;
-        case 128: build_impl<128>(g, s, b, counted); break;
+        case 32: build_impl<32>(g, s, b, counted, dense_tau); break;
+        case 64: build_impl<64>(g, s, b, counted, dense_tau); break;
+        case 128: build_impl<128>(g, s, b, counted, dense_tau); break;
         default: fail(BTC_ERR_ARG, "tile width K = %d (expected 32, 64 or 128)", K);
     }
 }

@@ -698,8 +698,8 @@ void canonicalise_device(const int32_t* src, const int32_t* dst, int64_t nnz, in
                                (size_t)nc);
             BTC_CHECK_LAUNCH("degree_kernel");
         }
-        BTC_LAUNCH(rank_keys_kernel, nc, s, deg.p, (size_t)nc, nc, 0xFFFFFFFFu, k0.p, v0.p);
-        bool alt = sort_pairs_u32(k0.p, v0.p, k1.p, v1.p, (size_t)nc, 32, s);
+        BTC_LAUNCH(rank_keys_kernel, nc, s, deg.p, (size_t)nc, nc, (uint32_t)nc, k0.p, v0.p);  // degrees are below nc
+        bool alt = sort_pairs_u32(k0.p, v0.p, k1.p, v1.p, (size_t)nc, id_bits((int64_t)nc + 1), s);
         if (segs) {
             // then a stable sort by segment: (segment, -degree, id)
             uint32_t* ord = alt ? v1.p : v0.p;

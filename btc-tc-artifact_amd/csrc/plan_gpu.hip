@@ -112,8 +112,8 @@ __global__ void dense_edges_kernel(const int32_t* __restrict__ col, const uint32
                                    const uint32_t* __restrict__ pop, int tau, uint8_t* __restrict__ dense) {
     GS_LOOP(e, m) {
         const uint32_t I = erow[e] / 16, jc = (uint32_t)col[e] / (uint32_t)K;
-        const uint32_t t = lower_bound_dev(indices, indptr[I], indptr[I + 1], jc);
-        dense[e] = (int)pop[t] > tau;
+        const uint32_t t0 = indptr[I], t1 = indptr[I + 1];  // no tiles: no dense tile in the row block
+        dense[e] = t0 != t1 && (int)pop[lower_bound_dev(indices, t0, t1, jc)] > tau;
     }
 }
 
@@ -215,19 +215,40 @@ __global__ void core_rows_kernel(const uint32_t* __restrict__ rowptr, const int3
     }
 }
 
-__global__ void core_fill_kernel(const uint32_t* __restrict__ rowptr, const int32_t* __restrict__ col,
-                                 const uint32_t* __restrict__ cend, const uint32_t* __restrict__ has,
-                                 const uint32_t* __restrict__ rbi, Cnt n_, uint32_t CW,
-                                 uint32_t* __restrict__ rowbits) {
-    const int64_t n = (int64_t)n_.get();
-    const int64_t waves = ((int64_t)gridDim.x * kT) >> 6;
-    const int lane = threadIdx.x & 63;
+// Core bitmaps, a wave per row that has one: lane w % 64 owns word w, taken
+// 64 words (2048 ids) at a time from the row's ids below C, so a bitmap is
+// cleared, set and written in one pass without atomics.
+// (R-MAT 2^20: 95 us; with a memset and an atomic per id 164 us and the memset).
+// has (NULL: rbi says it, kNoBitmap) = the row has a bitmap.
+__global__ __launch_bounds__(kT) void core_fill_kernel(const uint32_t* __restrict__ rowptr,
+                                                       const int32_t* __restrict__ col,
+                                                       const uint32_t* __restrict__ cend,
+                                                       const uint32_t* __restrict__ has,
+                                                       const uint32_t* __restrict__ rbi, Cnt n_, uint32_t C,
+                                                       uint32_t* __restrict__ rowbits) {
+    const int64_t n = n_.get(), waves = ((int64_t)gridDim.x * kT) >> 6;
+    const uint32_t lane = threadIdx.x & 63, CW = C / 32;
     for (int64_t i = (blockIdx.x * (int64_t)kT + threadIdx.x) >> 6; i < n; i += waves) {
-        if (!has[i]) continue;
+        if (has ? !has[i] : rbi[i] == kNoBitmap) continue;
         uint32_t* b = rowbits + (size_t)rbi[i] * CW;
-        for (uint32_t p = rowptr[i] + lane; p < cend[i]; p += 64) {
-            const uint32_t k = (uint32_t)col[p];
-            atomicOr(&b[k >> 5], 1u << (k & 31u));
+        const uint32_t p1 = cend[i];
+        uint32_t p = rowptr[i];
+        for (uint32_t w0 = 0; w0 < CW; w0 += 64) {
+            uint32_t word = 0;
+            // ids of this span, 64 at a time, each lane picking its word's
+            while (p < p1) {
+                const uint32_t at = p + lane;
+                const uint32_t id = at < p1 ? (uint32_t)col[at] : 0xFFFFFFFFu;
+                const uint64_t in = __ballot(id < (w0 + 64) * 32);
+                const int cnt = __popcll(in);
+                for (int k = 0; k < cnt; ++k) {
+                    const uint32_t kid = (uint32_t)__builtin_amdgcn_readlane((int)id, k);
+                    word |= (kid >> 5) - w0 == lane ? 1u << (kid & 31u) : 0u;
+                }
+                p += (uint32_t)cnt;
+                if (cnt < 64) break;
+            }
+            if (w0 + lane < CW) b[w0 + lane] = word;
         }
     }
 }
@@ -497,43 +518,6 @@ __global__ __launch_bounds__(kT) void pipe_lists_kernel(const uint32_t* __restri
     }
 }
 
-// Core bitmaps, a wave per row that has one: lane w % 64 owns word w, taken
-// 64 words (2048 ids) at a time from the row's ids below C, so a bitmap is
-// cleared, set and written in one pass without atomics.
-__global__ __launch_bounds__(kT) void pipe_core_fill_kernel(const uint32_t* __restrict__ rowptr,
-                                                            const int32_t* __restrict__ col,
-                                                            const uint32_t* __restrict__ cend,
-                                                            const uint32_t* __restrict__ rbi, uint32_t C,
-                                                            const PipeCtl* __restrict__ c,
-                                                            uint32_t* __restrict__ rowbits) {
-    if (c->nbm == 0) return;
-    const int64_t n = c->nc, waves = ((int64_t)gridDim.x * kT) >> 6;
-    const uint32_t lane = threadIdx.x & 63, CW = C / 32;
-    for (int64_t i = (blockIdx.x * (int64_t)kT + threadIdx.x) >> 6; i < n; i += waves) {
-        if (rbi[i] == kNoBitmap) continue;
-        uint32_t* b = rowbits + (size_t)rbi[i] * CW;
-        const uint32_t p1 = cend[i];
-        uint32_t p = rowptr[i];
-        for (uint32_t w0 = 0; w0 < CW; w0 += 64) {
-            uint32_t word = 0;
-            // ids of this span, 64 at a time, each lane picking its word's
-            while (p < p1) {
-                const uint32_t at = p + lane;
-                const uint32_t id = at < p1 ? (uint32_t)col[at] : 0xFFFFFFFFu;
-                const uint64_t in = __ballot(id < (w0 + 64) * 32);
-                const int cnt = __popcll(in);
-                for (int k = 0; k < cnt; ++k) {
-                    const uint32_t kid = (uint32_t)__builtin_amdgcn_readlane((int)id, k);
-                    word |= (kid >> 5) - w0 == lane ? 1u << (kid & 31u) : 0u;
-                }
-                p += (uint32_t)cnt;
-                if (cnt < 64) break;
-            }
-            if (w0 + lane < CW) b[w0 + lane] = word;
-        }
-    }
-}
-
 // List e opens a work item: the pivot's first list, or (pivots of more than
 // a wave's worth) where the running cost crosses a multiple of the cut, about
 // target_items items in all and at least 8192 checks each.  first[k] = the
@@ -718,7 +702,7 @@ void plan_device(btc_plan_s* p, int64_t chunk, hipStream_t s) {
     TmpBuf<uint8_t> dense;
     p->n_dense = 0;
     if (p->tau < 16 * p->K && m > 0) {
-        const btc_bitbsr_s* b = plan_bsr(p, s);
+        const btc_bitbsr_s* b = plan_bsr(p, s, true);
         TmpBuf<uint32_t> pop, flag, pos;
         pop.alloc(b->nblk, s);
         flag.alloc(b->nblk, s);
@@ -786,8 +770,7 @@ void plan_device(btc_plan_s* p, int64_t chunk, hipStream_t s) {
     uint32_t* rowbits = reinterpret_cast<uint32_t*>(p->lists.p + lb);
     int32_t* ur = reinterpret_cast<int32_t*>(p->lists.p + lb + bb);
     if (bb) {
-        BTC_HIP(hipMemsetAsync(rowbits, 0, bb, s));
-        BTC_LAUNCH(core_fill_kernel, (int64_t)n * 64, s, rowptr, col, cend.p, has.p, rbi.p, n, C / 32, rowbits);
+        BTC_LAUNCH(core_fill_kernel, (int64_t)n * 64, s, rowptr, col, cend.p, has.p, rbi.p, n, C, rowbits);
     }
     TmpBuf<uint64_t> cost, P;
     cost.alloc(ne, s);
@@ -874,11 +857,12 @@ unsigned cap_grid(int64_t cap) {
 
 void plan_capacity(const PlanCap& c, hipStream_t s) {
     PipeCtl* ctl = c.ctl;
+    const Cnt nc = Cnt::dev(&ctl->nc);
     const int64_t M = c.m_cap, N = c.n_cap, I = (int64_t)c.items_cap;
     const uint32_t C = c.core_ids;
     const SortUse su = dseq_sort(*c.seq, id_bits(c.n_cap));
     CAP_LAUNCH(pipe_rows_kernel, N, s, c.rowptr, c.col, ctl, C, c.cend, c.rbi);
-    if (C) CAP_LAUNCH(pipe_core_fill_kernel, N * 64, s, c.rowptr, c.col, c.cend, c.rbi, C, ctl, c.rowbits);
+    if (C) CAP_LAUNCH(core_fill_kernel, N * 64, s, c.rowptr, c.col, c.cend, nullptr, c.rbi, nc, C, c.rowbits);
     with_tile_per(M, [&](auto per) {
         constexpr int PER = decltype(per)::value;
         // prefix lists: records by entry, (pivot, entry) pairs, stably sorted by pivot
