@@ -8,7 +8,7 @@
 // (devtile.h); each pass kernel then ranks a tile stably in LDS (rocPRIM's
 // block_radix_rank, match form: per-wave ballots of equal digits) and finds
 // the tile's offset for each digit by decoupled look-back.  A pass of 131 K
-// u64 keys takes 10 us and one of 3.3 M 59 us (11 and 75 with two tickets a
+// u64 keys takes 10 us and one of 3.3 M 41 us (11 and 75 with two tickets a
 // workgroup, a finish counter and a histogram kernel's own read of the keys):
 // tickets and look-back round trips, not the 53 MB moved, bound the latter.
 #include <rocprim/block/block_radix_rank.hpp>
@@ -20,7 +20,6 @@ namespace btcx {
 namespace {
 
 constexpr int kT = kTileThreads;
-constexpr int kSortPer = (int)kSortTile / kT;
 
 size_t tiles(size_t cap, size_t tile) { return std::max<size_t>(1, (cap + tile - 1) / tile); }
 
@@ -85,10 +84,11 @@ __device__ __forceinline__ uint64_t look_back(const uint64_t* cells, int64_t j0,
 // order; padding keys (all bits set) rank after every real key of the tile.
 // Every look-back ends: a ticket is only taken by a running workgroup,
 // which publishes before it waits on anything.
-template <class K, bool V>
+template <class K, bool V, int kSortPer>
 __global__ __launch_bounds__(kT) void dsort_onesweep(const K* __restrict__ kin, const uint32_t* __restrict__ vin,
                                                      K* __restrict__ kout, uint32_t* __restrict__ vout,
                                                      const uint32_t* __restrict__ d_n, int pass, SortUse u) {
+    constexpr uint32_t kSortTile = kT * kSortPer;
     using Rank = rocprim::block_radix_rank<kT, kDigitBits, rocprim::block_radix_rank_algorithm::match>;
     static_assert(Rank::digits_per_thread == 1, "one digit per thread");
     __shared__ typename Rank::storage_type rank_lds;
@@ -149,13 +149,16 @@ __global__ __launch_bounds__(kT) void dsort_onesweep(const K* __restrict__ kin, 
 template <class K, bool V>
 bool dsort_t(K* keys, uint32_t* vals, K* kt, uint32_t* vt, size_t cap, const uint32_t* d_n, const SortUse& u,
              hipStream_t s) {
-    const unsigned g = (unsigned)std::min<size_t>(tiles(cap, kSortTile), 2048);  // tiles go by ticket
+    const unsigned g = (unsigned)std::min<size_t>(tiles(cap, u.tile), 2048);  // tiles go by ticket
     K* ki = keys;
     K* ko = kt;
     uint32_t* vi = vals;
     uint32_t* vo = vt;
     for (int p = 0; p < u.passes; ++p) {
-        hipLaunchKernelGGL((dsort_onesweep<K, V>), dim3(g), dim3(kT), 0, s, ki, vi, ko, vo, d_n, p, u);
+        if (u.tile == kSortTileMin)
+            hipLaunchKernelGGL((dsort_onesweep<K, V, kSortTileMin / kT>), dim3(g), dim3(kT), 0, s, ki, vi, ko, vo, d_n, p, u);
+        else
+            hipLaunchKernelGGL((dsort_onesweep<K, V, kSortTileMax / kT>), dim3(g), dim3(kT), 0, s, ki, vi, ko, vo, d_n, p, u);
         BTC_CHECK_LAUNCH("dsort_onesweep");
         std::swap(ki, ko);
         std::swap(vi, vo);
@@ -168,7 +171,7 @@ bool dsort_t(K* keys, uint32_t* vals, K* kt, uint32_t* vt, size_t cap, const uin
 size_t dseq_clear_words(size_t cap) { return kCtlWords + kMaxSorts * kTotalsWords + kMaxScans * scan_words(cap); }
 
 size_t dseq_bytes(size_t cap) {
-    return dseq_clear_words(cap) * 4 + (size_t)kMaxPasses * tiles(cap, kSortTile) * kDigits * 8;
+    return dseq_clear_words(cap) * 4 + (size_t)kMaxPasses * tiles(cap, sort_tile(cap)) * kDigits * 8;
 }
 
 SortUse dseq_sort(DevSeq& q, int end_bit) {
@@ -180,9 +183,10 @@ SortUse dseq_sort(DevSeq& q, int end_bit) {
     return SortUse{w + kSortTickets + 16 * k,
                    w + kCtlWords + (size_t)k * kTotalsWords,
                    reinterpret_cast<uint64_t*>(w + dseq_clear_words(q.cap)),
-                   tiles(q.cap, kSortTile) * kDigits,
+                   tiles(q.cap, sort_tile(q.cap)) * kDigits,
                    w + kSeqErr,
-                   passes};
+                   passes,
+                   sort_tile(q.cap)};
 }
 
 ScanUse dseq_scan(DevSeq& q) {

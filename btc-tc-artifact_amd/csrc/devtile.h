@@ -175,6 +175,7 @@ struct SortUse {
     size_t status_pass;
     uint32_t* err;
     int passes;
+    uint32_t tile;       // keys per tile
 };
 
 typedef uint32_t DigitHist[kMaxPasses][kDigits];  // __shared__
@@ -199,7 +200,7 @@ __device__ __forceinline__ void hist_flush(DigitHist& h, const SortUse& u) {
 
 // Clears the statuses of the tiles of n keys (the grid shares them).
 __device__ __forceinline__ void sort_status_clear(const SortUse& u, uint64_t n) {
-    const uint64_t words = (n + kSortTile - 1) / kSortTile * kDigits;
+    const uint64_t words = (n + u.tile - 1) / u.tile * kDigits;
     for (int p = 0; p < u.passes; ++p)
         for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < words;
              i += (uint64_t)gridDim.x * blockDim.x)

@@ -11,6 +11,8 @@
 // those of the reference's preprocess_for_triangle_counting
 // (btc/operations/convert.h:601-692) followed by planning and counting; the
 // reference runs them from the host for every graph.
+#include <omp.h>
+
 #include <algorithm>
 #include <cstring>
 #include <mutex>
@@ -233,7 +235,7 @@ __global__ __launch_bounds__(kT) void group_pairs_kernel(int32_t* __restrict__ s
 // engine drains what came before.
 void upload_pairs(btc_pipeline_s* p, char* pin, int32_t count, const int32_t* const* src, const int32_t* const* dst,
                   const int64_t* sizes, int64_t pairs, hipStream_t s) {
-    constexpr int64_t kPiece = int64_t(1) << 16, kRound = int64_t(1) << 20;  // ids
+    constexpr int64_t kPiece = int64_t(1) << 14, kRound = int64_t(1) << 20;  // ids
     int32_t* const stage = reinterpret_cast<int32_t*>(pin + kPinHeader);
     struct Piece {
         const int32_t* from;
@@ -249,19 +251,21 @@ void upload_pairs(btc_pipeline_s* p, char* pin, int32_t count, const int32_t* co
             at += sizes[g];
         }
     }
-    // each round goes out as one copy, cut where the destination array does
-    size_t k = 0;
-    while (k < pieces.size()) {
-        const int64_t from = pieces[k].to, end = from < pairs ? pairs : 2 * pairs;
+    // a round is staged together (threads pay from a quarter of a MiB on) and
+    // goes out as one copy per destination array
+    for (size_t k = 0; k < pieces.size();) {
         size_t z = k;
         int64_t n = 0;
-        while (z < pieces.size() && pieces[z].to < end && n < kRound) n += pieces[z++].n;
-        const int64_t team = n >> 17;  // threads pay from half a MiB on
-#pragma omp parallel for schedule(dynamic, 1) if (team > 1)
+        while (z < pieces.size() && n < kRound) n += pieces[z++].n;
+        const int team = (int)std::min<int64_t>(omp_get_max_threads(), n >> 15);
+#pragma omp parallel for schedule(static) num_threads(team) if (team > 1)
         for (size_t x = k; x < z; ++x)
             std::memcpy(stage + pieces[x].to, pieces[x].from, (size_t)pieces[x].n * 4);
-        int32_t* const to = from < pairs ? p->src + from : p->dst + (from - pairs);
-        BTC_HIP(hipMemcpyAsync(to, stage + from, (size_t)n * 4, hipMemcpyHostToDevice, s));
+        const int64_t from = pieces[k].to, end = from + n, cut = std::max(from, std::min(end, pairs));
+        if (from < cut)
+            BTC_HIP(hipMemcpyAsync(p->src + from, stage + from, (size_t)(cut - from) * 4, hipMemcpyHostToDevice, s));
+        if (cut < end)
+            BTC_HIP(hipMemcpyAsync(p->dst + (cut - pairs), stage + cut, (size_t)(end - cut) * 4, hipMemcpyHostToDevice, s));
         k = z;
     }
 }

@@ -36,7 +36,12 @@ void exclusive_scan_u64(const uint64_t* in, uint64_t* out, size_t n, hipStream_t
 // own, all of them in the words [0, dseq_clear_words) that the run's first
 // kernel clears (but for word kSeqErr, which stays).  A sort's statuses are
 // shared by all and cleared by the kernel that writes its keys.
-constexpr uint32_t kSortTile = 2048;  // keys of a sort's tile
+// Keys of a sort's tile, by capacity: large inputs pay for tickets and
+// look-back per tile, small ones for CUs without a tile (replays of one graph
+// of 131 K / 524 K / 1.6 M pairs with tiles of 2048 against 4096: 258 / 408 /
+// 964 us against 282 / 413 / 880, a group of 3.3 M 1914 against 1678).
+constexpr uint32_t kSortTileMin = 2048, kSortTileMax = 4096;
+inline uint32_t sort_tile(size_t cap) { return cap > (size_t(1) << 20) ? kSortTileMax : kSortTileMin; }
 constexpr int kMaxSorts = 6, kMaxScans = 8;
 constexpr uint32_t kSeqErr = 0;
 struct SortUse;

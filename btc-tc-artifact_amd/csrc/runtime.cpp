@@ -1,5 +1,7 @@
 // Error state, version, device selection, event timing and the scalar
 // dispatch rules shared by every path.
+#include <omp.h>
+
 #include <algorithm>
 #include <cstdarg>
 #include <chrono>
@@ -422,7 +424,7 @@ void PvBuf::copy_out(int32_t* h32, int64_t* h64, hipStream_t s) const {
         BTC_HIP(hipStreamSynchronize(s));
         if (wide() == (h64 != nullptr)) {
             char* const out = h64 ? reinterpret_cast<char*>(h64) : reinterpret_cast<char*>(h32);
-            const size_t total = bytes(), parts = std::max<size_t>(1, std::min<size_t>(8, total >> 17));
+            const size_t total = bytes(), parts = std::min<size_t>((size_t)omp_get_max_threads(), std::max<size_t>(1, std::min<size_t>(8, total >> 17)));
 #pragma omp parallel for num_threads((int)parts) if (parts > 1) schedule(static)
             for (size_t t = 0; t < parts; ++t) {
                 const size_t a = total * t / parts, z = total * (t + 1) / parts;
