@@ -289,13 +289,8 @@ __device__ __forceinline__ bool pivot_small(const uint32_t* __restrict__ rowptr,
 // pivots) the running cost crosses a multiple of chunk.
 __global__ void item_start_kernel(const uint32_t* __restrict__ rowptr, const int32_t* __restrict__ col,
                                   const uint32_t* __restrict__ key, const uint32_t* __restrict__ off,
-                                  const uint64_t* __restrict__ P, Cnt ne_, uint64_t chunk_,
-                                  const unsigned long long* __restrict__ d_checks, uint64_t target_items,
+                                  const uint64_t* __restrict__ P, int64_t ne, uint64_t chunk,
                                   uint32_t* __restrict__ start) {
-    const uint32_t ne = (uint32_t)ne_.get();
-    // with d_checks: about target_items items, at least 8192 checks each
-    const uint64_t chunk =
-        d_checks ? max((uint64_t)8192, ((uint64_t)*d_checks + target_items - 1) / target_items) : chunk_;
     GS_LOOP(e, ne) {
         const uint32_t j = key[e], eb = off[j];
         uint32_t st = e == eb;
@@ -309,7 +304,7 @@ __global__ void item_start_kernel(const uint32_t* __restrict__ rowptr, const int
 __global__ void items_kernel(const uint32_t* __restrict__ rowptr, const int32_t* __restrict__ col,
                              const uint32_t* __restrict__ key, const uint32_t* __restrict__ off,
                              const uint64_t* __restrict__ P, const uint32_t* __restrict__ first, Cnt nitems_,
-                             Cnt ne_, bool use_tiny, bool tiny_all, bool coarse, uint4* __restrict__ tmp_items,
+                             Cnt ne_, bool use_tiny, bool tiny_all, uint4* __restrict__ tmp_items,
                              uint32_t* __restrict__ skey, uint32_t* __restrict__ sval,
                              unsigned long long* __restrict__ stats) {
     const uint32_t nitems = (uint32_t)nitems_.get();
@@ -327,15 +322,8 @@ __global__ void items_kernel(const uint32_t* __restrict__ rowptr, const int32_t*
         tmp_items[2 * k] = make_uint4(t0, t1, eb, ee);
         tmp_items[2 * k + 1] = make_uint4(lo, hi, w32, 0u);
         const uint32_t cls = tiny ? 2u : small ? 1u : 0u;
-        if (coarse) {
-            // 8-bit key: class, then work by half octaves, heaviest first
-            const uint32_t len = w ? 64 - __clzll(w) : 0u;
-            const uint32_t half = len >= 2 ? (uint32_t)(w >> (len - 2)) & 1u : 0u;
-            skey[k] = (cls << 6) | (63u - min(63u, 2 * len + half));
-        } else {
-            const uint32_t w30 = (uint32_t)min(w, (uint64_t)0x3FFFFFFFu);
-            skey[k] = (cls << 30) | (0x3FFFFFFFu - w30);
-        }
+        const uint32_t w30 = (uint32_t)min(w, (uint64_t)0x3FFFFFFFu);
+        skey[k] = (cls << 30) | (0x3FFFFFFFu - w30);
         sval[k] = (uint32_t)k;
         words += t1 - t0;
         small_items += small;
@@ -352,19 +340,8 @@ __global__ void items_kernel(const uint32_t* __restrict__ rowptr, const int32_t*
     }
 }
 
-// With c set (a capacity plan), workgroup 0 also records the item counts of
-// the wedge kernel's launch (wave items, st[5], follow the workgroup items;
-// there are no tiny items) and clears the count's total and cursors.
 __global__ void place_items_kernel(const uint4* __restrict__ tmp_items, const uint32_t* __restrict__ order,
-                                   Cnt nitems_, uint4* __restrict__ items, PipeCtl* __restrict__ c,
-                                   unsigned long long* __restrict__ work) {
-    const uint32_t nitems = (uint32_t)nitems_.get();
-    if (c && blockIdx.x == 0 && threadIdx.x == 0) {
-        c->item_counts[0] = c->nitems - (uint32_t)c->st[5];
-        c->item_counts[1] = c->nitems;
-        work[0] = 0;
-        work[1] = 0;
-    }
+                                   int64_t nitems, uint4* __restrict__ items) {
     GS_LOOP(r, nitems) {
         const uint32_t k = order[r];
         items[2 * r] = tmp_items[2 * k];
@@ -786,8 +763,7 @@ void plan_device(btc_plan_s* p, int64_t chunk, hipStream_t s) {
     TmpBuf<uint32_t> start, spos;
     start.alloc(ne, s);
     spos.alloc((size_t)ne + 1, s);
-    if (ne) BTC_LAUNCH(item_start_kernel, ne, s, rowptr, col, key, off.p, P.p, ne, (uint64_t)chunk, nullptr, (uint64_t)1,
-                       start.p);
+    if (ne) BTC_LAUNCH(item_start_kernel, ne, s, rowptr, col, key, off.p, P.p, (int64_t)ne, (uint64_t)chunk, start.p);
     exclusive_scan_u32(start.p, spos.p, ne, s);
     const uint32_t nitems = read_dev(spos.p + ne, s);
     TmpBuf<uint32_t> first, sk0, sv0, sk1, sv1;
@@ -801,12 +777,11 @@ void plan_device(btc_plan_s* p, int64_t chunk, hipStream_t s) {
     sv1.alloc(nitems, s);
     if (nitems)
         BTC_LAUNCH_RED(items_kernel, nitems, s, rowptr, col, key, off.p, P.p, first.p, nitems, ne,
-                   p->use_tiny, p->tiny_all, false, tmp.p, sk0.p, sv0.p, st.p + 4);
+                   p->use_tiny, p->tiny_all, tmp.p, sk0.p, sv0.p, st.p + 4);
     const bool ialt = sort_pairs_u32(sk0.p, sv0.p, sk1.p, sv1.p, nitems, 32, s);
     p->items_dev.alloc_on((size_t)nitems * 2, s);
     if (nitems)
-        BTC_LAUNCH(place_items_kernel, nitems, s, tmp.p, ialt ? sv1.p : sv0.p, nitems, p->items_dev.p, nullptr,
-                   nullptr);
+        BTC_LAUNCH(place_items_kernel, nitems, s, tmp.p, ialt ? sv1.p : sv0.p, nitems, p->items_dev.p);
 
     // st: [0] dense edges, [1] sparse edges, [2] their merge work, [3] core
     // lists, [4] pivot row words over items, [5] wave items (tiny ones
