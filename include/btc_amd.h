@@ -376,8 +376,8 @@ void btc_batch_free(btc_batch b);
  * nnz_cap pairs, then replayed for each input with one hipGraphLaunch:
  * every kernel reads the live sizes (pairs, nnz(L), vertices, lists, work
  * items) from device memory, so a run makes no allocation and no host
- * round trip between its steps.  Buffers (about 180 bytes per pair and
- * 60 per id of capacity) are allocated once, at creation.  The plan has no
+ * round trip between its steps.  Buffers (about 135 bytes per pair and
+ * 90 per id of capacity) are allocated once, at creation.  The plan has no
  * dense tiles and no tiny items (the wedge kernel counts every edge), cut
  * into about 64 work items per CU; of opts, group_lanes, unroll, lookup,
  * schedule, waves_per_eu, core_ids and wide_offsets apply.  Counts equal
