@@ -261,24 +261,28 @@ void pool_free(void* p, bool ordered, hipStream_t s) {
     if (std::uncaught_exceptions() > 0) ordered = false;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) dev = 0;
-    std::vector<void*> old;
-    for (int k = 0; k < kPoolDevices; ++k) {
-        Pool& q = g_pools[(dev + k) % kPoolDevices];  // the current device's almost always
-        std::lock_guard<std::mutex> lk(q.mu);
-        const auto it = q.live.find(p);
-        if (it == q.live.end()) continue;
-        const size_t bytes = it->second;
-        q.live.erase(it);
-        if (bytes > kPoolKeep / 4) {  // one block does not crowd out the rest
-            old.push_back(p);
-        } else {
-            q.cached.push_back({p, bytes, s, ordered, ++q.releases, std::chrono::steady_clock::now()});
-            q.cached_bytes += bytes;
-            old = pool_trim(q, kPoolKeep);
+    bool kept = false;
+    try {  // called by destructors: no exception leaves
+        std::vector<void*> old;
+        for (int k = 0; k < kPoolDevices; ++k) {
+            Pool& q = g_pools[(dev + k) % kPoolDevices];  // the current device's almost always
+            std::lock_guard<std::mutex> lk(q.mu);
+            const auto it = q.live.find(p);
+            if (it == q.live.end()) continue;
+            const size_t bytes = it->second;
+            q.live.erase(it);
+            if (bytes <= kPoolKeep / 4) {  // one block does not crowd out the rest
+                q.cached.push_back({p, bytes, s, ordered, ++q.releases, std::chrono::steady_clock::now()});
+                kept = true;
+                q.cached_bytes += bytes;
+                old = pool_trim(q, kPoolKeep);
+            }
+            break;
         }
-        break;
+        give_back(old);
+    } catch (...) {
     }
-    give_back(old);
+    if (!kept) (void)hipFree(p);
 }
 
 void mem_pool_init() {
