@@ -3,6 +3,7 @@
 #include <omp.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdarg>
 #include <chrono>
 #include <cstring>
@@ -94,15 +95,34 @@ namespace {
 
 constexpr int kPoolDevices = 64;
 
+// The queue of work that a use is in order on.  A handle names one, except
+// hipStreamPerThread, which is a stream of its own in every host thread: a
+// number per thread, never given twice, tells those apart.  (hipStreamLegacy
+// and NULL are one stream under two handles: taken for two, which is safe.)
+// A destroyed stream's handle may come back for a new stream; no work of the
+// old one can be left on a block then, since every entry point waits for what
+// it released in order before it returns, or releases it unordered.
+struct Order {
+    bool ordered = false;
+    hipStream_t s = nullptr;
+    uint64_t thread = 0;
+    Order() = default;
+    Order(bool in_order, hipStream_t stream) : ordered(in_order), s(stream) {
+        static std::atomic<uint64_t> threads{0};
+        static thread_local const uint64_t mine = ++threads;
+        if (stream == hipStreamPerThread) thread = mine;
+    }
+    bool same(const Order& o) const { return ordered && o.ordered && s == o.s && thread == o.thread; }
+};
+
 // A freed block.  It may be handed out
-//  * for work on the stream its last use was on (stream order), or
+//  * for work in the order its last use was in, or
 //  * for any work once the device has been synchronised after its release
 //    (released <= the pool's synced count).
 struct FreeBlock {
     void* p;
     size_t bytes;
-    hipStream_t s;
-    bool ordered;
+    Order order;
     uint64_t released;  // position among the pool's releases
     std::chrono::steady_clock::time_point at;
 };
@@ -160,7 +180,7 @@ bool device_wait() {
 // Takes the best cached block for `want` bytes (at most an eighth larger,
 // or twice up to 64 KiB), or NULL.  *waits: a block would fit if the device
 // were synchronised.
-void* pool_take(Pool& q, size_t want, bool ordered, hipStream_t s, bool* waits) {
+void* pool_take(Pool& q, size_t want, const Order& order, bool* waits) {
     const size_t most = want <= (size_t(64) << 10) ? 2 * want : want + want / 8;
     size_t best = q.cached.size();
     int best_rank = 3;
@@ -168,7 +188,7 @@ void* pool_take(Pool& q, size_t want, bool ordered, hipStream_t s, bool* waits) 
     for (size_t k = q.cached.size(); k-- > 0;) {
         const FreeBlock& b = q.cached[k];
         if (b.bytes < want || b.bytes > most) continue;
-        const bool same = ordered && b.ordered && b.s == s;
+        const bool same = order.same(b.order);
         const bool idle = b.released <= q.synced;
         if (!same && !idle) {
             *waits = true;
@@ -212,13 +232,14 @@ void give_back(const std::vector<void*>& blocks) {
 
 void* pool_alloc(size_t bytes, bool ordered, hipStream_t s) {
     const size_t want = pool_round(bytes);
+    const Order order(ordered, s);
     Pool& q = g_pools[pool_device()];
     std::vector<void*> old;
     void* p = nullptr;
     {
         std::unique_lock<std::mutex> lk(q.mu);
         bool waits = false;
-        p = pool_take(q, want, ordered, s, &waits);
+        p = pool_take(q, want, order, &waits);
         if (!p && waits) {
             const uint64_t upto = q.releases;
             lk.unlock();
@@ -226,7 +247,7 @@ void* pool_alloc(size_t bytes, bool ordered, hipStream_t s) {
             lk.lock();
             if (ok) {
                 q.synced = std::max(q.synced, upto);
-                p = pool_take(q, want, ordered, s, &waits);
+                p = pool_take(q, want, order, &waits);
             }
         }
         old = pool_trim(q, kPoolKeep);
@@ -272,7 +293,7 @@ void pool_free(void* p, bool ordered, hipStream_t s) {
             const size_t bytes = it->second;
             q.live.erase(it);
             if (bytes <= kPoolKeep / 4) {  // one block does not crowd out the rest
-                q.cached.push_back({p, bytes, s, ordered, ++q.releases, std::chrono::steady_clock::now()});
+                q.cached.push_back({p, bytes, Order(ordered, s), ++q.releases, std::chrono::steady_clock::now()});
                 kept = true;
                 q.cached_bytes += bytes;
                 old = pool_trim(q, kPoolKeep);

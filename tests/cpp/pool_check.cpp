@@ -1,0 +1,165 @@
+// The device memory pool of csrc/runtime.cpp over a host stand-in for the HIP
+// calls it makes: "device" blocks are numbered addresses that nothing
+// dereferences, and every call is counted.  Each check is a run of its own
+// (argv[1]), so that it starts with an empty pool.  Prints "pool ok".
+#include <hip/hip_runtime.h>
+
+#include <atomic>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <functional>
+#include <set>
+#include <string>
+#include <thread>
+#include <vector>
+
+#include "common.h"
+
+// ------------------------------------------------------------- stand-in
+namespace {
+std::atomic<int> mallocs{0}, frees{0}, waits{0};
+size_t in_use = 0, capacity = size_t(1) << 50;
+uintptr_t next_address = uintptr_t(1) << 40;
+std::vector<std::pair<uintptr_t, size_t>> blocks;
+}  // namespace
+
+extern "C" {
+hipError_t hipMalloc(void** p, size_t bytes) {
+    ++mallocs;
+    if (in_use + bytes > capacity) return hipErrorOutOfMemory;
+    in_use += bytes;
+    *p = reinterpret_cast<void*>(next_address);
+    blocks.emplace_back(next_address, bytes);
+    next_address += (bytes + 4095) / 4096 * 4096;
+    return hipSuccess;
+}
+hipError_t hipFree(void* p) {
+    ++frees;
+    for (auto& b : blocks)
+        if (b.first == reinterpret_cast<uintptr_t>(p)) {
+            in_use -= b.second;
+            b = blocks.back();
+            blocks.pop_back();
+            return hipSuccess;
+        }
+    std::fprintf(stderr, "hipFree of %p, which is not allocated\n", p);
+    std::abort();
+}
+hipError_t hipDeviceSynchronize() {
+    ++waits;
+    return hipSuccess;
+}
+hipError_t hipGetDevice(int* d) {
+    *d = 0;
+    return hipSuccess;
+}
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetDeviceCount(int* n) {
+    *n = 1;
+    return hipSuccess;
+}
+hipError_t hipGetLastError() { return hipSuccess; }
+const char* hipGetErrorString(hipError_t) { return "stand-in error"; }
+hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode*) { return hipSuccess; }
+// not reached by the checks
+hipError_t hipDeviceGetDefaultMemPool(hipMemPool_t*, int) { return hipErrorNotSupported; }
+hipError_t hipMemPoolSetAttribute(hipMemPool_t, hipMemPoolAttr, void*) { return hipErrorNotSupported; }
+hipError_t hipMallocAsync(void**, size_t, hipStream_t) { return hipErrorNotSupported; }
+hipError_t hipFreeAsync(void*, hipStream_t) { return hipErrorNotSupported; }
+hipError_t hipEventCreate(hipEvent_t*) { return hipErrorNotSupported; }
+hipError_t hipEventCreateWithFlags(hipEvent_t*, unsigned) { return hipErrorNotSupported; }
+hipError_t hipEventDestroy(hipEvent_t) { return hipErrorNotSupported; }
+hipError_t hipEventElapsedTime(float*, hipEvent_t, hipEvent_t) { return hipErrorNotSupported; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipErrorNotSupported; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipErrorNotSupported; }
+hipError_t hipHostFree(void*) { return hipErrorNotSupported; }
+hipError_t hipHostMalloc(void**, size_t, unsigned) { return hipErrorNotSupported; }
+hipError_t hipMemcpyAsync(void*, const void*, size_t, hipMemcpyKind, hipStream_t) { return hipErrorNotSupported; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipErrorNotSupported; }
+}
+
+namespace btcx {
+unsigned long long* noalloc_workspace() { std::abort(); }
+}  // namespace btcx
+
+namespace {
+
+int failures = 0;
+
+#define EXPECT(cond)                                                                          \
+    do {                                                                                      \
+        if (!(cond)) {                                                                        \
+            std::fprintf(stderr, "%s:%d: check failed: %s\n", __FILE__, __LINE__, #cond);     \
+            ++failures;                                                                       \
+        }                                                                                     \
+    } while (0)
+
+hipStream_t stream(int k) { return reinterpret_cast<hipStream_t>(uintptr_t(0x1000) + 64 * (uintptr_t)k); }
+
+void on_thread(const std::function<void()>& f) {
+    std::thread t(f);
+    t.join();
+}
+
+using btcx::pool_alloc;
+using btcx::pool_free;
+
+// One handle value, another stream in each thread: a block that one thread
+// released in order is not handed to another without a wait for the device,
+// nor to a later thread that the system gave the first one's identity.
+void per_thread_stream() {
+    void* a = pool_alloc(4096, true, hipStreamPerThread);
+    pool_free(a, true, hipStreamPerThread);
+    on_thread([&] {
+        const int before = waits;
+        void* b = pool_alloc(4096, true, hipStreamPerThread);
+        EXPECT(b != a || waits > before);
+        pool_free(b, true, hipStreamPerThread);
+        void* c = pool_alloc(4096, true, hipStreamPerThread);
+        EXPECT(c == b);  // its own stream's order
+        pool_free(c, true, hipStreamPerThread);
+    });
+    for (int k = 0; k < 8; ++k) {
+        void* last = nullptr;
+        on_thread([&] {
+            last = pool_alloc(65536, true, hipStreamPerThread);
+            pool_free(last, true, hipStreamPerThread);
+        });
+        on_thread([&] {
+            const int before = waits;
+            void* b = pool_alloc(65536, true, hipStreamPerThread);
+            EXPECT(b != last || waits > before);
+            pool_free(b, true, hipStreamPerThread);
+        });
+    }
+    // one stream shared by threads stays one order
+    void* x = pool_alloc(1 << 20, true, stream(1));
+    pool_free(x, true, stream(1));
+    on_thread([&] {
+        const int before = waits;
+        void* y = pool_alloc(1 << 20, true, stream(1));
+        EXPECT(y == x && waits == before);
+        pool_free(y, true, stream(1));
+    });
+}
+
+const struct {
+    const char* name;
+    void (*run)();
+} kChecks[] = {
+    {"per_thread_stream", per_thread_stream},
+};
+
+}  // namespace
+
+int main(int argc, char** argv) {
+    for (const auto& c : kChecks)
+        if (argc == 2 && std::string(argv[1]) == c.name) {
+            c.run();
+            if (!failures) std::puts("pool ok");
+            return failures != 0;
+        }
+    std::fprintf(stderr, "usage: pool_check CHECK\n");
+    return 2;
+}
