@@ -393,6 +393,9 @@ int btc_batch_count(btc_batch b, void* stream, uint64_t* per_graph, uint64_t* to
     });
 }
 
-void btc_batch_free(btc_batch b) { delete b; }
+void btc_batch_free(btc_batch b) {
+    delete b;
+    btcx::pool_settle();
+}
 
 }  // extern "C"

@@ -1294,7 +1294,10 @@ int btc_bitbsr_copy_to_host(btc_bitbsr b, uint32_t* indptr, uint32_t* indices, u
     });
 }
 
-void btc_bitbsr_free(btc_bitbsr b) { delete b; }
+void btc_bitbsr_free(btc_bitbsr b) {
+    delete b;
+    btcx::pool_settle();
+}
 
 }  // extern "C"
 

@@ -716,6 +716,7 @@ void canonicalise_device(const int32_t* src, const int32_t* dst, int64_t nnz, in
         BTC_LAUNCH(rank_scatter_kernel, nc, s, alt ? v1.p : v0.p, nc, rank.p, labels.p, lab2.p);
         if (m) BTC_LAUNCH(relabel_kernel, m, s, keys, m, bn, rank.p, bn);
         keys = sort_u64(keys, spare, (size_t)m, 2 * bn, s);
+        labels.release_on(s);
         labels = std::move(lab2);
     }
 

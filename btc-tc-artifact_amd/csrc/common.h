@@ -73,9 +73,14 @@ int guard(F&& f) {
 // graph and 2.0 of the 3.2 ms of a 64^3 stencil's from host pairs.
 // `ordered`: the block's first (alloc) or last (free) use is in order on
 // stream s; otherwise nothing is known about the stream, and the block is
-// only reused once the device has been synchronised.
+// only reused once the device has been synchronised.  Neither call waits for
+// the device (but for blocks that go back to the driver): a thread that
+// builds a plan does not wait for the counts of others.  pool_settle does,
+// once, if blocks were released in no known order: a handle's free ends with
+// it, in place of hipFree's own wait.
 void* pool_alloc(size_t bytes, bool ordered, hipStream_t s);
 void pool_free(void* p, bool ordered, hipStream_t s);
+void pool_settle();
 
 // Owning device buffer (from the pool).
 template <class T>

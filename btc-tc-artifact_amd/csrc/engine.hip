@@ -737,8 +737,8 @@ void classify_dense(btc_plan_s* p, hipStream_t s, std::vector<uint8_t>& dense) {
         return;
     }
     const btc_bitbsr_s* b = plan_bsr(p, s);
-    DevBuf<uint32_t> d_pop;
-    d_pop.alloc_on(b->nblk, s);
+    TmpBuf<uint32_t> d_pop;
+    d_pop.alloc(b->nblk, s);
     launch_tile_popcount(b, d_pop.p, s);
     std::vector<uint32_t> pop(b->nblk), indptr((size_t)b->n_rb + 1), indices(b->nblk);
     BTC_HIP(hipMemcpyAsync(pop.data(), d_pop.p, (size_t)b->nblk * 4, hipMemcpyDeviceToHost, s));
@@ -756,7 +756,7 @@ void classify_dense(btc_plan_s* p, hipStream_t s, std::vector<uint8_t>& dense) {
     p->info.dense_tiles = p->n_dense;
     p->info.dense_edges = dense_edges;
     if (list.empty()) {
-        drop_plan_bsr(p);
+        drop_plan_bsr(p, s);
         return;
     }
     const int K = p->K;
@@ -1499,7 +1499,10 @@ int btc_plan_last_timing(btc_plan p, float* dense_ms, float* wedge_ms) {
     });
 }
 
-void btc_plan_free(btc_plan p) { delete p; }
+void btc_plan_free(btc_plan p) {
+    delete p;
+    btcx::pool_settle();
+}
 
 int btc_count(btc_graph g, const btc_count_opts* opts, void* stream, uint64_t* total, int32_t* per_vertex,
               float* kernel_ms) {

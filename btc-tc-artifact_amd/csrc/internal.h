@@ -359,7 +359,7 @@ void bitbsr_build(btc_graph_s* g, int K, hipStream_t s, btc_bitbsr_s* b, bool co
 
 // Sets p->bsr to the plan's Bit-BSR of width K: the caller's when the plan
 // was made on one, else one built on s (with dense_only, of the row blocks
-// its dense tiles need).  drop_plan_bsr releases it.
+// its dense tiles need).
 inline const btc_bitbsr_s* plan_bsr(btc_plan_s* p, hipStream_t s, bool dense_only = false) {
     if (p->ext_bsr) {
         p->bsr = p->ext_bsr;
@@ -370,7 +370,14 @@ inline const btc_bitbsr_s* plan_bsr(btc_plan_s* p, hipStream_t s, bool dense_onl
     }
     return p->bsr;
 }
-inline void drop_plan_bsr(btc_plan_s* p) {
+// Releases it, its last use being in order on s.
+inline void drop_plan_bsr(btc_plan_s* p, hipStream_t s) {
+    if (btc_bitbsr_s* b = p->own_bsr.get()) {
+        b->indptr.release_on(s);
+        b->indices.release_on(s);
+        b->row_indices.release_on(s);
+        b->tiles.release_on(s);
+    }
     p->own_bsr.reset();
     p->bsr = nullptr;
 }

@@ -690,6 +690,9 @@ int btc_pipeline_get_info(btc_pipeline p, btc_pipeline_info* info) {
     });
 }
 
-void btc_pipeline_free(btc_pipeline p) { delete p; }
+void btc_pipeline_free(btc_pipeline p) {
+    delete p;
+    btcx::pool_settle();
+}
 
 }  // extern "C"

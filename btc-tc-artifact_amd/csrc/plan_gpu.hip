@@ -697,7 +697,7 @@ void plan_device(btc_plan_s* p, int64_t chunk, hipStream_t s) {
             p->n_dense = nd;
         }
         BTC_HIP(hipStreamSynchronize(s));
-        if (!nd) drop_plan_bsr(p);
+        if (!nd) drop_plan_bsr(p, s);
     }
     p->info.dense_tiles = p->n_dense;
     p->info.dense_edges = (int64_t)read_dev(st.p + 0, s);

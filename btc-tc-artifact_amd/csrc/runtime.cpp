@@ -140,6 +140,7 @@ struct Pool {
     std::unordered_map<void*, size_t> live;    // bytes of every block handed out
     size_t cached_bytes = 0;
     uint64_t releases = 0, synced = 0;
+    uint64_t unordered = 0;  // the last release that was in no known order
 };
 
 // Never destroyed: buffers of static objects may outlive any order of
@@ -178,22 +179,17 @@ bool device_wait() {
 }
 
 // Takes the best cached block for `want` bytes (at most an eighth larger,
-// or twice up to 64 KiB), or NULL.  *waits: a block would fit if the device
-// were synchronised.
-void* pool_take(Pool& q, size_t want, const Order& order, bool* waits) {
+// or twice up to 64 KiB), or NULL.
+void* pool_take(Pool& q, size_t want, const Order& order) {
     const size_t most = want <= (size_t(64) << 10) ? 2 * want : want + want / 8;
     size_t best = q.cached.size();
     int best_rank = 3;
-    *waits = false;
     for (size_t k = q.cached.size(); k-- > 0;) {
         const FreeBlock& b = q.cached[k];
         if (b.bytes < want || b.bytes > most) continue;
         const bool same = order.same(b.order);
         const bool idle = b.released <= q.synced;
-        if (!same && !idle) {
-            *waits = true;
-            continue;
-        }
+        if (!same && !idle) continue;
         const int rank = b.bytes == want ? 0 : 1;
         if (rank < best_rank) {
             best = k;
@@ -237,19 +233,8 @@ void* pool_alloc(size_t bytes, bool ordered, hipStream_t s) {
     std::vector<void*> old;
     void* p = nullptr;
     {
-        std::unique_lock<std::mutex> lk(q.mu);
-        bool waits = false;
-        p = pool_take(q, want, order, &waits);
-        if (!p && waits) {
-            const uint64_t upto = q.releases;
-            lk.unlock();
-            const bool ok = device_wait();
-            lk.lock();
-            if (ok) {
-                q.synced = std::max(q.synced, upto);
-                p = pool_take(q, want, order, &waits);
-            }
-        }
+        std::lock_guard<std::mutex> lk(q.mu);
+        p = pool_take(q, want, order);
         old = pool_trim(q, kPoolKeep);
     }
     give_back(old);
@@ -293,6 +278,7 @@ void pool_free(void* p, bool ordered, hipStream_t s) {
             const size_t bytes = it->second;
             q.live.erase(it);
             if (bytes <= kPoolKeep / 4) {  // one block does not crowd out the rest
+                if (!ordered) q.unordered = q.releases + 1;
                 q.cached.push_back({p, bytes, Order(ordered, s), ++q.releases, std::chrono::steady_clock::now()});
                 kept = true;
                 q.cached_bytes += bytes;
@@ -304,6 +290,21 @@ void pool_free(void* p, bool ordered, hipStream_t s) {
     } catch (...) {
     }
     if (!kept) (void)hipFree(p);
+}
+
+void pool_settle() {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kPoolDevices) return;
+    Pool& q = g_pools[dev];
+    uint64_t upto;
+    {
+        std::lock_guard<std::mutex> lk(q.mu);
+        if (q.unordered <= q.synced) return;
+        upto = q.releases;
+    }
+    if (!device_wait()) return;
+    std::lock_guard<std::mutex> lk(q.mu);
+    q.synced = std::max(q.synced, upto);
 }
 
 void mem_pool_init() {

@@ -144,11 +144,39 @@ void per_thread_stream() {
     });
 }
 
+// An allocation never waits for the device: blocks that work of another
+// stream, or of no known one, may still use are left alone.  pool_settle waits
+// once for all of them.
+void no_waits() {
+    void* a = pool_alloc(1 << 16, true, stream(1));
+    pool_free(a, true, stream(1));
+    void* b = pool_alloc(1 << 16, true, stream(2));
+    EXPECT(b != a && waits == 0);
+    btcx::pool_settle();  // nothing was released in no known order
+    EXPECT(waits == 0);
+    pool_free(b, false, nullptr);
+    void* c = pool_alloc(1 << 16, false, nullptr);
+    void* d = pool_alloc(1 << 16, true, stream(2));
+    EXPECT(c != a && c != b && d != a && d != b && waits == 0);
+    btcx::pool_settle();
+    EXPECT(waits == 1);
+    btcx::pool_settle();
+    EXPECT(waits == 1);
+    const std::set<void*> idle{a, b};
+    void* e = pool_alloc(1 << 16, false, nullptr);
+    void* f = pool_alloc(1 << 16, true, stream(3));
+    EXPECT(idle.count(e) && idle.count(f) && e != f && waits == 1);
+    for (void* p : {c, d, e, f}) pool_free(p, false, nullptr);
+    btcx::pool_settle();
+    EXPECT(waits == 2 && mallocs == 4);
+}
+
 const struct {
     const char* name;
     void (*run)();
 } kChecks[] = {
     {"per_thread_stream", per_thread_stream},
+    {"no_waits", no_waits},
 };
 
 }  // namespace
