@@ -155,7 +155,7 @@ void batch_finish(btc_batch_s* b, const btc_count_opts* opts, hipStream_t s) {
     host_words(((size_t)b->count + 1) * 8);  // what a count returns through
     BTC_HIP(hipMemcpyAsync(b->d_voff.p, vo32.data(), vo32.size() * 4, hipMemcpyHostToDevice, s));
     batch_item_graphs(b, s);
-    BTC_HIP(hipStreamSynchronize(s));
+    stream_wait(s);
 }
 
 btc_batch_s* batch_from_graph(btc_graph_s&& g, const std::vector<int64_t>& voff, const btc_count_opts* opts,
@@ -186,7 +186,7 @@ btc_batch_s* batch_from_plan(btc_graph_s&& g, btc_plan_s* plan, const std::vecto
     host_words(((size_t)b->count + 1) * 8);  // what a count returns through
     BTC_HIP(hipMemcpyAsync(b->d_voff.p, vo32.data(), vo32.size() * 4, hipMemcpyHostToDevice, s));
     batch_item_graphs(b.get(), s);
-    BTC_HIP(hipStreamSynchronize(s));
+    stream_wait(s);
     return b.release();
 }
 
@@ -393,9 +393,6 @@ int btc_batch_count(btc_batch b, void* stream, uint64_t* per_graph, uint64_t* to
     });
 }
 
-void btc_batch_free(btc_batch b) {
-    delete b;
-    btcx::pool_settle();
-}
+void btc_batch_free(btc_batch b) { btcx::free_handle(b); }
 
 }  // extern "C"

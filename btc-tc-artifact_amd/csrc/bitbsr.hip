@@ -1260,7 +1260,7 @@ int btc_bitbsr_build(btc_graph g, int32_t tile_k, void* stream, btc_bitbsr* out)
                     "tile width K = %d (expected 32, 64 or 128)", tile_k);
         auto b = std::make_unique<btc_bitbsr_s>();
         btcx::bitbsr_build(g, tile_k, btcx::as_stream(stream), b.get(), true);
-        BTC_HIP(hipStreamSynchronize(btcx::as_stream(stream)));
+        btcx::stream_wait(btcx::as_stream(stream));
         *out = b.release();
     });
 }
@@ -1294,10 +1294,7 @@ int btc_bitbsr_copy_to_host(btc_bitbsr b, uint32_t* indptr, uint32_t* indices, u
     });
 }
 
-void btc_bitbsr_free(btc_bitbsr b) {
-    delete b;
-    btcx::pool_settle();
-}
+void btc_bitbsr_free(btc_bitbsr b) { btcx::free_handle(b); }
 
 }  // extern "C"
 

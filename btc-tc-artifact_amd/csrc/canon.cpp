@@ -286,10 +286,7 @@ int btc_graph_copy_labels(btc_graph g, int32_t* canon_to_input) {
     });
 }
 
-void btc_graph_free(btc_graph g) {
-    delete g;
-    btcx::pool_settle();
-}
+void btc_graph_free(btc_graph g) { btcx::free_handle(g); }
 
 // Host OpenMP merge over L: for every (i, j) in L count |N_L(i) & N_L(j)| by a
 // two-pointer walk (triangle_count_cpu.h:60-101); per_vertex[i] is the row sum.

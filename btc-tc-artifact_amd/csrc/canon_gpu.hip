@@ -736,7 +736,7 @@ void canonicalise_device(const int32_t* src, const int32_t* dst, int64_t nnz, in
     if (nc) BTC_LAUNCH_RED(stats_kernel, std::max<int64_t>(nc, m), s, g->d_rowptr.p, g->d_col.p, nc, m, st.p);
     unsigned long long h[3] = {0, 0, 0};
     BTC_HIP(hipMemcpyAsync(h, st.p, 24, hipMemcpyDeviceToHost, s));
-    BTC_HIP(hipStreamSynchronize(s));
+    stream_wait(s);
     g->max_row = (int32_t)h[0];
     g->wedges = (int64_t)h[1];
     g->merge_work = (int64_t)h[2];

@@ -47,6 +47,9 @@ inline void check_status(int rc) {
     if (rc != BTC_OK) throw Error{rc};
 }
 
+// Notes a call that failed, perhaps with work left on a stream (runtime.cpp).
+void pool_call_failed();
+
 // Runs f and maps library errors to status codes for the C ABI.
 template <class F>
 int guard(F&& f) {
@@ -55,11 +58,16 @@ int guard(F&& f) {
         f();
         return BTC_OK;
     } catch (const Error& e) {
+        // bad arguments are refused before any work is enqueued, or on the
+        // device's word once it has ended
+        if (e.code != BTC_ERR_ARG) pool_call_failed();
         return e.code;
     } catch (const std::bad_alloc&) {
+        pool_call_failed();
         set_error("host allocation failed");
         return BTC_ERR_NOMEM;
     } catch (...) {
+        pool_call_failed();
         set_error("unexpected exception");
         return BTC_ERR_STATE;
     }
@@ -73,14 +81,35 @@ int guard(F&& f) {
 // graph and 2.0 of the 3.2 ms of a 64^3 stencil's from host pairs.
 // `ordered`: the block's first (alloc) or last (free) use is in order on
 // stream s; otherwise nothing is known about the stream, and the block is
-// only reused once the device has been synchronised.  Neither call waits for
-// the device (but for blocks that go back to the driver): a thread that
-// builds a plan does not wait for the counts of others.  pool_settle does,
-// once, if blocks were released in no known order: a handle's free ends with
-// it, in place of hipFree's own wait.
+// only reused once it is idle.  Neither call waits for the device (but for
+// blocks that go back to the driver): a thread that builds a plan does not
+// wait for the counts of others.
 void* pool_alloc(size_t bytes, bool ordered, hipStream_t s);
 void pool_free(void* p, bool ordered, hipStream_t s);
+
+// Waits for the device, once, if blocks were released in no known order.
 void pool_settle();
+
+// hipStreamSynchronize at the end of a call: what the call released in order
+// on s is idle then.
+void stream_wait(hipStream_t s);
+
+// Around the destruction of a handle: no entry point returns before its work
+// has ended, so the handle's buffers are idle.  After a call that failed
+// (pool_call_failed) they are taken to be in use until the device has been
+// synchronised, which the scope's end does.
+struct IdleScope {
+    IdleScope();
+    ~IdleScope();
+    IdleScope(const IdleScope&) = delete;
+    IdleScope& operator=(const IdleScope&) = delete;
+};
+
+template <class H>
+void free_handle(H* h) {
+    IdleScope scope;
+    delete h;
+}
 
 // Owning device buffer (from the pool).
 template <class T>

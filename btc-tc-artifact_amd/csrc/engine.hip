@@ -1363,7 +1363,7 @@ btc_plan_s* plan_create(btc_graph g, const btc_count_opts* opts, hipStream_t s, 
     if (p->n_dense) p->n_units = btcx::build_dense_units(p->bsr, p->dense_list.p, p->n_dense, p->dense_units, s);
     p->scratch.alloc_on(btcx::kWorkWords, s);
     BTC_HIP(hipMemsetAsync(p->scratch.p, 0, p->scratch.bytes(), s));
-    BTC_HIP(hipStreamSynchronize(s));  // counts may run on other streams
+    btcx::stream_wait(s);  // counts may run on other streams
     p->scratch_clean = true;
     p->info.tile_k = p->K;
     p->info.tau = p->tau;
@@ -1499,10 +1499,7 @@ int btc_plan_last_timing(btc_plan p, float* dense_ms, float* wedge_ms) {
     });
 }
 
-void btc_plan_free(btc_plan p) {
-    delete p;
-    btcx::pool_settle();
-}
+void btc_plan_free(btc_plan p) { btcx::free_handle(p); }
 
 int btc_count(btc_graph g, const btc_count_opts* opts, void* stream, uint64_t* total, int32_t* per_vertex,
               float* kernel_ms) {

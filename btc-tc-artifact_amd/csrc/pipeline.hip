@@ -690,9 +690,6 @@ int btc_pipeline_get_info(btc_pipeline p, btc_pipeline_info* info) {
     });
 }
 
-void btc_pipeline_free(btc_pipeline p) {
-    delete p;
-    btcx::pool_settle();
-}
+void btc_pipeline_free(btc_pipeline p) { btcx::free_handle(p); }
 
 }  // extern "C"

@@ -8,6 +8,7 @@
 #include <chrono>
 #include <cstring>
 #include <exception>
+#include <map>
 #include <mutex>
 #include <unordered_map>
 #include <vector>
@@ -117,13 +118,13 @@ struct Order {
 
 // A freed block.  It may be handed out
 //  * for work in the order its last use was in, or
-//  * for any work once the device has been synchronised after its release
-//    (released <= the pool's synced count).
+//  * for any work when it is idle: released so (released == 0), or the device
+//    or its stream has been synchronised after its release.
 struct FreeBlock {
     void* p;
     size_t bytes;
     Order order;
-    uint64_t released;  // position among the pool's releases
+    uint64_t released;  // position among the pool's releases, from 1
     std::chrono::steady_clock::time_point at;
 };
 
@@ -139,9 +140,22 @@ struct Pool {
     std::vector<FreeBlock> cached;             // oldest release first
     std::unordered_map<void*, size_t> live;    // bytes of every block handed out
     size_t cached_bytes = 0;
-    uint64_t releases = 0, synced = 0;
-    uint64_t unordered = 0;  // the last release that was in no known order
+    uint64_t releases = 0, synced = 0;  // releases up to synced: device synchronised since
+    uint64_t unordered = 0;             // the last release that was in no known order
+    uint64_t failed_synced = 0;         // of g_failed: device synchronised since
+    std::map<std::pair<hipStream_t, uint64_t>, uint64_t> stream_synced;  // as synced, by order
+
+    bool idle(const FreeBlock& b) const {
+        if (b.released <= synced) return true;
+        if (!b.order.ordered) return false;
+        const auto it = stream_synced.find({b.order.s, b.order.thread});
+        return it != stream_synced.end() && b.released <= it->second;
+    }
 };
+
+thread_local int tl_idle_scopes = 0;
+std::atomic<uint64_t> g_failed{0};       // calls that failed, perhaps with work left on a stream
+std::atomic<bool> g_unsettled{false};    // blocks may wait for pool_settle
 
 // Never destroyed: buffers of static objects may outlive any order of
 // destruction, and the driver takes the memory back with the process.
@@ -187,9 +201,7 @@ void* pool_take(Pool& q, size_t want, const Order& order) {
     for (size_t k = q.cached.size(); k-- > 0;) {
         const FreeBlock& b = q.cached[k];
         if (b.bytes < want || b.bytes > most) continue;
-        const bool same = order.same(b.order);
-        const bool idle = b.released <= q.synced;
-        if (!same && !idle) continue;
+        if (!order.same(b.order) && !q.idle(b)) continue;
         const int rank = b.bytes == want ? 0 : 1;
         if (rank < best_rank) {
             best = k;
@@ -264,7 +276,8 @@ void* pool_alloc(size_t bytes, bool ordered, hipStream_t s) {
 void pool_free(void* p, bool ordered, hipStream_t s) {
     if (!p) return;
     // a buffer of a call that failed half-way: work may be left on any stream
-    if (std::uncaught_exceptions() > 0) ordered = false;
+    const bool unwinding = std::uncaught_exceptions() > 0;
+    if (unwinding) ordered = false;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) dev = 0;
     bool kept = false;
@@ -278,8 +291,15 @@ void pool_free(void* p, bool ordered, hipStream_t s) {
             const size_t bytes = it->second;
             q.live.erase(it);
             if (bytes <= kPoolKeep / 4) {  // one block does not crowd out the rest
-                if (!ordered) q.unordered = q.releases + 1;
-                q.cached.push_back({p, bytes, Order(ordered, s), ++q.releases, std::chrono::steady_clock::now()});
+                // a handle's own buffer: idle, as no call leaves work behind it
+                // (but for failed ones)
+                const bool idle = !ordered && !unwinding && tl_idle_scopes > 0 && q.failed_synced == g_failed;
+                const uint64_t at = idle ? 0 : ++q.releases;
+                if (!ordered && !idle) {
+                    q.unordered = at;
+                    g_unsettled = true;
+                }
+                q.cached.push_back({p, bytes, Order(ordered, s), at, std::chrono::steady_clock::now()});
                 kept = true;
                 q.cached_bytes += bytes;
                 old = pool_trim(q, kPoolKeep);
@@ -292,19 +312,50 @@ void pool_free(void* p, bool ordered, hipStream_t s) {
     if (!kept) (void)hipFree(p);
 }
 
+IdleScope::IdleScope() { ++tl_idle_scopes; }
+
+IdleScope::~IdleScope() {
+    if (--tl_idle_scopes == 0) pool_settle();
+}
+
 void pool_settle() {
+    if (!g_unsettled) return;  // no HIP call: handles that never saw a device are freed too
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kPoolDevices) return;
     Pool& q = g_pools[dev];
-    uint64_t upto;
+    uint64_t upto, failed;
     {
         std::lock_guard<std::mutex> lk(q.mu);
-        if (q.unordered <= q.synced) return;
+        if (q.unordered <= q.synced) return;  // another device's
+        upto = q.releases;
+        failed = g_failed;
+        g_unsettled = false;
+    }
+    const bool ok = device_wait();
+    std::lock_guard<std::mutex> lk(q.mu);
+    if (ok) {
+        q.synced = std::max(q.synced, upto);
+        q.failed_synced = std::max(q.failed_synced, failed);
+    } else {
+        g_unsettled = true;
+    }
+}
+
+void pool_call_failed() { ++g_failed; }
+
+void stream_wait(hipStream_t s) {
+    Pool& q = g_pools[pool_device()];
+    uint64_t upto;  // before the wait: other threads may use the stream meanwhile
+    {
+        std::lock_guard<std::mutex> lk(q.mu);
         upto = q.releases;
     }
-    if (!device_wait()) return;
+    BTC_HIP(hipStreamSynchronize(s));
+    const Order o(true, s);
     std::lock_guard<std::mutex> lk(q.mu);
-    q.synced = std::max(q.synced, upto);
+    if (q.stream_synced.size() >= 1024) q.stream_synced.clear();  // handles and threads come and go
+    uint64_t& at = q.stream_synced[{o.s, o.thread}];
+    at = std::max(at, upto);
 }
 
 void mem_pool_init() {

@@ -9,6 +9,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <functional>
+#include <memory>
 #include <set>
 #include <string>
 #include <thread>
@@ -22,6 +23,7 @@ std::atomic<int> mallocs{0}, frees{0}, waits{0};
 size_t in_use = 0, capacity = size_t(1) << 50;
 uintptr_t next_address = uintptr_t(1) << 40;
 std::vector<std::pair<uintptr_t, size_t>> blocks;
+std::function<void()> during_sync;
 }  // namespace
 
 extern "C" {
@@ -50,6 +52,10 @@ hipError_t hipDeviceSynchronize() {
     ++waits;
     return hipSuccess;
 }
+hipError_t hipStreamSynchronize(hipStream_t) {
+    if (during_sync) during_sync();
+    return hipSuccess;
+}
 hipError_t hipGetDevice(int* d) {
     *d = 0;
     return hipSuccess;
@@ -76,7 +82,6 @@ hipError_t hipEventSynchronize(hipEvent_t) { return hipErrorNotSupported; }
 hipError_t hipHostFree(void*) { return hipErrorNotSupported; }
 hipError_t hipHostMalloc(void**, size_t, unsigned) { return hipErrorNotSupported; }
 hipError_t hipMemcpyAsync(void*, const void*, size_t, hipMemcpyKind, hipStream_t) { return hipErrorNotSupported; }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipErrorNotSupported; }
 }
 
 namespace btcx {
@@ -171,12 +176,89 @@ void no_waits() {
     EXPECT(waits == 2 && mallocs == 4);
 }
 
+struct Handle {
+    btcx::DevBuf<char> x;
+};
+
+Handle* make(hipStream_t s) {
+    auto* h = new Handle;
+    h->x.alloc_on(1 << 16, s);
+    return h;
+}
+
+// A handle's buffers are idle when it is freed: no wait, and any stream may
+// have them next.  After a call that failed with work enqueued, perhaps, the
+// free waits, and the next one need not; bad arguments are not such a call.
+void handles() {
+    Handle* h = make(stream(1));
+    void* a = h->x.p;
+    btcx::free_handle(h);
+    EXPECT(waits == 0);
+    h = make(stream(2));
+    EXPECT(h->x.p == a && waits == 0);
+    EXPECT(btcx::guard([] { btcx::fail(BTC_ERR_ARG, "refused"); }) == BTC_ERR_ARG);
+    btcx::free_handle(h);
+    EXPECT(waits == 0);
+    h = make(stream(3));
+    EXPECT(h->x.p == a);
+    EXPECT(btcx::guard([] { btcx::fail(BTC_ERR_HIP, "failed"); }) == BTC_ERR_HIP);
+    btcx::free_handle(h);
+    EXPECT(waits == 1);
+    h = make(stream(4));
+    EXPECT(h->x.p == a);
+    btcx::free_handle(h);
+    EXPECT(waits == 1);
+    // a handle that a failing call drops: its work may be pending
+    EXPECT(btcx::guard([] {
+               std::unique_ptr<Handle> x(make(stream(5)));
+               btcx::fail(BTC_ERR_ARG, "half-way");
+           }) == BTC_ERR_ARG);
+    h = make(stream(6));
+    EXPECT(h->x.p != a && waits == 1);
+    btcx::free_handle(h);  // settles what the failing call left
+    EXPECT(waits == 2);
+}
+
+// A call's buffers, released in order on its stream, are idle once the call
+// has waited for the stream -- not those that another thread released on it
+// after that wait began.
+void waited_streams() {
+    void* a = pool_alloc(1 << 16, true, stream(1));
+    pool_free(a, true, stream(1));
+    during_sync = [] {
+        void* b = pool_alloc(1 << 18, true, stream(1));
+        pool_free(b, true, stream(1));
+    };
+    btcx::stream_wait(stream(1));
+    during_sync = nullptr;
+    void* c = pool_alloc(1 << 16, true, stream(2));
+    EXPECT(c == a && waits == 0);
+    const int before = mallocs;
+    void* d = pool_alloc(1 << 18, true, stream(2));
+    EXPECT(mallocs == before + 1 && waits == 0);
+    pool_free(c, true, stream(2));
+    pool_free(d, true, stream(2));
+    // the per-thread handle: another thread's wait says nothing about this one's stream
+    void* e = pool_alloc(1 << 20, true, hipStreamPerThread);
+    pool_free(e, true, hipStreamPerThread);
+    on_thread([] { btcx::stream_wait(hipStreamPerThread); });
+    void* f = pool_alloc(1 << 20, true, stream(2));
+    EXPECT(f != e);
+    btcx::stream_wait(hipStreamPerThread);
+    void* g = pool_alloc(1 << 20, true, stream(2));
+    EXPECT(g == e);
+    pool_free(f, true, stream(2));
+    pool_free(g, true, stream(2));
+}
+
 const struct {
     const char* name;
     void (*run)();
 } kChecks[] = {
     {"per_thread_stream", per_thread_stream},
     {"no_waits", no_waits},
+    {"handles", handles},
+    {"waited_streams", waited_streams},
 };
 
 }  // namespace
