@@ -7,7 +7,9 @@
 #include <cstdarg>
 #include <chrono>
 #include <cstring>
+#include <deque>
 #include <exception>
+#include <list>
 #include <map>
 #include <mutex>
 #include <unordered_map>
@@ -128,16 +130,21 @@ struct FreeBlock {
     std::chrono::steady_clock::time_point at;
 };
 
-// Bounded three ways: at most kPoolKeep cached bytes per device (3 % of its
-// memory; the oldest blocks go first), blocks that nothing took for
-// kPoolIdle are returned at the next call, and a failing allocation returns
-// every cached block before it is tried once more.
+// Bounded: at most kPoolKeep cached bytes per device (3 % of its memory) in at
+// most kPoolBlocks blocks, the oldest going first; blocks that nothing took
+// for kPoolIdle are returned by the calls that follow, up to kPoolIdleEach by
+// each; and a failing allocation returns every cached block before it is
+// tried once more.
 constexpr size_t kPoolKeep = size_t(8) << 30;
+constexpr size_t kPoolBlocks = 4096;
 constexpr std::chrono::seconds kPoolIdle{10};
+constexpr size_t kPoolIdleEach = 16;
 
 struct Pool {
     std::mutex mu;
-    std::vector<FreeBlock> cached;             // oldest release first
+    using At = std::list<FreeBlock>::iterator;
+    std::list<FreeBlock> cached;               // oldest release first
+    std::map<size_t, std::deque<At>> by_size;  // the same blocks, each size's oldest first
     std::unordered_map<void*, size_t> live;    // bytes of every block handed out
     size_t cached_bytes = 0;
     uint64_t releases = 0, synced = 0;  // releases up to synced: device synchronised since
@@ -192,43 +199,54 @@ bool device_wait() {
     return e == hipSuccess;
 }
 
-// Takes the best cached block for `want` bytes (at most an eighth larger,
-// or twice up to 64 KiB), or NULL.
+// Takes the cached block for `want` bytes that wastes least (at most an eighth
+// of them, or as much again up to 64 KiB), the newest of its size, or NULL.
 void* pool_take(Pool& q, size_t want, const Order& order) {
     const size_t most = want <= (size_t(64) << 10) ? 2 * want : want + want / 8;
-    size_t best = q.cached.size();
-    int best_rank = 3;
-    for (size_t k = q.cached.size(); k-- > 0;) {
-        const FreeBlock& b = q.cached[k];
-        if (b.bytes < want || b.bytes > most) continue;
-        if (!order.same(b.order) && !q.idle(b)) continue;
-        const int rank = b.bytes == want ? 0 : 1;
-        if (rank < best_rank) {
-            best = k;
-            best_rank = rank;
-            if (rank == 0) break;
+    for (auto sz = q.by_size.lower_bound(want); sz != q.by_size.end() && sz->first <= most; ++sz) {
+        auto& same = sz->second;
+        for (size_t k = same.size(); k-- > 0;) {
+            const FreeBlock b = *same[k];
+            if (!order.same(b.order) && !q.idle(b)) continue;
+            q.live[b.p] = b.bytes;  // may throw: before the block leaves the cache
+            q.cached.erase(same[k]);
+            same.erase(same.begin() + (std::ptrdiff_t)k);
+            if (same.empty()) q.by_size.erase(sz);
+            q.cached_bytes -= b.bytes;
+            return b.p;
         }
     }
-    if (best == q.cached.size()) return nullptr;
-    const FreeBlock b = q.cached[best];
-    q.cached.erase(q.cached.begin() + (std::ptrdiff_t)best);
-    q.cached_bytes -= b.bytes;
-    q.live[b.p] = b.bytes;
-    return b.p;
+    return nullptr;
 }
 
-// Blocks to give back now: idle for kPoolIdle, or the oldest beyond keep
-// bytes.
+void pool_keep(Pool& q, const FreeBlock& b) {
+    auto& same = q.by_size[b.bytes];
+    q.cached.push_back(b);
+    try {
+        same.push_back(std::prev(q.cached.end()));
+    } catch (...) {
+        q.cached.pop_back();
+        throw;
+    }
+    q.cached_bytes += b.bytes;
+}
+
+// Blocks to give back now: the oldest beyond `keep` bytes or kPoolBlocks, and
+// some of those idle for kPoolIdle.
 std::vector<void*> pool_trim(Pool& q, size_t keep) {
     std::vector<void*> out;
     const auto now = std::chrono::steady_clock::now();
-    size_t k = 0;
-    while (k < q.cached.size() && (q.cached_bytes > keep || now - q.cached[k].at > kPoolIdle)) {
-        out.push_back(q.cached[k].p);
-        q.cached_bytes -= q.cached[k].bytes;
-        ++k;
+    while (!q.cached.empty()) {
+        const FreeBlock& b = q.cached.front();
+        const bool idle = now - b.at > kPoolIdle && out.size() < kPoolIdleEach;
+        if (!idle && q.cached_bytes <= keep && q.cached.size() <= kPoolBlocks) break;
+        out.push_back(b.p);
+        q.cached_bytes -= b.bytes;
+        const auto sz = q.by_size.find(b.bytes);
+        sz->second.pop_front();  // the oldest of all is the oldest of its size
+        if (sz->second.empty()) q.by_size.erase(sz);
+        q.cached.pop_front();
     }
-    q.cached.erase(q.cached.begin(), q.cached.begin() + (std::ptrdiff_t)k);
     return out;
 }
 
@@ -299,9 +317,8 @@ void pool_free(void* p, bool ordered, hipStream_t s) {
                     q.unordered = at;
                     g_unsettled = true;
                 }
-                q.cached.push_back({p, bytes, Order(ordered, s), at, std::chrono::steady_clock::now()});
+                pool_keep(q, {p, bytes, Order(ordered, s), at, std::chrono::steady_clock::now()});
                 kept = true;
-                q.cached_bytes += bytes;
                 old = pool_trim(q, kPoolKeep);
             }
             break;

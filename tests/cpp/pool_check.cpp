@@ -4,11 +4,13 @@
 // (argv[1]), so that it starts with an empty pool.  Prints "pool ok".
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <functional>
+#include <map>
 #include <memory>
 #include <set>
 #include <string>
@@ -251,6 +253,60 @@ void waited_streams() {
     pool_free(g, true, stream(2));
 }
 
+// The cache is bounded in bytes and in blocks, and no call gives back more
+// than a few blocks beyond what it brings; larger blocks are not kept.
+void bounded() {
+    std::vector<void*> p;
+    for (int k = 0; k < 20000; ++k) p.push_back(pool_alloc(512, true, stream(1)));
+    int most = 0;
+    for (void* x : p) {
+        const int before = frees;
+        pool_free(x, true, stream(1));
+        most = std::max(most, frees - before);
+    }
+    EXPECT(blocks.size() <= 5000 && most <= 2);
+    p.clear();
+    for (int k = 0; k < 24; ++k) p.push_back(pool_alloc(size_t(1) << 30, true, stream(1)));
+    for (void* x : p) pool_free(x, true, stream(1));
+    EXPECT(in_use <= (size_t(8) << 30));
+    void* big = pool_alloc(size_t(5) << 30, true, stream(1));
+    const int before = frees;
+    pool_free(big, true, stream(1));
+    EXPECT(frees == before + 1);
+    // a refused allocation returns the cache and is tried again
+    capacity = size_t(9) << 30;
+    void* x = pool_alloc(size_t(8) << 30, true, stream(2));
+    EXPECT(x && in_use == (size_t(8) << 30));
+    EXPECT(btcx::guard([] { pool_alloc(size_t(2) << 30, true, stream(2)); }) == BTC_ERR_NOMEM);
+    pool_free(x, true, stream(2));
+    EXPECT(in_use == 0);
+}
+
+// The block that wastes least, at most an eighth (twice for small ones), and
+// the newest of its size that may be used.
+void sizes() {
+    const size_t kSizes[] = {1 << 20, (1 << 20) + (1 << 17), (1 << 20) + (1 << 18)};
+    std::map<size_t, void*> at;
+    for (size_t b : kSizes) at[b] = pool_alloc(b, true, stream(1));
+    for (size_t b : kSizes) pool_free(at[b], true, stream(1));
+    for (int k = 0; k < 3; ++k)
+        for (size_t b : kSizes) {
+            void* p = pool_alloc(b - 100, true, stream(1));
+            EXPECT(p == at[b]);
+            pool_free(p, true, stream(1));
+        }
+    void* p = pool_alloc(1 << 20, true, stream(1));
+    void* q = pool_alloc(1 << 20, true, stream(1));  // an eighth more
+    const int before = mallocs;
+    void* r = pool_alloc(1 << 20, true, stream(1));  // a quarter more is left
+    EXPECT(p == at[kSizes[0]] && q == at[kSizes[1]] && mallocs == before + 1);
+    pool_free(p, true, stream(1));
+    pool_free(r, true, stream(1));
+    pool_free(q, true, stream(2));  // another stream's
+    EXPECT(pool_alloc(1 << 20, true, stream(1)) == r);
+    EXPECT(pool_alloc(1 << 20, true, stream(1)) == p);
+}
+
 const struct {
     const char* name;
     void (*run)();
@@ -259,6 +315,8 @@ const struct {
     {"no_waits", no_waits},
     {"handles", handles},
     {"waited_streams", waited_streams},
+    {"bounded", bounded},
+    {"sizes", sizes},
 };
 
 }  // namespace
