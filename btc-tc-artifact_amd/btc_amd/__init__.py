@@ -115,6 +115,7 @@ _SIGS = {
     "btc_last_error": (C.c_char_p, []),
     "btc_version": (C.c_char_p, []),
     "btc_device_init": (C.c_int, [C.c_int32]),
+    "btc_memory_trim": (C.c_int, [C.POINTER(C.c_int64)]),
     "btc_gen_rmat": (C.c_int64, [C.c_int32, C.c_int32, C.c_double, C.c_double, C.c_double, C.c_uint64, vp, vp]),
     "btc_gen_er": (C.c_int64, [C.c_int32, C.c_double, C.c_uint64, vp, vp]),
     "btc_gen_stencil2d": (C.c_int64, [C.c_int32, C.c_int32, vp, vp]),
@@ -214,6 +215,14 @@ def _ptr(a):
 
 def version():
     return lib().btc_version().decode()
+
+
+def memory_trim():
+    """Returns the device memory that the library keeps of freed handles to
+    the driver; its bytes (btc_memory_trim)."""
+    got = C.c_int64(0)
+    _check(lib().btc_memory_trim(C.byref(got)))
+    return got.value
 
 
 def lite_tile_k(n, m, mode=0):

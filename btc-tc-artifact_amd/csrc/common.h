@@ -90,6 +90,9 @@ void pool_free(void* p, bool ordered, hipStream_t s);
 // Waits for the device, once, if blocks were released in no known order.
 void pool_settle();
 
+// Returns the current device's cached blocks to the driver; their bytes.
+int64_t pool_release_all();
+
 // hipStreamSynchronize at the end of a call: what the call released in order
 // on s is idle then.
 void stream_wait(hipStream_t s);

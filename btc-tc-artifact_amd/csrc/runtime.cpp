@@ -360,6 +360,19 @@ void pool_settle() {
 
 void pool_call_failed() { ++g_failed; }
 
+int64_t pool_release_all() {
+    Pool& q = g_pools[pool_device()];
+    std::vector<void*> all;
+    size_t bytes;
+    {
+        std::lock_guard<std::mutex> lk(q.mu);
+        bytes = q.cached_bytes;
+        all = pool_trim(q, 0);
+    }
+    give_back(all);
+    return (int64_t)bytes;
+}
+
 void stream_wait(hipStream_t s) {
     Pool& q = g_pools[pool_device()];
     uint64_t upto;  // before the wait: other threads may use the stream meanwhile
@@ -562,6 +575,13 @@ extern "C" {
 const char* btc_last_error(void) { return btcx::g_err; }
 
 const char* btc_version(void) { return "0.1.0-gfx950"; }
+
+int btc_memory_trim(int64_t* released_bytes) {
+    return btcx::guard([&] {
+        const int64_t bytes = btcx::pool_release_all();
+        if (released_bytes) *released_bytes = bytes;
+    });
+}
 
 int btc_device_init(int32_t device) {
     return btcx::guard([&] {

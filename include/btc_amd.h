@@ -56,6 +56,13 @@ const char* btc_last_error(void);
 const char* btc_version(void);
 /* Select the HIP device for calls from this thread; returns BTC_ERR_HIP if absent. */
 int btc_device_init(int32_t device);
+/* Device memory of freed handles and of temporary arrays is kept for later
+ * calls: per device at most 8 GiB in at most 4096 blocks, of which later calls
+ * return those that nothing took for 10 s.  This returns all of the current
+ * device's to the driver now (waiting for work that still uses them), for a
+ * program that goes on without this library; *released_bytes (may be NULL) =
+ * their size. */
+int btc_memory_trim(int64_t* released_bytes);
 
 /* --------------------------------------------------------- synthetic inputs
  * Seeded generators (host, OpenMP).  Every random draw is

@@ -307,6 +307,20 @@ void sizes() {
     EXPECT(pool_alloc(1 << 20, true, stream(1)) == p);
 }
 
+// What the cache holds goes back on request, handed-out blocks stay.
+void trim() {
+    void* a = pool_alloc(1 << 20, true, stream(1));
+    void* b = pool_alloc(3 << 20, true, stream(2));
+    void* c = pool_alloc(5 << 20, false, nullptr);
+    pool_free(a, true, stream(1));
+    pool_free(c, false, nullptr);
+    int64_t bytes = -1;
+    EXPECT(btc_memory_trim(&bytes) == BTC_OK && bytes == int64_t(6) << 20 && in_use == size_t(3) << 20);
+    EXPECT(btc_memory_trim(nullptr) == BTC_OK && btc_memory_trim(&bytes) == BTC_OK && bytes == 0);
+    pool_free(b, true, stream(2));
+    EXPECT(pool_alloc(3 << 20, true, stream(2)) == b);
+}
+
 const struct {
     const char* name;
     void (*run)();
@@ -317,6 +331,7 @@ const struct {
     {"waited_streams", waited_streams},
     {"bounded", bounded},
     {"sizes", sizes},
+    {"trim", trim},
 };
 
 }  // namespace
