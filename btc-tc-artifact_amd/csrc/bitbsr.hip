@@ -1350,7 +1350,7 @@ void bitbsr_count(btc_bitbsr b, int32_t variant, int32_t threshold_blocks, int32
     pv.copy_out(pv32, pv64, s);  // synchronises s
     b->work_clean = true;
     const uint64_t h = *h_total;
-    pv.release_on(s);
+    pv.release_idle();
     if (kernel_ms) *kernel_ms = tm.ms();
     *total = h;
 }

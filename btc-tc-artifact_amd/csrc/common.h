@@ -388,15 +388,18 @@ struct PvBuf {
         if (max_row <= kPv32MaxRow) b32.alloc(count);
         else b64.alloc(count);
     }
-    // for one count on s, which copy_out's wait ends
+    // for one count on s, which copy_out's wait ends (release_idle then)
     void alloc_on(size_t count, int32_t max_row, hipStream_t s) {
         n = count;
         if (max_row <= kPv32MaxRow) b32.alloc_on(count, s);
         else b64.alloc_on(count, s);
     }
-    void release_on(hipStream_t s) {
-        b32.release_on(s);
-        b64.release_on(s);
+    // after the wait for the work that used it (a failed call, whose stack
+    // unwinds, leaves it to the destructors instead)
+    void release_idle() {
+        IdleScope scope;
+        b32.release();
+        b64.release();
     }
     PvOut out() const { return PvOut{b32.p, b64.p}; }
     bool wide() const { return b64.p != nullptr; }

@@ -1281,7 +1281,7 @@ void plan_count(btc_plan_s* p, hipStream_t s, uint64_t* total, int32_t* pv32, in
     pv.copy_out(pv32, pv64, s);  // synchronises s
     p->scratch_clean = true;
     const uint64_t h = *h_total;
-    pv.release_on(s);
+    pv.release_idle();
     if (kernel_ms) {
         *kernel_ms = tm.ms();
         p->last_wedge_ms = parts ? tw.ms() : *kernel_ms;

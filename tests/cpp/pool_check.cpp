@@ -321,6 +321,30 @@ void trim() {
     EXPECT(pool_alloc(3 << 20, true, stream(2)) == b);
 }
 
+// Per-vertex sums of a count that has been waited for serve the next count on
+// any stream; those of a count that failed do not before a wait.
+void count_sums() {
+    void* first = nullptr;
+    for (int k = 1; k <= 5; ++k) {
+        btcx::PvBuf pv;
+        pv.alloc_on(1 << 16, k, stream(k));
+        if (!first) first = pv.data();
+        EXPECT(pv.data() == first);
+        pv.release_idle();
+    }
+    EXPECT(mallocs == 1 && waits == 0);
+    EXPECT(btcx::guard([] {
+               btcx::PvBuf pv;
+               pv.alloc_on(1 << 16, 1, stream(1));
+               btcx::fail(BTC_ERR_HIP, "failed");
+           }) == BTC_ERR_HIP);
+    btcx::PvBuf pv;
+    pv.alloc_on(1 << 16, 1, stream(1));
+    EXPECT(mallocs == 2 && waits == 0);
+    pv.release_idle();
+    EXPECT(waits == 1);
+}
+
 const struct {
     const char* name;
     void (*run)();
@@ -332,6 +356,7 @@ const struct {
     {"bounded", bounded},
     {"sizes", sizes},
     {"trim", trim},
+    {"count_sums", count_sums},
 };
 
 }  // namespace

@@ -28,7 +28,7 @@ def pool_check(tmp_path_factory):
 
 
 @pytest.mark.parametrize("check", ["per_thread_stream", "no_waits", "handles", "waited_streams", "bounded",
-                                   "sizes", "trim"])
+                                   "sizes", "trim", "count_sums"])
 def test_pool(pool_check, check):
     r = subprocess.run([pool_check, check], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
     assert r.returncode == 0 and "pool ok" in r.stdout, r.stdout[-4000:]
