@@ -5,8 +5,9 @@
 //             them on the GPU in one pass as separate vertex ranges and plans
 //             them as one block-diagonal unit (a single graph is planned on
 //             its own); admission keeps the resident set under the HBM
-//             budget, evicting idle units least recently used first
-//             (kResidentGrace after they became resident at the earliest)
+//             budget, evicting idle units least recently used first; a
+//             graph with results that nobody has polled yet keeps its pairs
+//             on the host and is prepared again for a request by its key
 //          -> [GPU worker] every ready request joins the next launch: the
 //             single-graph units in one persistent wedge-kernel launch over
 //             all of their plans, each multi-graph unit in one launch that
@@ -60,11 +61,22 @@ constexpr int64_t kPipeCacheBytes = int64_t(4) << 30;
 // Captured preparation turns to groups beyond this many queued graphs per
 // prep thread.
 constexpr size_t kBacklogPerThread = 8;
-// A unit stays resident this long at least, so that a request by key right
-// behind the graph's submission finds it however fast units are prepared.
-// It delays only budgets that preparation turns over within that time (1 GiB
-// in 10 ms is several times its rate).
-constexpr std::chrono::milliseconds kResidentGrace{10};
+// Pairs kept on the host for graphs with results that have not been polled, so
+// that a client that sends requests by key behind a graph's submission is
+// answered whatever has been evicted meanwhile.  Beyond this many bytes new
+// graphs' pairs go once they are prepared.  (Holding units resident for 10 ms
+// instead answered only clients quick enough, and kept a 4 MiB budget at 0.35
+// s for 410 graphs that take 0.09 s.)
+constexpr int64_t kKeptPairBytes = int64_t(64) << 20;
+// From this budget on none are kept: results are polled in the order they are
+// finished, so idle units whose results have been polled are the least
+// recently used ones, and the others are evicted only when they alone exceed
+// the budget -- not while they hold kKeptPairBytes of pairs in kKeptGraphs
+// graphs, which take at most 60 bytes a pair and 128 KiB a graph.  (Keeping
+// 430 MB for a client that submits 410 graphs before it polls costs 0.1 s of
+// page faults on top of 0.07 s.)
+constexpr int64_t kKeepBelowBudget = int64_t(1) << 30;
+constexpr int64_t kKeptGraphs = 4096;
 
 int64_t pow2_at_least(int64_t x, int64_t lo) {
     int64_t c = lo;
@@ -137,7 +149,6 @@ struct Unit {  // what is prepared, resident and evicted together
     int64_t bytes = 0;
     std::list<Unit*>::iterator lru;
     bool in_lru = false;
-    Clock::time_point published{};
     Unit() = default;
     Unit(const Unit&) = delete;
     Unit& operator=(const Unit&) = delete;
@@ -148,12 +159,21 @@ struct Unit {  // what is prepared, resident and evicted together
     }
 };
 
+struct Pairs {  // a submitted graph
+    std::vector<int32_t> src, dst;
+    int32_t n = 0;
+    int64_t bytes() const { return 8 * (int64_t)src.size(); }
+};
+
 struct Entry {  // one graph known to the server
     std::shared_ptr<Unit> unit;
     int idx = 0;    // its range in a multi-graph unit
-    int state = 0;  // 0 preparing, 1 resident, 2 failed
+    int state = 0;  // 0 preparing, 1 resident, 2 failed, 3 evicted with its pairs kept
     int status = BTC_OK;
     int pins = 0;   // requests holding the graph (waiting, ready or launched)
+    int unpolled = 0;                    // requests whose results have not been polled
+    std::shared_ptr<const Pairs> pairs;  // kept while there are any (kKeptPairBytes)
+    bool prepared = false;
 };
 
 struct Request {
@@ -165,19 +185,19 @@ struct Request {
 
 struct PrepJob {
     uint64_t key = 0;
-    std::vector<int32_t> src, dst;
-    int32_t n = 0;
+    std::shared_ptr<const Pairs> g;  // let go once its pairs are on the device
 };
 
 // Vertex count of a job (n, or max id + 1 when n <= 0); -1 when an id is
 // negative or not below n.
 int64_t job_vertices(const PrepJob& j) {
     int32_t lo = 0, hi = -1;
-    for (size_t e = 0; e < j.src.size(); ++e) {
-        lo = std::min(lo, std::min(j.src[e], j.dst[e]));
-        hi = std::max(hi, std::max(j.src[e], j.dst[e]));
+    const Pairs& g = *j.g;
+    for (size_t e = 0; e < g.src.size(); ++e) {
+        lo = std::min(lo, std::min(g.src[e], g.dst[e]));
+        hi = std::max(hi, std::max(g.src[e], g.dst[e]));
     }
-    const int64_t n = j.n > 0 ? j.n : (int64_t)hi + 1;
+    const int64_t n = g.n > 0 ? g.n : (int64_t)hi + 1;
     return (lo < 0 || hi >= n) ? -1 : n;
 }
 
@@ -194,6 +214,7 @@ struct btc_server_s {
     std::unordered_map<uint64_t, Entry> cache;
     std::list<Unit*> lru;  // front = most recently used resident unit
     int64_t resident_bytes = 0;
+    int64_t kept_bytes = 0, kept_graphs = 0;  // the entries' pairs
     std::deque<PrepJob> prep_queue;
     std::unordered_map<uint64_t, std::vector<Request>> waiting;  // key -> requests waiting for its plan
     std::deque<Request> ready;
@@ -209,22 +230,43 @@ struct btc_server_s {
         return true;
     }
 
-    // Caller holds mu.  Evicts idle resident units past their grace (LRU
-    // first) until `need`
+    // Caller holds mu.  Evicts idle resident units (LRU first) until `need`
     // more bytes fit; returns whether they fit.
     bool make_room(int64_t need) {
         auto it = lru.end();
         while (resident_bytes + need > opts.hbm_budget_bytes && it != lru.begin()) {
             --it;
             Unit* u = *it;
-            if (!unit_idle(u) || Clock::now() - u->published < kResidentGrace) continue;
+            if (!unit_idle(u)) continue;
             resident_bytes -= u->bytes;
             it = lru.erase(it);
             const std::vector<uint64_t> keys = u->keys;
-            for (uint64_t k : keys) cache.erase(k);  // the last reference frees the unit
+            for (uint64_t k : keys) {  // the last reference frees the unit
+                Entry& e = cache[k];
+                if (e.pairs) {
+                    e.state = 3;
+                    e.unit.reset();
+                } else {
+                    cache.erase(k);
+                }
+            }
             stats.evictions += (int64_t)keys.size();
         }
         return resident_bytes + need <= opts.hbm_budget_bytes;
+    }
+
+    // Caller holds mu: a result of `key` has been polled.  Returns pairs that
+    // nobody needs any more, to be freed without the lock.
+    std::shared_ptr<const Pairs> polled(uint64_t key) {
+        const auto it = cache.find(key);
+        if (it == cache.end() || it->second.unpolled == 0 || --it->second.unpolled > 0) return nullptr;
+        std::shared_ptr<const Pairs> g = std::move(it->second.pairs);
+        if (g) {
+            kept_bytes -= g->bytes();
+            --kept_graphs;
+        }
+        if (it->second.state == 3) cache.erase(it);
+        return g;
     }
 
     void finish(const Request& r, int status, uint64_t tri, int batch) {
@@ -262,14 +304,14 @@ struct btc_server_s {
         lru.push_front(u.get());
         u->lru = lru.begin();
         u->in_lru = true;
-        u->published = Clock::now();
         for (size_t k = 0; k < u->keys.size(); ++k) {
             const uint64_t key = u->keys[k];
             Entry& e = cache[key];
             e.unit = u;
             e.idx = (int)k;
             e.state = 1;
-            ++stats.prepared;
+            if (!e.prepared) ++stats.prepared;
+            e.prepared = true;
             for (Request& r : waiting[key]) ready.push_back(r);
             waiting.erase(key);
         }
@@ -283,7 +325,7 @@ struct btc_server_s {
         int rc = BTC_OK;
         if (cf & BTC_CANON_DEVICE) {
             rc = btcx::guard([&] {
-                const size_t nnz = job.src.size();
+                const size_t nnz = job.g->src.size();
                 btcx::TmpBuf<int32_t> ds, dd;
                 ds.alloc(nnz, s);
                 dd.alloc(nnz, s);
@@ -291,19 +333,18 @@ struct btc_server_s {
                     // staged through pinned memory: asynchronous copies (the
                     // canonicalisation synchronises s before the next use)
                     int32_t* h = reinterpret_cast<int32_t*>(pin.reserve(nnz * 8));
-                    std::memcpy(h, job.src.data(), nnz * 4);
-                    std::memcpy(h + nnz, job.dst.data(), nnz * 4);
+                    std::memcpy(h, job.g->src.data(), nnz * 4);
+                    std::memcpy(h + nnz, job.g->dst.data(), nnz * 4);
                     BTC_HIP(hipMemcpyAsync(ds.p, h, nnz * 4, hipMemcpyHostToDevice, s));
                     BTC_HIP(hipMemcpyAsync(dd.p, h + nnz, nnz * 4, hipMemcpyHostToDevice, s));
                 }
-                btcx::check_status(btc_graph_from_coo_device(ds.p, dd.p, (int64_t)nnz, job.n,
+                btcx::check_status(btc_graph_from_coo_device(ds.p, dd.p, (int64_t)nnz, job.g->n,
                                                              cf & ~BTC_CANON_DEVICE, s, &g));
             });
         } else {
-            rc = btc_graph_from_coo(job.src.data(), job.dst.data(), (int64_t)job.src.size(), job.n, cf, &g);
+            rc = btc_graph_from_coo(job.g->src.data(), job.g->dst.data(), (int64_t)job.g->src.size(), job.g->n, cf, &g);
         }
-        std::vector<int32_t>().swap(job.src);
-        std::vector<int32_t>().swap(job.dst);
+        job.g.reset();
         if (rc != BTC_OK) return rc;
         btc_graph_info gi;
         btc_graph_get_info(g, &gi);
@@ -339,9 +380,9 @@ struct btc_server_s {
     // pipeline (nothing done then).
     bool prepare_captured(PrepJob& job, uint32_t cf, const btc_count_opts& co, hipStream_t s, PipeCache& cache_p,
                           std::shared_ptr<Unit>& out, int& rc) {
-        const int64_t nnz = (int64_t)job.src.size();
+        const int64_t nnz = (int64_t)job.g->src.size();
         // with n given the pipeline checks the ids itself (on the device)
-        const int64_t nv = job.n > 0 ? (int64_t)job.n : job_vertices(job);
+        const int64_t nv = job.g->n > 0 ? (int64_t)job.g->n : job_vertices(job);
         if (nnz > kPipeMaxPairs || nv > kPipeMaxIds) return false;
         if (nv < 0) {
             rc = BTC_ERR_ARG;
@@ -353,9 +394,8 @@ struct btc_server_s {
         if (rc != BTC_OK) return true;
         const double t_start = now();
         uint64_t tri = 0;
-        rc = btc_pipeline_count(pipe, job.src.data(), job.dst.data(), nnz, job.n, 0, s, &tri, nullptr);
-        std::vector<int32_t>().swap(job.src);
-        std::vector<int32_t>().swap(job.dst);
+        rc = btc_pipeline_count(pipe, job.g->src.data(), job.g->dst.data(), nnz, job.g->n, 0, s, &tri, nullptr);
+        job.g.reset();
         if (rc != BTC_OK) return true;
         {
             // the requests waiting so far get their answer now
@@ -413,9 +453,9 @@ struct btc_server_s {
         std::vector<int64_t> sizes((size_t)k);
         int64_t nsum = 0, pairs = 0;
         for (int32_t g = 0; g < k; ++g) {
-            sp[(size_t)g] = jobs[(size_t)g].src.data();
-            dp[(size_t)g] = jobs[(size_t)g].dst.data();
-            sizes[(size_t)g] = (int64_t)jobs[(size_t)g].src.size();
+            sp[(size_t)g] = jobs[(size_t)g].g->src.data();
+            dp[(size_t)g] = jobs[(size_t)g].g->dst.data();
+            sizes[(size_t)g] = (int64_t)jobs[(size_t)g].g->src.size();
             nsum += nv[(size_t)g];
             pairs += sizes[(size_t)g];
         }
@@ -430,10 +470,7 @@ struct btc_server_s {
         rc = btcx::guard([&] {
             btcx::pipeline_count_checked(pipe, k, sp.data(), dp.data(), sizes.data(), nv.data(), s, per.data(), &tot);
         });
-        for (PrepJob& j : jobs) {
-            std::vector<int32_t>().swap(j.src);
-            std::vector<int32_t>().swap(j.dst);
-        }
+        for (PrepJob& j : jobs) j.g.reset();
         if (rc != BTC_OK) return rc;
         {
             std::lock_guard<std::mutex> lk(mu);
@@ -481,7 +518,7 @@ struct btc_server_s {
         size_t pairs = 0;
         for (size_t k = 0; k < jobs.size(); ++k) {
             segs[k + 1] = segs[k] + nv[k];
-            pairs += jobs[k].src.size();
+            pairs += jobs[k].g->src.size();
         }
         btc_graph_s G;
         int rc = btcx::guard([&] {
@@ -492,12 +529,12 @@ struct btc_server_s {
             size_t o = 0;
             for (size_t k = 0; k < jobs.size(); ++k) {
                 const int32_t v0 = (int32_t)segs[k];
-                for (size_t e = 0; e < jobs[k].src.size(); ++e, ++o) {
-                    src[o] = jobs[k].src[e] + v0;
-                    dst[o] = jobs[k].dst[e] + v0;
+                const Pairs& g = *jobs[k].g;
+                for (size_t e = 0; e < g.src.size(); ++e, ++o) {
+                    src[o] = g.src[e] + v0;
+                    dst[o] = g.dst[e] + v0;
                 }
-                std::vector<int32_t>().swap(jobs[k].src);
-                std::vector<int32_t>().swap(jobs[k].dst);
+                jobs[k].g.reset();
             }
             btcx::TmpBuf<int32_t> ds, dd;
             ds.alloc(pairs, s);
@@ -536,8 +573,7 @@ struct btc_server_s {
     // them; false when the server stops meanwhile.
     bool admit(int64_t est) {
         std::unique_lock<std::mutex> lk(mu);
-        // woken by unpinned units; a unit's grace ends without a signal
-        while (!(stop || make_room(est) || resident_bytes == 0)) cv_prep.wait_for(lk, std::chrono::milliseconds(1));
+        cv_prep.wait(lk, [&] { return stop || make_room(est) || resident_bytes == 0; });
         if (stop) return false;
         resident_bytes += est;  // reserved until the unit's real size is known
         return true;
@@ -575,8 +611,8 @@ struct btc_server_s {
                     const size_t cap =
                         (cf & BTC_CANON_DEVICE) && (!captured || backlog) ? (size_t)opts.group_graphs : 1;
                     while (!prep_queue.empty() && jobs.size() < cap &&
-                           (jobs.empty() || pairs + prep_queue.front().src.size() <= kGroupPairs)) {
-                        pairs += prep_queue.front().src.size();
+                           (jobs.empty() || pairs + prep_queue.front().g->src.size() <= kGroupPairs)) {
+                        pairs += prep_queue.front().g->src.size();
                         jobs.push_back(std::move(prep_queue.front()));
                         prep_queue.pop_front();
                     }
@@ -619,7 +655,7 @@ struct btc_server_s {
                         for (const PrepJob& j : good) keys.push_back(j.key);
                         std::shared_ptr<Unit> u;
                         int64_t pairs = 0;
-                        for (const PrepJob& j : good) pairs += (int64_t)j.src.size();
+                        for (const PrepJob& j : good) pairs += (int64_t)j.g->src.size();
                         const int rc = captured && pairs <= kPipeMaxPairs
                                            ? prepare_captured_group(good, nv, cf, co, s, pipes, u)
                                            : prepare_group(good, nv, cf, co, s, pin, u);
@@ -770,11 +806,10 @@ int btc_server_submit(btc_server sv, uint64_t graph_key, const int32_t* src, con
         BTC_REQUIRE(nnz >= 0 && (nnz == 0 || (src && dst)) , BTC_ERR_ARG, "bad edge arrays");
         // the pairs are copied before the lock is taken: preparation threads
         // and the GPU worker keep running meanwhile
-        PrepJob job;
-        job.key = graph_key;
-        job.src.assign(src, src + nnz);
-        job.dst.assign(dst, dst + nnz);
-        job.n = n;
+        auto g = std::make_shared<Pairs>();
+        g->src.assign(src, src + nnz);
+        g->dst.assign(dst, dst + nnz);
+        g->n = n;
         std::lock_guard<std::mutex> lk(sv->mu);
         BTC_REQUIRE(!sv->stop, BTC_ERR_STATE, "server is stopping");
         Request r;
@@ -788,15 +823,30 @@ int btc_server_submit(btc_server sv, uint64_t graph_key, const int32_t* src, con
             BTC_REQUIRE(nnz > 0 || n > 0, BTC_ERR_ARG, "graph %llu is not resident and no graph was given",
                         (unsigned long long)graph_key);
             Entry& e = sv->cache[graph_key];
-            e.pins = 1;
-            sv->prep_queue.push_back(std::move(job));
+            e.pins = e.unpolled = 1;
+            if (sv->opts.hbm_budget_bytes < kKeepBelowBudget && sv->kept_graphs < kKeptGraphs &&
+                sv->kept_bytes + g->bytes() <= kKeptPairBytes) {
+                e.pairs = g;
+                sv->kept_bytes += g->bytes();
+                ++sv->kept_graphs;
+            }
             sv->waiting[graph_key].push_back(r);
+            sv->prep_queue.push_back({graph_key, std::move(g)});
             // prep threads and admission waiters share cv_prep: wake them all so
             // an idle prep thread sees the job
             sv->cv_prep.notify_all();
             return;
         }
         Entry& e = it->second;
+        ++e.unpolled;
+        if (e.state == 3) {  // evicted: prepared again
+            e.state = 0;
+            ++e.pins;
+            sv->waiting[graph_key].push_back(r);
+            sv->prep_queue.push_back({graph_key, e.pairs});
+            sv->cv_prep.notify_all();
+            return;
+        }
         r.resident_hit = true;
         ++sv->stats.resident_hits;
         if (e.state == 2) {
@@ -817,6 +867,7 @@ int btc_server_submit(btc_server sv, uint64_t graph_key, const int32_t* src, con
 int btc_server_poll(btc_server sv, btc_result* out, int32_t capacity, int32_t wait_ms, int32_t* count) {
     return btcx::guard([&] {
         BTC_REQUIRE(sv && out && count && capacity > 0, BTC_ERR_ARG, "bad argument");
+        std::vector<std::shared_ptr<const Pairs>> gone;  // freed after the lock
         std::unique_lock<std::mutex> lk(sv->mu);
         if (sv->done.empty() && wait_ms > 0)
             sv->cv_done.wait_for(lk, std::chrono::milliseconds(wait_ms), [&] { return !sv->done.empty(); });
@@ -824,6 +875,7 @@ int btc_server_poll(btc_server sv, btc_result* out, int32_t capacity, int32_t wa
         while (k < capacity && !sv->done.empty()) {
             out[k++] = sv->done.front();
             sv->done.pop_front();
+            if (auto g = sv->polled(out[k - 1].graph_key)) gone.push_back(std::move(g));
         }
         *count = k;
     });

@@ -508,7 +508,10 @@ typedef struct {
 void btc_server_opts_default(btc_server_opts* opts);
 int btc_server_create(const btc_server_opts* opts, btc_server* out);
 /* src/dst/n describe the graph (copied); they may be NULL/0 when graph_key
- * was submitted before. */
+ * was submitted before and is resident still, or has results that have not
+ * been polled (for up to 4096 such graphs of 64 MiB of pairs in all: an
+ * evicted one is prepared again).  Else BTC_ERR_ARG: the graph has to be sent
+ * again. */
 int btc_server_submit(btc_server s, uint64_t graph_key, const int32_t* src, const int32_t* dst, int64_t nnz,
                       int32_t n, uint64_t* request_id);
 /* Moves up to `capacity` finished results into out, waiting up to wait_ms
