@@ -139,14 +139,13 @@ __global__ void relabel_kernel(uint64_t* __restrict__ keys, Cnt m_, int b, const
 // (some 19 G/s).  One copy and one run of 64 keys at a time against this:
 // R-MAT 2^20 (14 M edges) 873 -> 541 us, 24 graphs (3.3 M) 280 -> 159 us.
 constexpr uint32_t kDegWindow = 8192;
-
-// deg[v] over the copies
-__device__ __forceinline__ uint32_t degree_sum(const uint32_t* __restrict__ deg, size_t stride, int64_t v) {
-    uint32_t d = 0;
-#pragma unroll
-    for (uint32_t k = 0; k < kDegCopies; ++k) d += deg[k * stride + (size_t)v];
-    return d;
-}
+// The eager build keeps the copies from one edge per id on, or for few ids:
+// clearing and summing them is 64 bytes of traffic an id.  Builds in degree
+// order with 8 copies against one: Erdos-Renyi 2^22 ids with m / n = 1/4, 1/2,
+// 1, 2 901 / 1044 / 1379 / 1993 us against 858 / 996 / 1326 / 1947, R-MAT 2^22
+// 920 / 1067 / 1428 / 2087 against 922 / 1103 / 1502 / 2304, 2^17 ids and
+// fewer 5 to 10 us less whatever the edges.
+constexpr int64_t kDegCopyIds = int64_t(1) << 17;
 
 // key_at(e): key e, e < m; every thread of the workgroup calls it with its
 // own window h and degree copy.
@@ -192,18 +191,21 @@ __device__ __forceinline__ void count_degrees(KeyAt&& key_at, int64_t m, int b, 
 }
 
 __global__ __launch_bounds__(kT) void degree_kernel(const uint64_t* __restrict__ keys, int64_t m, int b,
-                                                    uint32_t* __restrict__ deg, size_t stride_deg) {
+                                                    uint32_t* __restrict__ deg, size_t stride_deg,
+                                                    uint32_t copies) {
     __shared__ uint32_t h[kDegWindow];
-    count_degrees([&](int64_t e) { return keys[e]; }, m, b, h, deg + (blockIdx.x % kDegCopies) * stride_deg);
+    count_degrees([&](int64_t e) { return keys[e]; }, m, b, h, deg + (blockIdx.x % copies) * stride_deg);
 }
 
 // key = top - degree (ascending = descending degree; top is at least the
 // largest degree), value = vertex
-__global__ void rank_keys_kernel(const uint32_t* __restrict__ deg, size_t stride_deg, Cnt n_, uint32_t top,
-                                 uint32_t* __restrict__ key, uint32_t* __restrict__ val) {
+__global__ void rank_keys_kernel(const uint32_t* __restrict__ deg, size_t stride_deg, uint32_t copies, Cnt n_,
+                                 uint32_t top, uint32_t* __restrict__ key, uint32_t* __restrict__ val) {
     const int64_t n = n_.get();
     for (int64_t v = blockIdx.x * (int64_t)kT + threadIdx.x; v < n; v += (int64_t)gridDim.x * kT) {
-        key[v] = top - degree_sum(deg, stride_deg, v);
+        uint32_t d = 0;
+        for (uint32_t k = 0; k < copies; ++k) d += deg[k * stride_deg + (size_t)v];
+        key[v] = top - d;
         val[v] = (uint32_t)v;
     }
 }
@@ -685,20 +687,22 @@ void canonicalise_device(const int32_t* src, const int32_t* dst, int64_t nnz, in
     if (flags & BTC_CANON_DEGREE_ORDER) {
         TmpBuf<uint32_t> deg, k0, v0, k1, v1, rank;
         DevBuf<int32_t> lab2;
-        deg.alloc((size_t)nc * kDegCopies, s);
+        uint32_t copies = m >= (int64_t)nc || nc <= kDegCopyIds ? kDegCopies : 1;
         k0.alloc((size_t)nc, s);
         v0.alloc((size_t)nc, s);
+        if (!deg.try_alloc((size_t)nc * copies, s)) deg.alloc((size_t)nc * (copies = 1), s);
+        BTC_HIP(hipMemsetAsync(deg.p, 0, (size_t)nc * copies * 4, s));
+        if (m) {
+            hipLaunchKernelGGL(degree_kernel, dim3(std::min(grid_for(m), kRedBlocks)), dim3(kT), 0, s, keys, m, bn, deg.p,
+                               (size_t)nc, copies);
+            BTC_CHECK_LAUNCH("degree_kernel");
+        }
+        BTC_LAUNCH(rank_keys_kernel, nc, s, deg.p, (size_t)nc, copies, nc, (uint32_t)nc, k0.p, v0.p);  // degrees are below nc
+        deg.release();
         k1.alloc((size_t)nc, s);
         v1.alloc((size_t)nc, s);
         rank.alloc((size_t)nc, s);
         lab2.alloc_on((size_t)nc, s);
-        BTC_HIP(hipMemsetAsync(deg.p, 0, (size_t)nc * kDegCopies * 4, s));
-        if (m) {
-            hipLaunchKernelGGL(degree_kernel, dim3(std::min(grid_for(m), kRedBlocks)), dim3(kT), 0, s, keys, m, bn, deg.p,
-                               (size_t)nc);
-            BTC_CHECK_LAUNCH("degree_kernel");
-        }
-        BTC_LAUNCH(rank_keys_kernel, nc, s, deg.p, (size_t)nc, nc, (uint32_t)nc, k0.p, v0.p);  // degrees are below nc
         bool alt = sort_pairs_u32(k0.p, v0.p, k1.p, v1.p, (size_t)nc, id_bits((int64_t)nc + 1), s);
         if (segs) {
             // then a stable sort by segment: (segment, -degree, id)

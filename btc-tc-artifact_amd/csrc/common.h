@@ -241,6 +241,18 @@ struct TmpBuf {
         p = static_cast<T*>(pool_alloc(count * sizeof(T), true, s));
         n = count;
     }
+    // alloc() of an array that the caller can do without: false when there is
+    // no memory for it
+    bool try_alloc(size_t count, hipStream_t st) {
+        try {
+            alloc(count, st);
+        } catch (const Error& e) {
+            if (e.code != BTC_ERR_NOMEM) throw;
+            clear_error();
+            return false;
+        }
+        return true;
+    }
     void release() {
         if (p) {
             if (!from_arena) {
