@@ -735,10 +735,14 @@ void plan_device(btc_plan_s* p, int64_t chunk, hipStream_t s) {
     const bool alt = sort_pairs_u32(k0.p, v0.p, k1.p, v1.p, ne, id_bits(n), s);
     const uint32_t* key = alt ? k1.p : k0.p;
     const uint32_t* val = alt ? v1.p : v0.p;
+    // the sort's spare arrays go before the lists come, the prefix sums come
+    // after the entries' records have gone: some 56 bytes an entry at the most
+    // beside L and the dense tiles
+    (alt ? k0 : k1).release();
+    (alt ? v0 : v1).release();
     TmpBuf<uint32_t> off;
     off.alloc((size_t)n + 1, s);
     BTC_LAUNCH(pivot_offsets_kernel, (int64_t)n + 1, s, key, ne, n, off.p);
-
 
     // one allocation: list records, row bitmaps, list rows; items apart
     const size_t lb = (size_t)ne * sizeof(uint4), bb = (size_t)nbm * (C / 32) * 4, rb = (size_t)ne * 4;
@@ -751,11 +755,11 @@ void plan_device(btc_plan_s* p, int64_t chunk, hipStream_t s) {
     }
     TmpBuf<uint64_t> cost, P;
     cost.alloc(ne, s);
-    P.alloc((size_t)ne + 1, s);
     if (ne)
         BTC_LAUNCH_CLIP(records_kernel, ne, s, rowptr, col, erow.p, key, val, (int64_t)ne, rec.p, C, lst, ur, cost.p,
                         st.p + 3, st.p + 6);
     rec.release();
+    P.alloc((size_t)ne + 1, s);
     exclusive_scan_u64(cost.p, P.p, ne, s);
     erow.release();
 
