@@ -1334,7 +1334,8 @@ void bitbsr_count(btc_bitbsr b, int32_t variant, int32_t threshold_blocks, int32
         // every dense tile holds more than tau entries, every unit one
         const uint64_t m = (uint64_t)b->rows.m;
         max_units = std::min<uint64_t>(std::min<uint64_t>(b->nblk, m / ((uint64_t)tau + 1)) * (uint64_t)(b->K / 16), m);
-        units.alloc(2 * max_units, s);
+        // no room for them: every tile row by row, the counts are the same
+        if (max_units >= 0xFFFFFFFFull || !units.try_alloc(2 * max_units, s)) tau = 16 * b->K;
     }
     btcx::host_words(pv.staged());
     unsigned long long* const h_total = btcx::host_total();

@@ -1,5 +1,6 @@
 """Calls that still fit when the device is nearly full: a GPU-planned plan in
-the bytes that lists, keys and prefix sums of every entry take (60 a list)."""
+the bytes that lists, keys and prefix sums of every entry take (60 a list), and
+an explicit small threshold whose dense units find no room."""
 import ctypes as C
 
 import numpy as np
@@ -59,6 +60,8 @@ def test_nearly_full_device(gpu, orc):
     p = gpu.Plan(g, planner=2, tau=64 * 16)  # no dense tiles
     i = p.info
     p.close()
+    b = gpu.BitBSR(g, 32)
+    assert b.count(tau=0)[0] == want  # every kernel is loaded by now
     gpu.memory_trim()
     need = 60 * max_lists(rp, col) + i["core_rows"] * i["core_ids"] // 8 + 40 * g.n + 128 * i["work_items"]
     fill = Fill()
@@ -67,6 +70,13 @@ def test_nearly_full_device(gpu, orc):
         p = gpu.Plan(g, planner=2, tau=64 * 16)
         assert p.info == i and p.count()[0] == want
         p.close()
+        gpu.memory_trim()
+        fill.leave(128 * MIB)  # of 500 for 32 bytes a unit
+        total, pv, _ = b.count(tau=0, per_vertex=True)
+        assert total == want and int(pv.sum()) == want
+        assert b.count()[0] == want
     finally:
         fill.drop()
+    assert b.count(tau=0)[0] == want
+    b.close()
     g.close()
