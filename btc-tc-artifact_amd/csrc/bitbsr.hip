@@ -223,14 +223,13 @@ struct RowBits<128> {
     }
 };
 
-// FILL = false: counts[I] = number of tiles of row block I; with `needed`,
-// the row blocks that counting the dense tiles (more than tau bits) reads are
-// marked: a dense tile's own and those of its columns.
-// FILL = true: writes tile I's indices / row_indices / bits at offs[I] and,
-// with pop, every tile's set bits (pop) and, beside each entry of L, those
-// of its tile (epop); *max_pop becomes the largest of them.  With `needed`
-// only the marked row blocks are written.
-template <int K, bool FILL>
+// FILL = false: counts[I] = number of tiles of row block I; with MORE, the row
+// blocks that counting the dense tiles (more than tau bits) reads are marked
+// in `needed`: a dense tile's own and those of its columns.
+// FILL = true: writes tile I's indices / row_indices / bits at offs[I]; with
+// `needed` only those of the marked row blocks; with MORE every tile's set
+// bits (pop) and, beside each entry of L, those of its tile (epop).
+template <int K, bool FILL, bool MORE>
 __global__ __launch_bounds__(256) void build_kernel(int n, int n_rb, const uint32_t* __restrict__ rowptr,
                                                      const int32_t* __restrict__ col,
                                                      uint32_t* __restrict__ counts,
@@ -238,8 +237,8 @@ __global__ __launch_bounds__(256) void build_kernel(int n, int n_rb, const uint3
                                                      uint32_t* __restrict__ indices,
                                                      uint32_t* __restrict__ row_indices,
                                                      uint64_t* __restrict__ tiles, uint32_t* __restrict__ pop,
-                                                     uint16_t* __restrict__ epop, uint32_t* __restrict__ max_pop,
-                                                     uint32_t* __restrict__ needed, int tau) {
+                                                     uint16_t* __restrict__ epop, uint32_t* __restrict__ needed,
+                                                     int tau) {
     const int lane = threadIdx.x & 63;
     const int r = lane & 15;
     const int64_t I = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * 4 + (lane >> 4);
@@ -251,7 +250,7 @@ __global__ __launch_bounds__(256) void build_kernel(int n, int n_rb, const uint3
         e = rowptr[row + 1];
     }
     uint64_t t = (FILL && valid) ? offs[I] : 0;
-    uint32_t cnt = 0, most = 0;
+    uint32_t cnt = 0;
     // the row's next four ids (kNoId past its end), refilled one load
     // ahead per consumed id so a run of ids in one tile waits on memory
     // once every four ids instead of once per id
@@ -264,7 +263,7 @@ __global__ __launch_bounds__(256) void build_kernel(int n, int n_rb, const uint3
         if (__all(cur == kNoTile)) break;
         if (cur != kNoTile) {
             RowBits<K> bits;
-            const uint32_t p0 = p;
+            [[maybe_unused]] const uint32_t p0 = p;
             while (b0 != kNoId && b0 / K == cur) {
                 bits.set((int)(b0 % K));
                 ++p;
@@ -287,20 +286,14 @@ __global__ __launch_bounds__(256) void build_kernel(int n, int n_rb, const uint3
                     tiles[t * 32 + 2 * r] = bits.w0;
                     tiles[t * 32 + 2 * r + 1] = bits.w1;
                 }
-                if (pop) {
-                    uint32_t c = p - p0;
-#pragma unroll
-                    for (int o = 8; o > 0; o >>= 1) c += (uint32_t)__shfl_xor((int)c, o, 16);
+                if constexpr (MORE) {
+                    const uint32_t c = row16_sum(p - p0);
                     if (r == 0) pop[t] = c;
                     for (uint32_t q = p0; q < p; ++q) epop[q] = (uint16_t)c;
-                    most = max(most, c);
                 }
                 ++t;
-            }
-            if (!FILL && needed) {
-                uint32_t c = p - p0;
-#pragma unroll
-                for (int o = 8; o > 0; o >>= 1) c += (uint32_t)__shfl_xor((int)c, o, 16);
+            } else if constexpr (MORE) {
+                const uint32_t c = row16_sum(p - p0);
                 if (c > (uint32_t)tau) {
                     const int64_t rb = (int64_t)cur * (K / 16) + r;
                     if (r < K / 16 && rb < n_rb) needed[rb] = 1;
@@ -311,10 +304,36 @@ __global__ __launch_bounds__(256) void build_kernel(int n, int n_rb, const uint3
         }
     }
     if (!FILL && valid && r == 0) counts[I] = cnt;
-    if (FILL && pop) {
+}
+
+// out[0] = the largest of the tiles' set bits, out[1] = the bits in tiles of
+// more than tau (both cleared before).  On few workgroups, with an atomic each: from the
+// fill's own waves the same-address atomics took most of its time where row
+// blocks are short (166 K of them: fill 402 -> 23 us).
+__global__ __launch_bounds__(256) void tile_stats_kernel(const uint32_t* __restrict__ pop, uint32_t nblk, uint32_t tau,
+                                                         uint32_t* __restrict__ out) {
+    __shared__ uint32_t s_most[4], s_dense[4];
+    uint32_t most = 0, dense = 0;
+    for (uint64_t t = (uint64_t)blockIdx.x * 256 + threadIdx.x; t < nblk; t += (uint64_t)gridDim.x * 256) {
+        const uint32_t c = pop[t];
+        most = max(most, c);
+        dense += c > tau ? c : 0u;  // at most nnz(L) in all
+    }
 #pragma unroll
-        for (int o = 32; o >= 16; o >>= 1) most = max(most, (uint32_t)__shfl_xor((int)most, o));
-        if (lane == 0 && most > *max_pop) atomicMax(max_pop, most);  // most waves find it raised already
+    for (int o = 32; o > 0; o >>= 1) most = max(most, (uint32_t)__shfl_xor((int)most, o));
+    dense = wave_sum_u32(dense);
+    if ((threadIdx.x & 63) == 0) {
+        s_most[threadIdx.x >> 6] = most;
+        s_dense[threadIdx.x >> 6] = dense;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 4; ++w) {
+            most = max(most, s_most[w]);
+            dense += s_dense[w];
+        }
+        if (most) atomicMax(&out[0], most);
+        if (dense) atomicAdd(&out[1], dense);
     }
 }
 
@@ -349,9 +368,9 @@ void build_impl(btc_graph_s* g, hipStream_t s, btc_bitbsr_s* b, bool counted, in
         BTC_HIP(hipMemsetAsync(needed.p, 0, (size_t)n_rb * 4, s));
     }
     if (grid) {
-        hipLaunchKernelGGL((build_kernel<K, false>), dim3(grid), dim3(256), 0, s, n, n_rb, g->d_rowptr.p,
-                           g->d_col.p, counts.p, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, needed.p,
-                           dense_tau);
+        auto count = needed.p ? build_kernel<K, false, true> : build_kernel<K, false, false>;
+        hipLaunchKernelGGL(count, dim3(grid), dim3(256), 0, s, n, n_rb, g->d_rowptr.p, g->d_col.p, counts.p, nullptr,
+                           nullptr, nullptr, nullptr, nullptr, nullptr, needed.p, dense_tau);
         BTC_CHECK_LAUNCH("build_kernel<count>");
         if (needed.p) {
             hipLaunchKernelGGL(drop_counts_kernel, dim3((unsigned)((n_rb + 255) / 256)), dim3(256), 0, s, counts.p,
@@ -371,7 +390,7 @@ void build_impl(btc_graph_s* g, hipStream_t s, btc_bitbsr_s* b, bool counted, in
     b->row_indices.alloc_on(nblk, s);
     b->tiles.alloc_on(nblk * (size_t)b->wpt, s);
     if (counted) {
-        build_row_lists(g, b->rows, s);
+        alloc_row_lists(g, b->rows, s);
         b->pop.alloc_on(nblk, s);
         b->work.alloc_on(kWorkWords, s);
     }
@@ -379,13 +398,21 @@ void build_impl(btc_graph_s* g, hipStream_t s, btc_bitbsr_s* b, bool counted, in
                        b->indptr.p, (size_t)n_rb + 1);
     BTC_CHECK_LAUNCH("narrow_u64_to_u32");
     if (grid && nblk) {
-        hipLaunchKernelGGL((build_kernel<K, true>), dim3(grid), dim3(256), 0, s, n, n_rb, g->d_rowptr.p,
-                           g->d_col.p, nullptr, offs.p, b->indices.p, b->row_indices.p, b->tiles.p,
-                           counted ? b->pop.p : nullptr, b->rows.epop, counted ? b->rows.d_count + 3 : nullptr,
-                           needed.p, dense_tau);
+        auto fill = counted ? build_kernel<K, true, true> : build_kernel<K, true, false>;
+        hipLaunchKernelGGL(fill, dim3(grid), dim3(256), 0, s, n, n_rb, g->d_rowptr.p, g->d_col.p, nullptr, offs.p,
+                           b->indices.p, b->row_indices.p, b->tiles.p, b->pop.p, b->rows.epop, needed.p, dense_tau);
         BTC_CHECK_LAUNCH("build_kernel<fill>");
+        if (counted) {
+            const unsigned sg = (unsigned)std::min<uint64_t>((nblk + 1023) / 1024, 256);
+            hipLaunchKernelGGL(tile_stats_kernel, dim3(sg), dim3(256), 0, s, b->pop.p, (uint32_t)nblk,
+                               (uint32_t)(2 * K), b->rows.d_count + 3);
+            BTC_CHECK_LAUNCH("tile_stats_kernel");
+        }
     }
     if (counted) {
+        // behind the fill pass, which finds the counting pass's lines of L in
+        // the L2 caches (complete graph of 2500 ids: 519 us, 886 behind this copy)
+        build_row_lists(g, b->rows, s);
         BTC_HIP(hipMemcpyAsync(b->rows.count, b->rows.d_count, sizeof(b->rows.count), hipMemcpyDeviceToHost, s));
         BTC_HIP(hipStreamSynchronize(s));
     }

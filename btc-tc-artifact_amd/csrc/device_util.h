@@ -65,6 +65,15 @@ __device__ __forceinline__ uint32_t group_min_u32(uint32_t v, int width) {
     return v;
 }
 
+// Sum over the 16 lanes of a DPP row, in every lane (all 16 active).
+__device__ __forceinline__ uint32_t row16_sum(uint32_t v) {
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xF, 0xF, false);  // row_ror:8
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x124, 0xF, 0xF, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x122, 0xF, 0xF, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x121, 0xF, 0xF, false);
+    return v;
+}
+
 __device__ __forceinline__ int popc64(uint64_t x) { return __popcll(x); }
 
 }  // namespace btcx

@@ -17,8 +17,11 @@ struct RowLists {
     uint32_t* rowptr = nullptr;   // n + 1
     int32_t* col = nullptr;       // m + kColPad
     uint16_t* epop = nullptr;     // m: set bits of the entry's tile (16 x 128 at most)
-    uint32_t* d_count = nullptr;  // items per class, then the largest tile popcount
-    uint32_t count[4] = {0, 0, 0, 0};  // d_count once it has been read back
+    // items per class, the largest tile popcount, entries in tiles of more than
+    // 2 K bits; count = d_count once it has been read back
+    static constexpr int kCounts = 8;
+    uint32_t* d_count = nullptr;
+    uint32_t count[kCounts] = {};
     int64_t m = 0, merge_work = 0;
 };
 
@@ -382,8 +385,10 @@ inline void drop_plan_bsr(btc_plan_s* p, hipStream_t s) {
     p->bsr = nullptr;
 }
 
-// Enqueues the copy of g's CSR and the row items on s; r.count is valid once
-// d_count has been read back.
+// Allocates the row lists of g (d_count cleared on s); then enqueues the copy
+// of its CSR and the row items.  r.count is valid once d_count has been read
+// back.
+void alloc_row_lists(const btc_graph_s* g, RowLists& r, hipStream_t s);
 void build_row_lists(const btc_graph_s* g, RowLists& r, hipStream_t s);
 
 // Counts the mask bits outside dense tiles (those of more than tau bits) row

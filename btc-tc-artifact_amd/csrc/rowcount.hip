@@ -551,7 +551,7 @@ __global__ __launch_bounds__(kT, 8) void rows_kernel(RowsArgs a) {
 
 }  // namespace
 
-void build_row_lists(const btc_graph_s* g, RowLists& r, hipStream_t s) {
+void alloc_row_lists(const btc_graph_s* g, RowLists& r, hipStream_t s) {
     const size_t n = (size_t)g->n, m = (size_t)g->m;
     r.m = (int64_t)m;
     r.merge_work = g->merge_work;
@@ -564,17 +564,21 @@ void build_row_lists(const btc_graph_s* g, RowLists& r, hipStream_t s) {
     r.cap1 = cap1;
     const size_t ib = (size_t)(cap0 + cap1 + cap2) * sizeof(uint4);
     const size_t rb = ((n + 1) * 4 + 255) & ~size_t(255);
-    r.block.alloc_on(ib + rb + (m + kColPad) * 4 + 16 + m * 2, s);
+    r.block.alloc_on(ib + rb + (m + kColPad) * 4 + 4 * RowLists::kCounts + m * 2, s);
     r.items = reinterpret_cast<uint4*>(r.block.p);
     r.rowptr = reinterpret_cast<uint32_t*>(r.block.p + ib);
     r.col = reinterpret_cast<int32_t*>(r.block.p + ib + rb);
     r.d_count = reinterpret_cast<uint32_t*>(r.col + m + kColPad);
-    r.epop = reinterpret_cast<uint16_t*>(r.d_count + 4);
-    BTC_HIP(hipMemsetAsync(r.d_count, 0, 16, s));
+    r.epop = reinterpret_cast<uint16_t*>(r.d_count + RowLists::kCounts);
+    BTC_HIP(hipMemsetAsync(r.d_count, 0, 4 * RowLists::kCounts, s));
+}
+
+void build_row_lists(const btc_graph_s* g, RowLists& r, hipStream_t s) {
+    const size_t n = (size_t)g->n, m = (size_t)g->m;
     const size_t work = std::max(n + 1, m + kColPad);
     const unsigned grid = (unsigned)std::min<size_t>((work + kT - 1) / kT, 2048);
     hipLaunchKernelGGL(row_items_kernel, dim3(grid), dim3(kT), 0, s, g->d_rowptr.p, g->d_col.p, (uint32_t)n,
-                       (uint64_t)(m + kColPad), r.rowptr, r.col, r.items, cap0, cap1, r.d_count);
+                       (uint64_t)(m + kColPad), r.rowptr, r.col, r.items, r.cap0, r.cap1, r.d_count);
     BTC_CHECK_LAUNCH("row_items_kernel");
 }
 
