@@ -683,16 +683,18 @@ __global__ __launch_bounds__(256) void dense_units_kernel(const uint32_t* __rest
 }
 
 // Dense tiles of one count (pop > tau): their units, in any order but each
-// tile's together, at units[0, *n_units).  A workgroup looks at kSelTiles tiles and takes the
-// dense ones 16 lanes each (a lane per tile row, then per slab).  Its units
-// get their places with one atomic: one per dense tile on the same address
-// took 54 of planted 2^17's 284 us.
+// tile's together, at units[0, *n_units).  A workgroup looks at `per` tiles
+// (at most kSelTiles) and takes the dense ones 16 lanes each (a lane per tile
+// row, then per slab).  Its units get their places with one atomic: one per
+// dense tile on the same address took 54 of planted 2^17's 284 us.  With 1024
+// tiles to every workgroup a graph of few tiles, all of them dense, waited for
+// a handful of workgroups (complete graph of 2500 ids, 16 x 128: 92 us).
 constexpr uint32_t kSelTiles = 1024;
 template <int K>
 __global__ __launch_bounds__(256) void select_dense_kernel(
     const uint32_t* __restrict__ pop, uint32_t nblk, int tau, int n_rb, const uint32_t* __restrict__ indptr,
     const uint32_t* __restrict__ indices, const uint32_t* __restrict__ row_indices,
-    const uint64_t* __restrict__ tiles, uint4* __restrict__ units, uint32_t* __restrict__ n_units) {
+    const uint64_t* __restrict__ tiles, uint4* __restrict__ units, uint32_t* __restrict__ n_units, uint32_t per) {
     constexpr int SLABS = K / 16;
     __shared__ uint32_t tile[kSelTiles];  // the workgroup's dense tiles
     __shared__ uint16_t have[kSelTiles];  // their slabs with a unit
@@ -700,8 +702,8 @@ __global__ __launch_bounds__(256) void select_dense_kernel(
     const uint32_t tid = threadIdx.x, lane = tid & 63, r = tid & 15, grp = tid >> 4;
     if (tid == 0) nd_s = 0;
     __syncthreads();
-    for (uint32_t x = tid; x < kSelTiles; x += 256) {
-        const uint64_t t = (uint64_t)blockIdx.x * kSelTiles + x;
+    for (uint32_t x = tid; x < per; x += 256) {
+        const uint64_t t = (uint64_t)blockIdx.x * per + x;
         if (t < nblk && (int)pop[t] > tau) tile[atomicAdd(&nd_s, 1u)] = (uint32_t)t;
     }
     __syncthreads();
@@ -1193,10 +1195,13 @@ void launch_dense_part(const btc_bitbsr_s* b, int tau, bool mfma, uint4* units, 
     BTC_REQUIRE(max_units < 0xFFFFFFFFull, BTC_ERR_OVERFLOW, "%llu dense units exceed a u32 index",
                 (unsigned long long)max_units);
     uint32_t* n_units = reinterpret_cast<uint32_t*>(d_slots - kWorkSlots + 1);  // the work words' first counter
-    const unsigned grid = (unsigned)(((uint64_t)b->nblk + kSelTiles - 1) / kSelTiles);
+    // four workgroups a CU, each with a dense tile for every 16 lanes at least
+    const uint64_t even = ((uint64_t)b->nblk + 4 * (uint64_t)device_cu_count() - 1) / (4 * (uint64_t)device_cu_count());
+    const uint32_t per = (uint32_t)std::min<uint64_t>(kSelTiles, std::max<uint64_t>(16, even));
+    const unsigned grid = (unsigned)(((uint64_t)b->nblk + per - 1) / per);
     auto launch = [&](auto kern) {
         hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, s, b->pop.p, b->nblk, tau, b->n_rb, b->indptr.p,
-                           b->indices.p, b->row_indices.p, b->tiles.p, units, n_units);
+                           b->indices.p, b->row_indices.p, b->tiles.p, units, n_units, per);
         BTC_CHECK_LAUNCH("select_dense_kernel");
     };
     switch (b->K) {
