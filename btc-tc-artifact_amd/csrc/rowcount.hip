@@ -212,15 +212,6 @@ struct RowBuckets {
     }
 };
 
-// The row itself in HBM (rows of more than half the table's slots over a
-// wide span).
-struct RowSearch {
-    const int32_t* col;
-    uint32_t t0, t1;
-    __device__ __forceinline__ uint32_t has(uint32_t k) const { return sorted_has(col, t0, t1, k); }
-    __device__ __forceinline__ uint32_t has4(uint4 k) const { return has(k.x) + has(k.y) + has(k.z) + has(k.w); }
-};
-
 // Spreads the units of the lanes' lists (units[x] of lane x, 0 = none) over
 // the wave, 64 at a time in list order: f(active, lane x's a, b, c, unit
 // index within the list).  Lists of a wave differ in length by orders of
@@ -288,8 +279,10 @@ struct WaveRows {
 // at a time get their bounds, a lane each, two rounds ahead (the ids) and
 // one round ahead (the bounds) of the round being scanned: a round of short
 // lists is otherwise a chain of three dependent loads.  The first bounds are
-// asked for before the sets are built.  Rounds start at c0, step cs.
-template <int TN>
+// asked for before the sets are built.  Rounds start at c0, step cs; lane x
+// takes list c + x LS of a round, so that the waves of a workgroup (LS = 4, c0
+// = wave) share the long lists at a row's end.
+template <int TN, uint32_t LS>
 struct ListFeed {
     const RowsArgs& a;
     const WaveRows<TN>& w;
@@ -312,7 +305,7 @@ struct ListFeed {
             }
     }
     __device__ __forceinline__ uint32_t id(uint32_t at) const {
-        const uint32_t g = at + lane;
+        const uint32_t g = at + lane * LS;
         uint32_t r, e, t0, j = kEmptySlot;
         place(g, r, e, t0);
         // nothing of the row lies below its first id
@@ -338,13 +331,35 @@ struct ListFeed {
     }
 };
 
+// Whether a list of len ids is searched for the pc ids of the row below it.
+__device__ __forceinline__ bool searched(uint32_t len, uint32_t pc) {
+    return len > kSearchLen && (uint64_t)len > (uint64_t)pc * kSearchCost * (uint32_t)(32 - __clz((int)len));
+}
+
+// Aligned quads that hold col[r0, r1).
+__device__ __forceinline__ uint32_t list_quads(uint32_t r0, uint32_t r1) {
+    return r0 < r1 ? (r1 - (r0 & ~3u) + 3) / 4 : 0u;
+}
+
+// Quad u of the list of n ids at a0 (col is padded past its end): ids before
+// the list (o wraps) or past it become kNoId, which no set holds.
+__device__ __forceinline__ uint4 list_quad(const int32_t* __restrict__ col, uint32_t a0, uint32_t n, uint32_t u) {
+    uint4 v = *reinterpret_cast<const uint4*>(col + (a0 & ~3u) + (size_t)u * 4);
+    const uint32_t o = 4 * u - (a0 & 3u);
+    v.x = o + 0 < n ? v.x : kNoId;
+    v.y = o + 1 < n ? v.y : kNoId;
+    v.z = o + 2 < n ? v.z : kNoId;
+    v.w = o + 3 < n ? v.w : kNoId;
+    return v;
+}
+
 // Scans the lists of a feed: set(r) gives row r's set, the lists' ids stream
 // through the sets, 4 per lane and step.  Only the row's ids below j can
 // match in N(j): where they are so few that searching them in a long list
 // takes less, that list is searched instead.  hits(r, h) collects h hits of
 // row r.
-template <int TN, class SetOf, class Hits>
-__device__ __forceinline__ void scan_wave(ListFeed<TN>& f, SetOf&& set, Hits&& hits) {
+template <int TN, uint32_t LS, class SetOf, class Hits>
+__device__ __forceinline__ void scan_wave(ListFeed<TN, LS>& f, SetOf&& set, Hits&& hits) {
     const RowsArgs& a = f.a;
     const int lane = (int)f.lane;
     while (f.c < f.w.upto[TN]) {
@@ -352,25 +367,13 @@ __device__ __forceinline__ void scan_wave(ListFeed<TN>& f, SetOf&& set, Hits&& h
         f.bounds(f.next_j, n0, n1);
         f.next_j = f.id(f.c + 2 * f.cs);
         uint32_t r, e, t0;
-        f.place(f.c + f.lane, r, e, t0);
+        f.place(f.c + f.lane * LS, r, e, t0);
         const uint32_t r0 = f.r0, len = f.r1 - f.r0, pc = e - t0;
-        const bool search = len > kSearchLen &&
-                            (uint64_t)len > (uint64_t)pc * kSearchCost * (uint32_t)(32 - __clz((int)len));
-        const uint32_t quads = len && !search ? (f.r1 - (r0 & ~3u) + 3) / 4 : 0u;
+        const bool search = searched(len, pc);
+        const uint32_t quads = search ? 0u : list_quads(r0, f.r1);
         auto quad = [&](bool on, uint32_t a0, uint32_t n, uint32_t row, uint32_t u) {
-            uint32_t h = 0;
             const auto st = set(row);  // reads other lanes
-            if (on) {
-                uint4 v = *reinterpret_cast<const uint4*>(a.col + (a0 & ~3u) + (size_t)u * 4);  // padded past its end
-                // ids before the list (o wraps) or past it become kNoId, which no set holds
-                const uint32_t o = 4 * u - (a0 & 3u);
-                v.x = o + 0 < n ? v.x : kNoId;
-                v.y = o + 1 < n ? v.y : kNoId;
-                v.z = o + 2 < n ? v.z : kNoId;
-                v.w = o + 3 < n ? v.w : kNoId;
-                h = st.has4(v);
-            }
-            hits(row, h);
+            hits(row, on ? st.has4(list_quad(a.col, a0, n, u)) : 0u);
         };
         if (__any(quads > kShortQuads)) {
             spread_units(quads, r0, len, r, lane, quad);
@@ -427,6 +430,61 @@ __device__ __forceinline__ void build_buckets(const int32_t* __restrict__ col, u
     row_sync<NT>();
 }
 
+// Lists of a row that fits neither LDS set (more than half the table's slots
+// over a span beyond the bitmap's), by a workgroup: windows of the id space one
+// after the other, each with the bitmap of the row's ids in it, and of every
+// list the part in the window.  `f` holds a wave's lists, at most 64.  Lists
+// that are searched take no window.  Bound: one workgroup a row's item, and
+// where the last few lists are long that is all a row has (60 rows of 100 K
+// ids over 3 M: count 2.9 ms; this kernel alone 83 with a search of the row for
+// every id).
+template <int W, uint32_t LS, class Hits>
+__device__ __forceinline__ void scan_windows(ListFeed<1, LS>& f, uint32_t t1, uint32_t lo, uint32_t hi, uint32_t* lds,
+                                             uint32_t tid, Hits&& hits) {
+    // the last word stays empty: ids outside the window (kNoId) land there
+    constexpr uint32_t kSpan = 32u * (W - 1);
+    const RowsArgs& a = f.a;
+    const int lane = (int)f.lane;
+    uint32_t r, e, t0;
+    f.place(f.c + f.lane * LS, r, e, t0);
+    const uint32_t first = f.w.t0[0], r0 = f.r0, r1 = f.r1, pc = e - t0;
+    const bool search = searched(r1 - r0, pc);
+    spread_units(search ? pc : 0u, r0, r1 - r0, 0u, lane, [&](bool on, uint32_t a0, uint32_t n, uint32_t, uint32_t u) {
+        hits(0u, on ? sorted_has(a.col, a0, a0 + n, (uint32_t)a.col[first + u]) : 0u);
+    });
+    uint32_t p = search ? r1 : r0;  // the list's ids from here on are still to come
+    uint32_t at = first;            // the row's
+    uint32_t base = lo & ~31u;
+    while (__syncthreads_or(p < r1)) {
+        const uint32_t end = base + kSpan;  // below 2^32: ids are below 2^31
+        for (uint32_t w = 4 * tid; w < (uint32_t)W; w += 4 * kT)
+            *reinterpret_cast<uint4*>(lds + w) = make_uint4(0, 0, 0, 0);
+        __syncthreads();
+        for (;;) {
+            const uint32_t k = (uint64_t)at + tid < t1 ? (uint32_t)a.col[at + tid] : 0xFFFFFFFFu;
+            if (k < end) atomicOr(&lds[(k - base) >> 5], 1u << ((k - base) & 31u));
+            const uint32_t in = (uint32_t)__syncthreads_count(k < end);
+            at += in;
+            if (in < (uint32_t)kT) break;
+        }
+        __syncthreads();
+        uint32_t z = p, zh = r1;  // first id of the list at or past the window's end
+        while (z < zh) {
+            const uint32_t mid = z + ((zh - z) >> 1);
+            if ((uint32_t)a.col[mid] < end) z = mid + 1;
+            else zh = mid;
+        }
+        const RowBitmap<W> set{lds, base};
+        spread_units(list_quads(p, z), p, z - p, 0u, lane, [&](bool on, uint32_t a0, uint32_t n, uint32_t, uint32_t u) {
+            hits(0u, on ? set.has4(list_quad(a.col, a0, n, u)) : 0u);
+        });
+        p = z;
+        __syncthreads();  // the next window rewrites the bitmap
+        if (end > hi) break;  // workgroup-uniform; list ids are below hi
+        base = end;
+    }
+}
+
 // Lists [it.z, ee) of one row by a wave (NT = 64) or a workgroup.
 template <int NT, int W, bool PV>
 __device__ __forceinline__ uint64_t row_item(const RowsArgs& a, uint4 it, uint32_t ee, uint32_t* lds, uint32_t tid) {
@@ -434,18 +492,29 @@ __device__ __forceinline__ uint64_t row_item(const RowsArgs& a, uint4 it, uint32
     const uint32_t lo = uniform((uint32_t)a.col[t0]), hi = uniform((uint32_t)a.col[t0 + d - 1]);
     const uint32_t base = lo & ~31u;
     const WaveRows<1> w{{t0}, {uniform(it.z)}, {0u, uniform(ee) - uniform(it.z)}};
-    const uint32_t c0 = NT == kT ? uniform(tid / 64) * 64 : 0u;
-    ListFeed<1> feed(a, w, tid & 63, c0, NT);
+    constexpr uint32_t LS = NT / 64;
+    ListFeed<1, LS> feed(a, w, tid & 63, NT == kT ? uniform(tid / 64) : 0u, NT);
     uint32_t mine = 0;
     auto add = [&](uint32_t, uint32_t h) { mine += h; };
-    if (hi - base < 32u * W - 1u) {
+    // Where dense tiles are left out, whole items have no list to scan (most
+    // of 12 K items of a complete graph of 2500 ids: kernel 376 -> 282 us with
+    // 16 x 128 tiles of more than 512 bits left out).  The answer waits for the
+    // lists' bounds, so other counts do not ask.
+    static_assert(kBlockLists <= kT && kWaveLists <= 64, "the first round holds every list");
+    bool none = false;
+    if (a.epop) {
+        const bool some = feed.r0 < feed.r1;
+        none = NT == kT ? !__syncthreads_or(some) : !__any(some);
+    }
+    if (none) {
+    } else if (hi - base < 32u * W - 1u) {
         build_window<NT, W>(a.col, t0, d, base, hi, lds, tid);
         scan_wave(feed, [&](uint32_t) { return RowBitmap<W>{lds, base}; }, add);
     } else if (NT < kT || d <= (uint32_t)W / 2) {
         build_buckets<NT, W>(a.col, t0, d, lds, tid);
         scan_wave(feed, [&](uint32_t) { return RowBuckets<W>{lds}; }, add);
-    } else {
-        scan_wave(feed, [&](uint32_t) { return RowSearch{a.col, t0, t0 + d}; }, add);
+    } else if constexpr (NT == kT) {
+        scan_windows<W>(feed, t0 + d, lo, hi, lds, tid, add);
     }
     row_sync<NT>();  // the next item rewrites the set
     if constexpr (PV) {
@@ -474,7 +543,7 @@ __device__ __forceinline__ uint64_t light_rows(const RowsArgs& a, uint4 it, uint
         w.t0[k] = w.e0[k] = (uint32_t)__builtin_amdgcn_readlane((int)t0, k * kRowTeam);
         w.upto[k + 1] = w.upto[k] + (uint32_t)__builtin_amdgcn_readlane((int)d, k * kRowTeam);
     }
-    ListFeed<4> feed(a, w, (uint32_t)lane, 0u, 64u);
+    ListFeed<4, 1> feed(a, w, (uint32_t)lane, 0u, 64u);
     uint32_t all = 0;
     auto add = [&](uint32_t row, uint32_t h) {
         if constexpr (PV) {
