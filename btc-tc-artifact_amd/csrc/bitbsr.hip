@@ -1332,14 +1332,32 @@ void btc_bitbsr_free(btc_bitbsr b) { btcx::free_handle(b); }
 
 namespace {
 
-// With no threshold given, graphs whose merge work (the sum of d(i) + d(j)
-// over the edges) is below this count every tile row by row: the dense part
-// is two more kernels and an allocation in front of the rows.  Planted
-// communities (16 x 32 / 16 x 128 tiles, us with the dense part against rows
-// only): work 19 M 112 / 123 against 72, 75 M 155 / 152 against 105, 151 M
-// 203 / 175 against 165, 301 M 246 / 242 against 239 / 266, 874 M 279 / 312
-// against 423.
-constexpr int64_t kDenseMinWork = int64_t(1) << 28;
+// The threshold that a count uses for a given one.  Where most entries lie in
+// tiles of more than 2 K bits (an eighth) and the lists are long enough (merge
+// work, the sum of d(i) + d(j) over the entries, of 96 an entry, or of 64 in
+// large graphs), the dense part's two kernels pay, whatever higher threshold
+// is given: from 64 bits a tile on, or 2 K where the lists are shorter.
+// Elsewhere the rows count every tile, unless a threshold below the default
+// asks for the dense part.  Counts in us, 64 bits / 2 K / the default against
+// the rows alone (w: merge work an entry):
+//   complete graph of 150 ids    16 x 32  34 against 49   16 x 128  38 /  38 /  40 against 49
+//   complete graph of 2500 ids            73 against 1406           76 /  93 / 332 against 1420
+//   band of 40, 10^5 ids (w 78)          103 against 175           103 / 143 / 184 against 178
+//   planted 128 x 0.5 (w 68), 2^17 ids   168 against 236           185 / 175 / 188 against 237
+//     the same, 2^15 ids (work 7.5e7)     85 against 94            113 /  91 /  96 against 92
+//   planted 64 x 0.6 (w 42), 2^17 ids    156 against 142           181 / 168 / 157 against 143
+//   R-MAT 2^17 in id order               650 against 461             default 429 against 409
+//   60 rows of 10^5 ids over 3 x 10^6    183 ms against 3.0          default 33 ms against 3.0
+int32_t count_tau(const btc_bitbsr_s* b, int32_t tau) {
+    const int32_t dflt = btc_default_tau(b->K);
+    if (tau < 0) tau = dflt;
+    const int64_t m = b->rows.m, work = b->rows.merge_work;
+    if (2 * (int64_t)b->rows.count[4] >= m) {
+        if (work >= 96 * m) return std::min(tau, 64);
+        if (work >= 64 * m && work >= (int64_t(1) << 27)) return std::min(tau, 2 * b->K);
+    }
+    return tau < dflt ? tau : 16 * b->K;
+}
 
 // btc_bitbsr_count with per-vertex output to int32 (pv32) or int64 (pv64).
 void bitbsr_count(btc_bitbsr b, int32_t variant, int32_t threshold_blocks, int32_t tau, void* stream,
@@ -1350,8 +1368,7 @@ void bitbsr_count(btc_bitbsr b, int32_t variant, int32_t threshold_blocks, int32
     BTC_REQUIRE(variant >= BTC_VARIANT_AUTO && variant <= BTC_VARIANT_DIRECT, BTC_ERR_ARG,
                 "unknown variant %d", variant);
     hipStream_t s = btcx::as_stream(stream);
-    if (tau < 0)
-        tau = mfma || b->rows.merge_work >= kDenseMinWork ? btc_default_tau(b->K) : 16 * b->K;
+    tau = count_tau(b, tau);
     (void)threshold_blocks;  // both variants find a tile's row block the same way here
     BTC_REQUIRE(b->nblk == 0 || btcx::lane_sums_fit(b->max_row, b->K), BTC_ERR_OVERFLOW,
                 "longest row %d: a lane's 32-bit sum over %d tile columns could overflow", b->max_row, b->K / 4);

@@ -156,16 +156,19 @@ int btc_bitbsr_copy_to_host(btc_bitbsr b, uint32_t* indptr, uint32_t* indices,
 void btc_bitbsr_free(btc_bitbsr b);
 
 /* Reference-semantics hybrid count over a Bit-BSR ("btc-plain"):
- * popcount(tile) > tau routes a mask tile to the dense AND+popcount path, else
- * to the sparse per-bit path (tc_16x128_mma_v5.h:9-211,
+ * popcount(tile) > tau routes a mask tile to the dense path (AND + popcount, or
+ * i8 MFMA), else to the sparse per-bit path (tc_16x128_mma_v5.h:9-211,
  * tc_16x32_mma_v6.h:9-238), which takes the sparse tiles' bits row by row.
- * The counts do not depend on variant, threshold_blocks or tau.
- *   variant: BTC_VARIANT_AUTO picks BINSEARCH when num_blocks <
- *            threshold_blocks, else DIRECT (tc_16x128_adaptive.h:12-29,
- *            tc_16x32_adaptive.h:14-31); threshold_blocks <= 0 takes the
- *            reference default for K (2048 for K=128, 40000 for K=32 and 64).
- *   tau:     < 0 takes the default for K (512 for 128, 64 for 32, 128 for 64),
- *            or, for graphs with little work, the sparse path for every tile.
+ * The counts depend on none of variant, threshold_blocks and tau.
+ *   variant: BTC_VARIANT_AUTO, _BINSEARCH or _DIRECT, by which the reference
+ *            picks how a tile's row block is found (tc_16x128_adaptive.h:12-29,
+ *            tc_16x32_adaptive.h:14-31); accepted, and the same here.  With
+ *            BTC_DENSE_MFMA or-ed in, dense tiles take the MFMA form.
+ *   threshold_blocks: accepted with AUTO, and the same here.
+ *   tau:     < 0 takes the default for K (512 for 128, 64 for 32, 128 for 64).
+ *            Where most entries lie in tiles of more than 2 K bits and lists
+ *            are long, a higher tau counts as 64 or 2 K; elsewhere every tile
+ *            takes the sparse path from the default on.
  *   per_vertex: host int32[n] row sums of L .* (L L^T), or NULL.
  *   kernel_ms: event time of the count kernel(s) on `stream`, or NULL. */
 #define BTC_VARIANT_AUTO 0
