@@ -491,6 +491,10 @@ class Pipeline:
         """(total, per-graph uint64 array, kernel_ms) of [(src, dst, n), ...]
         in one run (btc_pipeline_count_graphs)."""
         k = len(graphs)
+        if k == 0:
+            raise ValueError("no graphs")
+        if any(np.ndim(x) == 0 for g in graphs for x in g[:2]):
+            raise TypeError("src and dst are arrays")
         pairs = [(np.ascontiguousarray(g[0], np.int32), np.ascontiguousarray(g[1], np.int32)) for g in graphs]
         if any(u.shape != v.shape for u, v in pairs):
             raise ValueError("src and dst differ in length")
