@@ -257,7 +257,7 @@ void upload_pairs(btc_pipeline_s* p, char* pin, int32_t count, const int32_t* co
         size_t z = k;
         int64_t n = 0;
         while (z < pieces.size() && n < kRound) n += pieces[z++].n;
-        const int team = (int)std::min<int64_t>(omp_get_max_threads(), n >> 15);
+        const int team = (int)std::max<int64_t>(1, std::min<int64_t>(omp_get_max_threads(), n >> 15));
 #pragma omp parallel for schedule(static) num_threads(team) if (team > 1)
         for (size_t x = k; x < z; ++x)
             std::memcpy(stage + pieces[x].to, pieces[x].from, (size_t)pieces[x].n * 4);
