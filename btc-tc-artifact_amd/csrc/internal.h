@@ -220,12 +220,10 @@ struct PipeCtl {
     uint32_t nc;     // vertices of L (after compaction)
     uint32_t ne;     // prefix lists
     uint32_t nbm;    // rows with a hub-core bitmap
-    uint32_t nbm_words;
     uint32_t nitems;           // work items
     uint32_t item_counts[2];   // {workgroup items, workgroup + wave items}
     unsigned long long rs[3];  // longest row, sum C(d, 2), merge work
     unsigned long long st[8];  // planner statistics (as plan_device's)
-    unsigned long long chunk;  // wedge checks per work item
     unsigned long long checks; // wedge checks in all
     unsigned long long total;  // triangles of the run
     unsigned long long err;    // the sorts' and scans' error word
