@@ -433,8 +433,9 @@ int btc_pipeline_count(btc_pipeline p, const int32_t* src, const int32_t* dst, i
                        int32_t device_pairs, void* stream, uint64_t* total, float* kernel_ms);
 /* count graphs in one run (host pairs, the layout of btc_batch_from_coo:
  * graph k's pairs are src/dst[edge_offsets[k], edge_offsets[k+1]) over ids
- * [0, n_per_graph[k]), n <= 0: its largest id + 1; an id out of
- * range refuses the call and leaves the last run as it was); per_graph[k] (may be NULL) = graph k's triangles, *total = all. */
+ * [0, n_per_graph[k]), n <= 0: its largest id + 1; an id out of range refuses
+ * the call and leaves the last run as it was); per_graph[k] (may be NULL) =
+ * graph k's triangles, *total = all. */
 int btc_pipeline_count_batch(btc_pipeline p, const int32_t* src, const int32_t* dst, const int64_t* edge_offsets,
                              const int32_t* n_per_graph, int32_t count, void* stream, uint64_t* per_graph,
                              uint64_t* total, float* kernel_ms);
@@ -449,7 +450,9 @@ int btc_pipeline_graph(btc_pipeline p, void* stream, btc_graph* out);
 /* The last accepted run's L and plan, copied into buffers of their own:
  * *graph is btc_pipeline_graph's graph, *plan a plan of it (no dense tiles,
  * no tiny items) that btc_plan_count and the others count like any plan,
- * unaffected by later runs.  Free the plan before the graph. */
+ * unaffected by later runs.  The order of its work items and the numbering of
+ * its hub-core bitmaps may differ between runs of the same pairs; counts, L
+ * and the plan's info do not.  Free the plan before the graph. */
 int btc_pipeline_export(btc_pipeline p, void* stream, btc_graph* graph, btc_plan* plan);
 /* The last run of a pipeline of several graphs as a batch (btc_batch_count
  * gives its per-graph counts again), independent of later runs. */
