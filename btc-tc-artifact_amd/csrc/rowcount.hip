@@ -14,9 +14,9 @@
 // mask tile walks two tile-column lists for one row intersection, most of
 // whose matched tile pairs are empty in that row.  Rows read only ids that
 // can match.  Count calls on MI355X, a wave per mask tile with per-lane
-// merges against rows: Erdos-Renyi 2^14 (131 K edges, 16 x 32) 718 -> 48 us,
-// planted 2^17 (4.4 M edges, 16 x 128, dense tiles apart) 944 -> 230 us,
-// R-MAT 2^17 in id order (1.9 M edges, 16 x 128, per vertex) 7406 -> 587 us.
+// merges against rows: Erdos-Renyi 2^14 (131 K edges, 16 x 32) 720 -> 35 us,
+// planted 2^17 (4.4 M edges, 16 x 128, dense tiles apart) 939 -> 206 us,
+// R-MAT 2^17 in id order (1.9 M edges, 16 x 128, per vertex) 7445 -> 479 us.
 // Bound: VALU issue in the membership tests (60 to 75 % of the issue slots
 // on the last two), the rest the latency of short rows' load chains.
 #include "device_util.h"
