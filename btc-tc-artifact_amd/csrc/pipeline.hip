@@ -14,6 +14,7 @@
 #include <omp.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstring>
 #include <mutex>
 
@@ -230,11 +231,24 @@ __global__ __launch_bounds__(kT) void group_pairs_kernel(int32_t* __restrict__ s
     if (bad != 0xFFFFFFFFu) atomicMin(&w[2 * (kMaxPipelineGraphs + 1)], bad);
 }
 
+// Threads that stage pairs at the moment: they share the process's cores, so
+// that pipelines side by side do not each bring a whole team.  Eight host
+// threads with a pipeline each, time of a replay by run: 1.54-1.76 ms with
+// whole teams, 1.29-1.57 ms so (four: 0.83-0.91 and 0.77-0.83; one: the same).
+std::atomic<int> g_staging{0};
+struct Staging {
+    const int sharers;
+    Staging() : sharers(++g_staging) {}
+    ~Staging() { --g_staging; }
+};
+
 // Host pairs of `count` arrays to p->src / p->dst, one after the other,
 // through the pinned buffer: threads fill 4 MiB at a time while the DMA
 // engine drains what came before.
 void upload_pairs(btc_pipeline_s* p, char* pin, int32_t count, const int32_t* const* src, const int32_t* const* dst,
                   const int64_t* sizes, int64_t pairs, hipStream_t s) {
+    const Staging staging;
+    const int64_t most = std::max(1, omp_get_max_threads() / staging.sharers);
     constexpr int64_t kPiece = int64_t(1) << 14, kRound = int64_t(1) << 20;  // ids
     int32_t* const stage = reinterpret_cast<int32_t*>(pin + kPinHeader);
     struct Piece {
@@ -257,7 +271,7 @@ void upload_pairs(btc_pipeline_s* p, char* pin, int32_t count, const int32_t* co
         size_t z = k;
         int64_t n = 0;
         while (z < pieces.size() && n < kRound) n += pieces[z++].n;
-        const int team = (int)std::max<int64_t>(1, std::min<int64_t>(omp_get_max_threads(), n >> 15));
+        const int team = (int)std::max<int64_t>(1, std::min<int64_t>(most, n >> 15));
 #pragma omp parallel for schedule(static) num_threads(team) if (team > 1)
         for (size_t x = k; x < z; ++x)
             std::memcpy(stage + pieces[x].to, pieces[x].from, (size_t)pieces[x].n * 4);
